@@ -166,7 +166,8 @@ int femgpu_csrmv_f32(femgpu_csr *A, const float *d_P, float *d_Q);
  * slices at most 16 wide, else FEMGPU_ERR_ARG). femgpu_csr_autotune times every candidate on A's
  * structure and current values (20 launches each, HIP events) and keeps the fastest; us[] =
  * microseconds per launch for L = 1, 2, 4, 8, 16, us_sell for L = 0 (0 where not possible).
- * Synchronises the context's stream. Default L = 8. No reference counterpart (the reference's
+ * Synchronises the context's stream. Until one of the two is called, a kernel chosen from the
+ * matrix's size and row length reads the CSR arrays. No reference counterpart (the reference's
  * csrmv is one loop per row). */
 typedef struct {
     int lanes;             /* the L chosen */

@@ -223,13 +223,14 @@ static int csr_setup(femgpu_csr *A, int n, int nnz, const int *IA, const int *JA
         if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), false, A->fplan);
     }
     if (!rc) rc = build_sell(ctx, A, IA, JA);
+    if (!rc) rc = build_staged(ctx, A, IA, JA);
     if (plans & FEMGPU_PLANS_MIXED) {   // parallel FP32 ILU(0) and Jacobi iterations
         if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), true, A->fplan_nat);
         if (!rc) rc = build_jacobi_ell(ctx, A, IA, JA, diag.data());
         if (!rc) rc = build_parilu_sell(ctx, A, IA, JA, diag.data());
     }
     // a rebuilt matrix keeps FP64 sliced ELL only where its new structure allows it
-    if (!rc && A->spmv_lanes == 0 && !sell64_possible(A)) rc = set_spmv_lanes(A, 8);
+    if (!rc && A->spmv_lanes == 0 && !sell64_possible(A)) rc = set_spmv_lanes(A, -1);
     if (!rc && hipMemsetAsync(A->AA.p, 0, sizeof(double) * (nnz + 1), s) != hipSuccess) rc = FEMGPU_ERR_HIP;
     if (!rc && sell64_active(A)) rc = launch_sell_values(ctx, A);
     if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = FEMGPU_ERR_HIP;

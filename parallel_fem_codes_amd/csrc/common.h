@@ -255,7 +255,11 @@ struct femgpu_csr {
     int prec64_jacobi = 0;              // FP64 ILU apply: 0 exact sweeps, k > 0 k Jacobi iterations
     bool par64_factored = false;        // the FP64 parallel factors hold the current values
     fg::DevBuf<double> par64_v, par64_a, par64_b, par64_d, par64_db, ell64_vl, ell64_vu, jac64_a, jac64_b;
-    int spmv_lanes = 8;             // lanes per row of the FP64 CSR kernels; 0: sliced ELL (sell_val64)
+    int spmv_lanes = -1;            // FP64 products: -1 the default (staged CSR where it applies, else 4 or 8 lanes
+                                    // per row), else lanes per row of the CSR kernels; 0: sliced ELL (sell_val64)
+    int staged_cap = 0;                 // staged CSR products: entries of the densest 64-row slice (0: not used)
+    bool staged16 = false;              // their columns as 16-bit distances from the slice's first row
+    fg::DevBuf<short> staged_d16;
     int plans = 3;                  // FEMGPU_PLANS_* built at creation
 };
 
@@ -371,6 +375,7 @@ int launch_jacobi_apply32_scaled(femgpu_ctx *ctx, femgpu_csr *A, int it, const d
 int launch_parilu64(femgpu_ctx *ctx, femgpu_csr *A, int sweeps);
 int launch_jacobi_apply64(femgpu_ctx *ctx, femgpu_csr *A, int it, const double *b, double *x, const int *skip);
 int build_sell(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA);
+int build_staged(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA);
 int build_parilu_sell(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag);
 int launch_parilu_to_csr(femgpu_ctx *ctx, femgpu_csr *A);
 int launch_sell_values(femgpu_ctx *ctx, femgpu_csr *A);

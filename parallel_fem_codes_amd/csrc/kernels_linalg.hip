@@ -301,11 +301,134 @@ __global__ __launch_bounds__(256) void k_residual(int n, const int *__restrict__
     if (lane == 0) r[row] = f[row] - acc;
 }
 
+// Staged CSR products (FP64, the default): a wave takes 64 consecutive rows, whose entries are one
+// contiguous run of AA. The wave loads the run's values and columns in order (lane l the entries l,
+// l + 64, ...; every load one contiguous span, U of them in flight), leaves the products in its own
+// part of LDS, and lane l then adds row l's products in their order, so the sum is the serial one.
+// What bounds it is the stream of values and columns; with LPR lanes per row most lanes of a 7-entry
+// row idle and the row loop is a chain of short dependent loads. Columns are 16-bit distances from the
+// slice's first row where the band allows (CT = short), else JA. The kernel reads AA itself, so
+// in-place assembly needs no refresh before it, as with k_spmv. 1237 x 812 nodes (n = 1.0e6, 7.0e6
+// entries): 15.6 us, 6.7 TB/s of the 104 MB with int columns (k_spmv: 32.1 us with 8 lanes per row,
+// 19.7 with 2; sliced ELL 14.2, but that needs its copy of the values). Slices of up to kStagedMax entries (31 per row; 62 KB of LDS
+// per block); denser slices stay with k_spmv.
+// RESIDUAL: y = f - A x, with the block's partial of ||y||^2 in sumsq where it is set.
+constexpr int kStagedMax = 1984;   // entries of a 64-row slice at most
+// Entries from which the staged kernel is the default. Its chain (load, product through LDS, sum) takes
+// 3.7-5 us whatever the size, a wave per 64 rows: 300 x 261 nodes 4.0 us against 3.1 with 4 lanes per
+// row, 500 x 500 (1.7e6 entries) 5.6 against 5.7, 600 x 600 7.3 against 8.1; rows of 21 entries
+// (Navier-Stokes) at 170 x 170 (1.8e6) 6.5 against 5.9 with 8 lanes, at 200 x 200 (2.5e6) 6.7 against 7.7.
+constexpr int kStagedMinEntries = 2 << 20;
+// Lanes per row below that: 4 for rows of about 7 entries (300 x 261 nodes: 3.1 us, 4.2 with 8), 8 for
+// wide ones (170 x 170 Navier-Stokes: 5.9 us, 6.3 with 4).
+static int default_lanes(const femgpu_csr *A) { return A->nnz / 12 <= A->n ? 4 : 8; }
+
+template <typename CT, int U, bool RESIDUAL>
+__global__ __launch_bounds__(256) void k_spmv_staged(int n, int cap, const int *__restrict__ IA,
+                                                     const CT *__restrict__ col, const double *__restrict__ AA,
+                                                     const double *__restrict__ x, const double *__restrict__ xs_ptr,
+                                                     double *__restrict__ xout, const double *__restrict__ f,
+                                                     double *__restrict__ y, double *__restrict__ sumsq,
+                                                     const int *__restrict__ skip)
+{
+    if (skip && *skip) return;
+    extern __shared__ double prod[];
+    __shared__ double red[4];
+    const int blk = xcd_block(), l = threadIdx.x & 63;
+    const int r0 = blk * 256 + static_cast<int>(threadIdx.x & ~63u), row = r0 + l;
+    double *mine = prod + (threadIdx.x >> 6) * cap;
+    const double xs = xs_ptr ? *xs_ptr : 1.0;
+    const int a = IA[row < n ? row : n], b = IA[row + 1 < n ? row + 1 : n];
+    const double fr = RESIDUAL ? f[row < n ? row : n - 1] : 0.0;
+    const int p0 = __builtin_amdgcn_readfirstlane(a), cnt = __builtin_amdgcn_readlane(b, 63) - p0;
+    for (int e0 = l; e0 < cnt; e0 += 64 * U) {
+        double v[U], g[U];
+        int c[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = e0 + 64 * u, q = p0 + (e < cnt ? e : e0);
+            v[u] = AA[q];
+            c[u] = sell_colof(col[q], r0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) g[u] = x[c[u]] * xs;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (e0 + 64 * u < cnt) mine[e0 + 64 * u] = v[u] * g[u];
+    }
+    // the wave's own LDS writes before its reads (no other wave touches this part)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double acc = 0.0;
+    for (int q = a - p0; q < b - p0; q += 8) {
+        double t[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t[u] = mine[q + u < b - p0 ? q + u : q];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc = q + u < b - p0 ? acc + t[u] : acc;
+    }
+    if (RESIDUAL) {
+        const double rv = fr - acc;
+        if (row < n) y[row] = rv;
+        if (sumsq) {   // the block's partial of ||r||^2 (a later kernel sums the blocks in order)
+            const double q = block_sum<256>(row < n ? rv * rv : 0.0, red);
+            if (threadIdx.x == 0) sumsq[blk] = q;
+        }
+    } else if (row < n) {
+        y[row] = acc;
+        if (xout) xout[row] = x[row] * xs;
+    }
+}
+
+int build_staged(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA)
+{
+    const int n = A->n;
+    A->staged_cap = 0;
+    if (n == 0 || A->nnz < kStagedMinEntries) return FEMGPU_OK;
+    int cap = 0;
+    for (int r = 0; r < n; r += 64) cap = std::max(cap, IA[std::min(n, r + 64)] - IA[r]);
+    if (cap > kStagedMax) return FEMGPU_OK;
+    std::vector<short> d(static_cast<size_t>(IA[n]));
+    bool fits = true;
+    for (int r = 0; r < n && fits; ++r)
+        for (int p = IA[r]; p < IA[r + 1]; ++p) {
+            const int t = JA[p] - (r & ~63);
+            fits = fits && t >= -32768 && t <= 32767;
+            d[p] = static_cast<short>(t);
+        }
+    A->staged16 = fits;
+    if (fits) {
+        FG_TRY(A->staged_d16.upload(d.data(), d.size(), ctx->stream));
+        FG_HIP(hipStreamSynchronize(ctx->stream));   // the host array ends with this call
+    }
+    A->staged_cap = (cap + 1) & ~1;
+    return FEMGPU_OK;
+}
+
+static bool staged_active(const femgpu_csr *A) { return A->spmv_lanes < 0 && A->staged_cap > 0 && A->n > 0; }
+
+template <bool RESIDUAL>
+static int staged_launch(femgpu_ctx *ctx, const femgpu_csr *A, const double *x, const double *xs, double *xout,
+                         const double *f, double *y, double *sumsq, const int *skip)
+{
+    const int n = A->n, cap = A->staged_cap, grid = xcd_grid((n + 255) / 256);
+    const size_t lds = sizeof(double) * 4 * cap;
+    if (A->staged16)
+        k_spmv_staged<short, 8, RESIDUAL><<<grid, 256, lds, ctx->stream>>>(n, cap, A->IA.p, A->staged_d16.p, A->AA.p, x, xs,
+                                                                          xout, f, y, sumsq, skip);
+    else
+        k_spmv_staged<int, 8, RESIDUAL><<<grid, 256, lds, ctx->stream>>>(n, cap, A->IA.p, A->JA.p, A->AA.p, x, xs, xout, f,
+                                                                        y, sumsq, skip);
+    FG_HIP(hipGetLastError());
+    return FEMGPU_OK;
+}
+
 template <typename T>
 static int spmv_dispatch(femgpu_ctx *ctx, const femgpu_csr *A, const T *AA, const T *x, const double *xs,
                          T *xout, T *y, const int *skip)
 {
-    const int L = A->spmv_lanes > 0 ? A->spmv_lanes : 8;   // 0 (sliced ELL) is dispatched before this
+    const int L = A->spmv_lanes > 0 ? A->spmv_lanes : default_lanes(A);   // 0 (sliced ELL) and the staged default are dispatched before this
     const long threads = static_cast<long>(A->n) * L;
     const int grid = xcd_grid(static_cast<int>((threads + 255) / 256));
     if (A->n == 0) return FEMGPU_OK;
@@ -348,6 +471,7 @@ int launch_spmv64(femgpu_ctx *ctx, const femgpu_csr *A, const double *x, const d
                   double *y, const int *skip)
 {
     if (A->n > 0 && sell64_active(A)) return sell_dispatch<double>(ctx, A, A->sell_val64.p, x, xs, xout, y, skip);
+    if (staged_active(A)) return staged_launch<false>(ctx, A, x, xs, xout, nullptr, y, nullptr, skip);
     return spmv_dispatch<double>(ctx, A, A->AA.p, x, xs, xout, y, skip);
 }
 
@@ -359,7 +483,10 @@ int launch_spmv32(femgpu_ctx *ctx, const femgpu_csr *A, const float *x, const do
 }
 
 // blocks of the fused residual launch (the XCD-rounded grid; padding blocks write zero partials)
-int residual_sumsq_blocks(const femgpu_csr *A) { return sell64_active(A) && A->n > 0 ? xcd_grid((A->n + 255) / 256) : 0; }
+int residual_sumsq_blocks(const femgpu_csr *A)
+{
+    return (sell64_active(A) || staged_active(A)) && A->n > 0 ? xcd_grid((A->n + 255) / 256) : 0;
+}
 
 int launch_residual64(femgpu_ctx *ctx, const femgpu_csr *A, const double *x, const double *f, double *r,
                       double *sumsq)
@@ -385,7 +512,8 @@ int launch_residual64(femgpu_ctx *ctx, const femgpu_csr *A, const double *x, con
         FG_HIP(hipGetLastError());
         return FEMGPU_OK;
     }
-    const int L = A->spmv_lanes > 0 ? A->spmv_lanes : 8;
+    if (staged_active(A)) return staged_launch<true>(ctx, A, x, nullptr, nullptr, f, r, sumsq, nullptr);
+    const int L = A->spmv_lanes > 0 ? A->spmv_lanes : default_lanes(A);
     const int grid = xcd_grid(static_cast<int>((static_cast<long>(A->n) * L + 255) / 256));
     switch (L) {
     case 1: k_residual<1><<<grid, 256, 0, ctx->stream>>>(A->n, A->IA.p, A->JA.p, A->AA.p, x, f, r); break;
@@ -412,7 +540,7 @@ int csr_autotune(femgpu_csr *A, femgpu_tune_info *info)
     // candidates: CSR with 1, 2, 4, 8, 16 lanes per row, then FP64 sliced ELL (lanes 0) where possible
     static constexpr int kLanes[6] = {1, 2, 4, 8, 16, 0};
     femgpu_tune_info out{};
-    out.lanes = A->spmv_lanes;
+    out.lanes = A->spmv_lanes < 0 ? 8 : A->spmv_lanes;
     if (A->n == 0) {
         if (info) *info = out;
         return FEMGPU_OK;
