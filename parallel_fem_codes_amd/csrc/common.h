@@ -296,17 +296,19 @@ struct femgpu_mesh {
     fg::DevBuf<int> type, invP, ien, lm;   // type/invP per dof, lm[nel*3*ndof]
     fg::DevBuf<int> rhs_ptr, rhs_src;   // unknown -> (element*s + i) contributions, element order
     fg::DevBuf<int> aa_ptr, aa_src;     // CSR slot -> (element*s*s + ij) contributions, element order
+                                        // (transport: only where the fused assembly does not apply)
     fg::DevBuf<int> rhs_dst, aa_dst;    // the lists are ordered by first element: list k -> unknown / slot
     fg::DevBuf<double> fe, lift;        // per element: s loads / residual entries, 9 coupling terms
     fg::DevBuf<int> mask;               // per element: Dirichlet-vertex bit mask
     fg::DevBuf<double> ke;              // element matrices when the caller passes none
-    // Fused transient assembly (CSR values and residual with no element arrays in memory): rows in
+    bool has_scheme = false;            // created with a CSR slot table
+    // Fused transport assembly (CSR values and residual with no element arrays in memory): rows in
     // blocks of compact mesh patches; per block its elements (sorted; two int4 each: vertices,
     // their equation numbers and the LDS slot of each vertex row in the block), per row thread
     // fz_ki incidence codes (LDS slot | CSR positions) and {row, first CSR slot, row length,
-    // incidences}. Built on first use; fz_state 0 unknown, 1 built, -1 not applicable (a row longer
-    // than 15 entries or with more than 16 incidences).
-    int fz_state = 0, fz_nblocks = 0, fz_slots = 0, fz_maxlen = 0, fz_ki = 0;
+    // incidences}. Built with the mesh (a rebuilt mesh's on its first transient
+    // assembly); fz_state 1 built, 0 not yet, -1 not applicable (the slot lists instead).
+    int fz_state = -1, fz_nblocks = 0, fz_slots = 0, fz_maxlen = 0, fz_ki = 0;
     fg::DevBuf<int> fz_eptr;
     fg::DevBuf<int4> fz_ent;
     fg::DevBuf<unsigned> fz_inc;
