@@ -220,12 +220,12 @@ static int csr_setup(femgpu_csr *A, int n, int nnz, const int *IA, const int *JA
         if (!rc) rc = build_stream_plan(ctx, n, IA, JA, diag.data(), true, A->sup);
         if (!rc) rc = build_stream_maps(ctx, A);
         if (!rc) rc = build_stream_factor(ctx, A, IA, JA, diag.data());
-        if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), false, A->fplan);
+        if (!rc) rc = build_rows_factor(ctx, A, IA, JA, diag.data());
     }
     if (!rc) rc = build_sell(ctx, A, IA, JA);
     if (!rc) rc = build_staged(ctx, A, IA, JA);
     if (plans & FEMGPU_PLANS_MIXED) {   // parallel FP32 ILU(0) and Jacobi iterations
-        if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), true, A->fplan_nat);
+        if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), A->fplan_nat);
         if (!rc) rc = build_jacobi_ell(ctx, A, IA, JA, diag.data());
         if (!rc) rc = build_parilu_sell(ctx, A, IA, JA, diag.data());
     }

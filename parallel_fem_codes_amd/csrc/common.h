@@ -157,12 +157,22 @@ struct StreamFactor {
     DevBuf<double> dinv;     // general, n + kStreamThreads: inverse pivots in schedule order
 };
 
-// Numeric ILU(0) plan: for every row in the lower sweep's level schedule, its CSR position, length,
-// number of L entries, and its update list -- (U entry position k of a dependency row, target slot
-// in this row, index t of the L entry it belongs to) -- in the serial factorisation's order.
+// Level-synchronous ILU(0) factorisation of rows of at most 32 entries, 16 lanes per row (factor_rows.hip).
+struct RowsFactor {
+    bool ok = false;
+    bool wide = false;       // rows with more than 16 L or 15 U entries: 8-bit codes, two passes
+    int maxlevel = 0;        // most rows of a level
+    DevBuf<int4> info;       // schedule position -> {first entry, length, L count, row}
+    DevBuf<int2> dep;        // per L entry: {first U entry of its row, its row}
+    DevBuf<unsigned long long> code;   // U columns of the (entry, L entry) pairs
+};
+
+// Update lists of the parallel factorisation: for every row its CSR position, length, number of L
+// entries, and its update list -- (U entry position k of a dependency row, target slot in this row,
+// index t of the L entry it belongs to) -- in the serial factorisation's order.
 struct FactorPlan {
     int maxrow = 0, nupd = 0, maxupd = 0;
-    DevBuf<int4> rowinfo;   // per schedule position: {p0, len, nL, first update}
+    DevBuf<int4> rowinfo;   // per row: {p0, len, nL, first update}
     DevBuf<int2> upd;       // {k, dest | t << 16}; dest == nL marks the pivot
 };
 
@@ -232,7 +242,7 @@ struct femgpu_csr {
     fg::PackedSweep plo, pup;       // packed lower / upper sweeps
     fg::StreamSweep slo, sup;       // streamed single-workgroup sweeps (used when both exist)
     int sweep_kernel = 0;           // 0: streamed when available, 1: packed
-    int factor_kernel = 0;          // 0: streamed when available, 1: level-synchronous update lists
+    int factor_kernel = 0;          // 0: streamed when available, 1: level-synchronous
     fg::DevBuf<int> stream_l2u;     // upper-schedule position -> lower-schedule position of its row
     fg::DevBuf<int> stream_pos_up;  // row -> upper-schedule position
     fg::DevBuf<double> stream_t64;  // 2n: schedule-ordered vectors of the streamed pair
@@ -247,8 +257,8 @@ struct femgpu_csr {
     bool ell16 = false;                 // the kernels read the columns as 16-bit distances from the row:
     fg::DevBuf<unsigned short> ell_dl, ell_du;   // lower i - j, upper j - i (padding 0), when all fit
     fg::DevBuf<float> ell_vl, ell_vu;   // their FP32 factor values (padding 0), refreshed with LU32
-    fg::FactorPlan fplan;           // numeric factorisation (level schedule)
-    fg::FactorPlan fplan_nat;       // the same lists in row order (parallel FP32 factorisation)
+    fg::RowsFactor rfac;            // level-synchronous factorisation (rows of at most 32 entries)
+    fg::FactorPlan fplan_nat;       // update lists in row order (parallel FP32 factorisation)
     fg::StreamFactor sfac;          // streamed single-workgroup factorisation (when available)
     // FP64 parallel ILU(0) applied by Jacobi iterations (the mixed solver's preconditioner at FP64):
     // factors in the sliced-ELL layout, strict triangles in the Jacobi sliced-ELL arrays
@@ -334,9 +344,9 @@ int build_stream_maps(femgpu_ctx *ctx, femgpu_csr *A);
 int build_stream_factor(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag);
 size_t factor_lds_bytes(const StreamSweep &P);
 int launch_stream_factor(femgpu_ctx *ctx, femgpu_csr *A);
-// natural: rows in index order (the parallel factorisation); else the lower sweep's level schedule.
-int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, bool natural,
-                      FactorPlan &F);
+int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag);
+int launch_rows_factor(femgpu_ctx *ctx, femgpu_csr *A);
+int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, FactorPlan &F);
 // LDS bytes one workgroup of the packed sweep needs for T-typed values.
 template <typename T>
 inline size_t packed_lds_bytes(const PackedSweep &P)

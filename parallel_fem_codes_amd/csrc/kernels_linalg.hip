@@ -653,109 +653,13 @@ __global__ __launch_bounds__(kFactorThreads) void k_ilu0_factor_levels(int depth
     }
 }
 
-// Numeric ILU(0) from the update lists: one persistent workgroup, rows of a level in parallel (one
-// thread per row), a barrier between levels. A row first issues all of its loads at once -- its
-// update list, the finished U values and pivots it reads, its own values -- so a level costs a few
-// memory round trips instead of one per update; the row's values and multipliers live in a private
-// LDS slice. Same operations in the same order as the serial factorisation, contraction off.
-// Longer update lists are taken in chunks of MAXU. Rows beyond the compile-time bounds (MAXROW
-// values, MAXL multipliers) take a sequential path with the same arithmetic.
-template <int MAXROW, int MAXL, int MAXU, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_ilu0_factor_lists(int depth, const int *__restrict__ lvl_ptr,
-                                                               const int4 *__restrict__ rowinfo,
-                                                               const int2 *__restrict__ upd, const int *__restrict__ JA,
-                                                               const double *__restrict__ AA, double *LU, double *Dinv,
-                                                               int *err)
-{
-#pragma clang fp contract(off)
-    __shared__ double scratch[(MAXROW + MAXL) * THREADS];
-    double *v = scratch + threadIdx.x;                 // row value e at v[e * THREADS]
-    double *dj = scratch + MAXROW * THREADS + threadIdx.x;   // pivot inverse of L entry t at dj[t * THREADS]
-    for (int l = 0; l < depth; ++l) {
-        const int q1 = lvl_ptr[l + 1];
-        for (int q = lvl_ptr[l] + threadIdx.x; q < q1; q += THREADS) {
-            const int4 ri = rowinfo[q];
-            const int p0 = ri.x, len = ri.y, nL = ri.z, ub = ri.w;
-            const int nu = rowinfo[q + 1].w - ub;   // rowinfo has a sentinel entry after the last row
-            const int i = JA[p0 + nL];
-            double piv;
-            if (len <= MAXROW && nL <= MAXL) {
-                int jr[MAXL];
-#pragma unroll
-                for (int t = 0; t < MAXL; ++t)
-                    if (t < nL) jr[t] = JA[p0 + t];
-#pragma unroll
-                for (int e = 0; e < MAXROW; ++e)
-                    if (e < len) v[e * THREADS] = AA[p0 + e];
-#pragma unroll
-                for (int t = 0; t < MAXL; ++t)
-                    if (t < nL) dj[t * THREADS] = Dinv[jr[t]];
-                int sc = 0;   // L entries [0, sc) already turned into multipliers
-                // the update list in chunks of MAXU: each chunk's list entries and U values are
-                // loaded together, then applied in list order
-                for (int u0 = 0; u0 < nu; u0 += MAXU) {
-                    int2 U[MAXU];
-                    double Uv[MAXU];
-#pragma unroll
-                    for (int u = 0; u < MAXU; ++u)
-                        if (u0 + u < nu) U[u] = upd[ub + u0 + u];
-#pragma unroll
-                    for (int u = 0; u < MAXU; ++u)
-                        if (u0 + u < nu) Uv[u] = LU[U[u].x];
-#pragma unroll
-                    for (int u = 0; u < MAXU; ++u) {
-                        if (u0 + u < nu) {
-                            const int t = U[u].y >> 16, dest = U[u].y & 0xffff;
-                            for (; sc <= t; ++sc) v[sc * THREADS] = v[sc * THREADS] * dj[sc * THREADS];
-                            v[dest * THREADS] -= v[t * THREADS] * Uv[u];
-                        }
-                    }
-                }
-                for (; sc < nL; ++sc) v[sc * THREADS] = v[sc * THREADS] * dj[sc * THREADS];
-#pragma unroll
-                for (int e = 0; e < MAXROW; ++e)
-                    if (e < len) LU[p0 + e] = v[e * THREADS];
-                piv = (nL < MAXROW) ? v[nL * THREADS] : LU[p0 + nL];
-            } else {
-                // sequential path directly on the factors in global memory
-                for (int e = 0; e < len; ++e) LU[p0 + e] = AA[p0 + e];
-                int u = ub;
-                const int ue = ub + nu;
-                for (int t = 0; t < nL; ++t) {
-                    const double lij = LU[p0 + t] * Dinv[JA[p0 + t]];
-                    LU[p0 + t] = lij;
-                    for (; u < ue && (upd[u].y >> 16) == t; ++u)
-                        LU[p0 + (upd[u].y & 0xffff)] -= lij * LU[upd[u].x];
-                }
-                piv = LU[p0 + nL];
-            }
-            if (piv == 0.0) {
-                __hip_atomic_store(err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                Dinv[i] = 0.0;
-            } else {
-                Dinv[i] = 1.0 / piv;
-            }
-        }
-        __syncthreads();
-    }
-}
-
 int launch_ilu_factor(femgpu_ctx *ctx, femgpu_csr *A)
 {
     if (A->n == 0) return FEMGPU_OK;
-    const FactorPlan &F = A->fplan;
     if (A->sfac.ok && A->factor_kernel == 0) {
         FG_TRY(launch_stream_factor(ctx, A));
-    } else if (F.maxrow <= 8) {
-        k_ilu0_factor_lists<8, 8, 24, 512><<<1, 512, 0, ctx->stream>>>(A->plo.depth, A->plo.lvl_ptr.p, F.rowinfo.p,
-                                                                        F.upd.p, A->JA.p, A->AA.p, A->LU.p, A->Dinv.p,
-                                                                        ctx->err.p);
-    } else if (F.maxrow <= 32) {
-        // 256 threads: the levels of the 9x9-block systems hold up to ~260 rows (513 x 513 cavity:
-        // 180 ms per factorisation against 220 ms with 128 threads); 96 KB of LDS
-        k_ilu0_factor_lists<32, 16, 32, 256><<<1, 256, 0, ctx->stream>>>(A->plo.depth, A->plo.lvl_ptr.p, F.rowinfo.p,
-                                                                          F.upd.p, A->JA.p, A->AA.p, A->LU.p, A->Dinv.p,
-                                                                          ctx->err.p);
+    } else if (A->rfac.ok) {
+        FG_TRY(launch_rows_factor(ctx, A));
     } else {
         FG_HIP(hipMemcpyAsync(A->LU.p, A->AA.p, sizeof(double) * A->nnz, hipMemcpyDeviceToDevice, ctx->stream));
         k_ilu0_factor_levels<<<1, kFactorThreads, 0, ctx->stream>>>(A->plo.depth, A->plo.lvl_ptr.p, A->plo.row_of.p,

@@ -1,0 +1,76 @@
+"""The level-synchronous ILU(0) factorisation (16 lanes per row) at the edges of its row shapes: factors
+bit-identical to the CPU oracle's serial elimination."""
+import numpy as np
+import pytest
+
+from parallel_fem_codes_amd import fem
+
+pytestmark = pytest.mark.gpu
+
+
+def random_pattern(n, reach, max_l, max_u, rng):
+    """Rows with up to max_l strict lower and max_u strict upper entries within reach of the diagonal."""
+    rows = []
+    for i in range(n):
+        lo, hi = np.arange(max(0, i - reach), i), np.arange(i + 1, min(n, i + reach + 1))
+        lo = rng.choice(lo, min(len(lo), rng.integers(0, max_l + 1)), replace=False)
+        hi = rng.choice(hi, min(len(hi), rng.integers(0, max_u + 1)), replace=False)
+        rows.append(np.sort(np.concatenate([lo, [i], hi])))
+    IA = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    return IA, np.concatenate(rows).astype(np.int32)
+
+
+def block_pattern(m, ndof):
+    """The SYMRCM-ordered pattern of an m x m mesh with ndof unknowns per node (rows of 7 ndof entries)."""
+    x, y, ien = fem.structured_mesh(m, m)
+    t = np.repeat(fem.boundary_types(x, y), ndof).astype(np.int32)
+    inv, neq = fem.number_unknowns(t, ndof)
+    c = fem.csr_Initialization(fem.Fill_LM(ien, t, inv, neq, ndof), 3 * ndof, neq, "SYMRCM", type_=t, invP_id=inv)
+    return c.IA, c.JA
+
+
+@pytest.mark.parametrize("case", ["n1", "diag300", "l16u15", "l17u14", "l15u16", "l31", "u31", "wide_level", "ns24",
+                                  "euler16", "euler40"])
+def test_factor_rows_bit_exact(oracle, case):
+    rng = np.random.default_rng(len(case) * 7 + ord(case[-1]))
+    if case == "n1":
+        IA, JA = np.array([0, 1], np.int32), np.array([0], np.int32)
+    elif case == "diag300":
+        IA, JA = np.arange(301, dtype=np.int32), np.arange(300, dtype=np.int32)   # one level
+    elif case == "wide_level":
+        IA, JA = random_pattern(3000, 1500, 9, 9, rng)      # levels of several hundred rows
+    elif case.startswith("ns"):
+        IA, JA = block_pattern(24, 3)
+    elif case.startswith("euler"):
+        IA, JA = block_pattern(int(case[5:]), 4)
+    else:
+        l, u = {"l16u15": (16, 15), "l17u14": (17, 14), "l15u16": (15, 16), "l31": (31, 0), "u31": (0, 31)}[case]
+        IA, JA = random_pattern(700, 60, l, u, rng)
+    n = len(IA) - 1
+    AA = rng.uniform(-1, 1, len(JA))
+    rows = np.repeat(np.arange(n), np.diff(IA))
+    AA[JA == rows] = 2.0 + np.bincount(rows, weights=np.abs(AA), minlength=n)
+    dev = fem.Device(0)
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_factor_kernel("lists")
+    A.set_values(AA)
+    LUo, Dio, rc = oracle.ilu0_factor(IA, JA, np.append(AA, 0.0))
+    assert rc == 0
+    for _ in range(2):
+        A.ilu0_factor()
+        LU, Di = A.ilu0_factors()
+        assert np.array_equal(LU, LUo[:-1]) and np.array_equal(Di, Dio)
+
+
+def test_factor_rows_zero_pivot():
+    """A zero pivot in the middle of the schedule is reported."""
+    IA, JA = block_pattern(12, 3)
+    n = len(IA) - 1
+    rows = np.repeat(np.arange(n), np.diff(IA))
+    AA = np.where(JA == rows, 4.0, 0.0)
+    AA[(JA == rows) & (rows == n // 2)] = 0.0
+    dev = fem.Device(0)
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(AA)
+    with pytest.raises(Exception, match="zero pivot"):
+        A.ilu0_factor()
