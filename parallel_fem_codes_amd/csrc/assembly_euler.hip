@@ -4,20 +4,22 @@
 // Jacobians of Ax_Ay_calculations.c (dimensionless :3-53 or dimensional :55-99) and the CAU
 // shock-capture coefficient of Delta_CAU.c:4-83.
 //
-// One thread per element. The element matrices are built row by row: for dof row i of vertex a,
-// the Galerkin/SUPG convection block C_a = (b_a Ax + c_a Ay)/6, the SUPG products
-// b_a (AxAx, AxAy) + c_a (AyAx, AyAy) and the CAU coupling give every column, and the row's
-// residual and Ae entries are formed on the spot. Each quantity is evaluated in the reference's
-// operation order with contraction off; the reference's hand-expanded 4x4 products skip only
-// terms with a structural zero factor, so the dense products used here have equal values.
+// The element matrices are built row by row: for dof row i of vertex a, the Galerkin/SUPG convection
+// block C_a = (b_a Ax + c_a Ay)/6, the SUPG products b_a (AxAx, AxAy) + c_a (AyAx, AyAy) and the CAU
+// coupling give every column, and the row's residual and Ae entries are formed on the spot. Each
+// quantity is evaluated in the reference's operation order with contraction off; the reference's
+// hand-expanded 4x4 products skip only terms with a structural zero factor, so the dense products
+// used here have equal values.
 // Global accumulation is the element-order gather shared with the Navier-Stokes assembly.
 #include "common.h"
+#include "device_util.h"
 
 namespace fg {
 
 struct EulerIn {
     const double *x, *y, *presc, *u, *du;
     const int *type, *invP, *ien;
+    int neq;
     femgpu_euler_problem pb;
 };
 
@@ -82,57 +84,97 @@ __device__ __forceinline__ double a0_form_dev(const double A0[4][4], const doubl
            w[2] * (A0[2][2] * w[2] + 2.0 * A0[2][3] * w[3]) + w[3] * A0[3][3] * w[3];
 }
 
-// Entry (i, j) of A B, accumulated over k from the k = 0 term.
-__device__ __forceinline__ double mul4_entry(const double A[4][4], const double B[4][4], int i, int j)
+// Orders a wavefront's LDS writes before its later LDS reads of other lanes' words, and the reverse.
+__device__ __forceinline__ void wave_lds_fence()
 {
-#pragma clang fp contract(off)
-    double acc = A[i][0] * B[0][j];
-#pragma unroll
-    for (int k = 1; k < 4; ++k) acc += A[i][k] * B[k][j];
-    return acc;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ __launch_bounds__(256) void k_elem_euler(int nel, EulerIn in, double *__restrict__ Ae, double *__restrict__ Res)
+// Component j of a quad's value: lane j of each four lanes to all four.
+template <int J>
+__device__ __forceinline__ double quad_bcast(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), J * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), J * 0x55, 0xf, 0xf, true);
+    return __longlong_as_double(static_cast<long long>(static_cast<unsigned>(lo)) | (static_cast<long long>(hi) << 32));
+}
+__device__ __forceinline__ void quad_all(double v, double (&all)[4])
+{
+    all[0] = quad_bcast<0>(v);
+    all[1] = quad_bcast<1>(v);
+    all[2] = quad_bcast<2>(v);
+    all[3] = quad_bcast<3>(v);
+}
+__device__ __forceinline__ double sel4(int i, double v0, double v1, double v2, double v3)
+{
+    return i < 2 ? (i == 0 ? v0 : v1) : (i == 2 ? v2 : v3);
+}
+
+// Four lanes per element, lane i of a quad on dof i: it loads its dof of the three vertices, forms its
+// component of the element's state and gradients, exchanges components with the quad (DPP moves), evaluates
+// the rest of the element's state, and forms rows i, 4 + i and 8 + i. What bounds it: the 1 152 bytes an
+// element writes (184 MB at 401 x 201 nodes), about forty FP64 divisions (half of them shared out over the
+// quad) and 2 900 FP64 operations of entries. One thread per element held the whole element in registers
+// (one wavefront per SIMD) and stored its rows 64 cache lines per instruction: 105 us. Here a wavefront turns
+// its rows through LDS and stores runs of 384 bytes: 74 us (160 000 elements; about 2 200 instructions a
+// lane, 36 us of issue at two wavefronts per SIMD).
+__global__ __launch_bounds__(256, 2) void k_elem_euler(int nel, EulerIn in, double *__restrict__ Ae, double *__restrict__ Res)
 {
 #pragma clang fp contract(off)
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= nel) return;
+    __shared__ double turn_all[4 * 64 * 13];
+    const int l = threadIdx.x & 63, i = l & 3;
+    const int ew = xcd_block() * 64 + static_cast<int>(threadIdx.x >> 6) * 16;   // the wavefront's 16 elements
+    if (ew >= nel) return;
+    const int n = min(16, nel - ew), e = ew + min(l >> 2, n - 1);   // idle quads repeat the last element
+    double *turn = turn_all + (threadIdx.x >> 6) * (64 * 13);
     const femgpu_euler_problem &p = in.pb;
     const double third = 1.0 / 3.0, sixth = 1.0 / 6.0;
     const double gamma = p.gamma, alpha = p.alpha, delta_t = p.dt;
-    int v[3];
+    int v[3], eq[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) v[a] = in.ien[3 * e + a];
     const double X0 = in.x[v[0]], X1 = in.x[v[1]], X2 = in.x[v[2]];
     const double Y0 = in.y[v[0]], Y1 = in.y[v[1]], Y2 = in.y[v[2]];
+    // this lane's dof of the vertices: mark, number and prescribed value, then state
+    double U[3], dU[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int q = 4 * v[a] + i;
+        eq[a] = in.type[q] > 0 ? in.invP[q] : -1;
+        U[a] = in.presc[q];
+        dU[a] = 0.0;
+    }
+    if (in.neq > 0)   // else every dof is prescribed
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const int q = eq[a] >= 0 ? eq[a] : 0;
+            const double un = in.u[q], dn = in.du[q];
+            U[a] = eq[a] >= 0 ? un : U[a];
+            dU[a] = eq[a] >= 0 ? dn : 0.0;
+        }
     const double b[3] = {Y1 - Y2, Y2 - Y0, Y0 - Y1};
     const double c[3] = {X2 - X1, X0 - X2, X1 - X0};
     const double twoArea = fabs(c[2] * b[1] - c[1] * b[2]);
     const double Area = 0.5 * twoArea;
-    double Ue[12], dUe[12];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int q = 4 * v[a] + k;
-            const bool unk = in.type[q] > 0;
-            Ue[4 * a + k] = unk ? in.u[in.invP[q]] : in.presc[q];
-            dUe[4 * a + k] = unk ? in.du[in.invP[q]] : 0.0;
-        }
-    double Ub[4], dUb[4], gUx[4], gUy[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        Ub[i] = (Ue[i] + Ue[i + 4] + Ue[i + 8]) * third;
-        dUb[i] = (dUe[i] + dUe[i + 4] + dUe[i + 8]) * third;
-        gUx[i] = (Ue[i] * b[0] + Ue[i + 4] * b[1] + Ue[i + 8] * b[2]) / twoArea;
-        gUy[i] = (Ue[i] * c[0] + Ue[i + 4] * c[1] + Ue[i + 8] * c[2]) / twoArea;
-    }
+    const double gxi = (U[0] * b[0] + U[1] * b[1] + U[2] * b[2]) / twoArea;
+    const double gyi = (U[0] * c[0] + U[1] * c[1] + U[2] * c[2]) / twoArea;
+    double Ub[4], gUx[4], gUy[4];
+    quad_all((U[0] + U[1] + U[2]) * third, Ub);
+    quad_all(gxi, gUx);
+    quad_all(gyi, gUy);
     const double v1 = Ub[1] / Ub[0], v2 = Ub[2] / Ub[0], E = Ub[3] / Ub[0];
     double Ax[4][4], Ay[4][4];
     euler_jacobians_dev(p, Ub, Ax, Ay);
     // CAU coefficient (Delta_CAU.c) with the entropy-variable metric A0^-1 (:134-160)
     double delta = 0.0;
     if (p.shock) {
+        double dUb[4], gkx[4], gky[4], LUh[4];
+        quad_all((dU[0] + dU[1] + dU[2]) * third, dUb);
+        quad_all((b[0] * gxi + c[0] * gyi) / twoArea, gkx);
+        quad_all((b[1] * gxi + c[1] * gyi) / twoArea, gky);
         const double nU = (Ub[1] * Ub[1]) + (Ub[2] * Ub[2]);
         const double rho_i = Ub[3] - ((nU * 0.5) / Ub[0]);
         const double V2 = Ub[1] / rho_i, V3 = Ub[2] / rho_i, V4 = (-Ub[0]) / rho_i;
@@ -149,13 +191,7 @@ __global__ __launch_bounds__(256) void k_elem_euler(int nel, EulerIn in, double 
         A0[2][2] = rhoi_e * (V3 * V3 - V4);
         A0[2][3] = rhoi_e * (V3 * V4);
         A0[3][3] = rhoi_e * V4 * V4;
-        A0[1][0] = A0[0][1];
-        A0[2][0] = A0[0][2];
-        A0[2][1] = A0[1][2];
-        A0[3][0] = A0[0][3];
-        A0[3][1] = A0[1][3];
-        A0[3][2] = A0[2][3];
-        double AgUx[4], AgUy[4], gkx[4], gky[4], LUh[4];
+        double AgUx[4], AgUy[4];
         AgUx[0] = gUx[1];
         AgUx[1] = Ax[1][0] * gUx[0] + Ax[1][1] * gUx[1] + Ax[1][2] * gUx[2] + Ax[1][3] * gUx[3];
         AgUx[2] = Ax[2][0] * gUx[0] + Ax[2][1] * gUx[1] + Ax[2][2] * gUx[2];
@@ -165,11 +201,7 @@ __global__ __launch_bounds__(256) void k_elem_euler(int nel, EulerIn in, double 
         AgUy[2] = Ay[2][0] * gUy[0] + Ay[2][1] * gUy[1] + Ay[2][2] * gUy[2] + Ay[2][3] * gUy[3];
         AgUy[3] = Ay[3][0] * gUy[0] + Ay[3][1] * gUy[1] + Ay[3][2] * gUy[2] + Ay[3][3] * gUy[3];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            gkx[i] = (b[0] * gUx[i] + c[0] * gUy[i]) / twoArea;
-            gky[i] = (b[1] * gUx[i] + c[1] * gUy[i]) / twoArea;
-            LUh[i] = dUb[i] + AgUx[i] + AgUy[i];
-        }
+        for (int k = 0; k < 4; ++k) LUh[k] = dUb[k] + AgUx[k] + AgUy[k];
         const double n_gk = sqrt(a0_form_dev(A0, gkx) + a0_form_dev(A0, gky));
         const double n_LUh = sqrt(a0_form_dev(A0, LUh));
         const double n_gU = sqrt(a0_form_dev(A0, gUx) + a0_form_dev(A0, gUy));
@@ -198,56 +230,84 @@ __global__ __launch_bounds__(256) void k_elem_euler(int nel, EulerIn in, double 
     const double Kc01 = delta4area * (b[0] * b[1] + c[0] * c[1]);
     const double Kc02 = delta4area * (b[0] * b[2] + c[0] * c[2]);
     const double Kc12 = delta4area * (b[1] * b[2] + c[1] * c[2]);
-    double *A = Ae + 144 * static_cast<size_t>(e);
-    double *R = Res + 12 * static_cast<size_t>(e);
+    // row i of the Jacobians and of their four products, each entry accumulated over k from the k = 0 term;
+    // the rows 4a + i share them
+    double xi[4], yi[4], Pxx[4], Pxy[4], Pyx[4], Pyy[4], C[3][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // row i of the four Jacobian products, shared by the three vertex rows 4a+i
-        double Pxx[4], Pxy[4], Pyx[4], Pyy[4];
+    for (int k = 0; k < 4; ++k) {
+        xi[k] = sel4(i, Ax[0][k], Ax[1][k], Ax[2][k], Ax[3][k]);
+        yi[k] = sel4(i, Ay[0][k], Ay[1][k], Ay[2][k], Ay[3][k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            Pxx[j] = mul4_entry(Ax, Ax, i, j);
-            Pxy[j] = mul4_entry(Ax, Ay, i, j);
-            Pyx[j] = mul4_entry(Ay, Ax, i, j);
-            Pyy[j] = mul4_entry(Ay, Ay, i, j);
+            Pxx[j] = k == 0 ? xi[0] * Ax[0][j] : Pxx[j] + xi[k] * Ax[k][j];
+            Pxy[j] = k == 0 ? xi[0] * Ay[0][j] : Pxy[j] + xi[k] * Ay[k][j];
+            Pyx[j] = k == 0 ? yi[0] * Ax[0][j] : Pyx[j] + yi[k] * Ax[k][j];
+            Pyy[j] = k == 0 ? yi[0] * Ay[0][j] : Pyy[j] + yi[k] * Ay[k][j];
         }
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const int o1 = a == 0 ? 1 : 0, o2 = a == 2 ? 1 : 2;
-            const double Kca1 = (a == 0) ? Kc01 : (a == 1 ? Kc01 : Kc02);   // Kcau(a, o1)
-            const double Kca2 = (a == 0) ? Kc02 : Kc12;                      // Kcau(a, o2)
-            double MdU = 0, KU = 0;
+    for (int a = 0; a < 3; ++a)
 #pragma unroll
-            for (int bb = 0; bb < 3; ++bb) {
-                const double Kab = (a == bb) ? 0.0 : ((a + bb == 1) ? Kc01 : (a + bb == 2 ? Kc02 : Kc12));
+        for (int j = 0; j < 4; ++j) C[a][j] = (b[a] * xi[j] + c[a] * yi[j]) * sixth;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const double Ca_ij = (b[a] * Ax[i][j] + c[a] * Ay[i][j]) * sixth;
-                    const double Mpg = Ca_ij * tau;
-                    const double AXij = b[a] * Pxx[j] + c[a] * Pyx[j];
-                    const double AYij = b[a] * Pxy[j] + c[a] * Pyy[j];
-                    double m, k;
-                    if (i == j) m = (a == bb ? Mg1 : Mg2) + Mpg;
-                    else m = Mpg;
-                    if (a == bb) {
-                        const double k1v = tau4area * (b[o1] * AXij + c[o1] * AYij);
-                        const double k2v = tau4area * (b[o2] * AXij + c[o2] * AYij);
-                        k = Ca_ij - (k1v + k2v);
-                        if (i == j) k = k - (Kca1 + Kca2);
-                    } else {
-                        const double kp = tau4area * (b[bb] * AXij + c[bb] * AYij);
-                        const double Cb_ij = (b[bb] * Ax[i][j] + c[bb] * Ay[i][j]) * sixth;
-                        k = Cb_ij + kp;
-                        if (i == j) k = k + Kab;
-                    }
-                    const int col = 4 * bb + j;
-                    MdU += m * dUe[col];
-                    KU += k * Ue[col];
-                    A[12 * (4 * a + i) + col] = m + alpha * delta_t * k;
+    for (int a = 0; a < 3; ++a) {
+        const int o1 = a == 0 ? 1 : 0, o2 = a == 2 ? 1 : 2;
+        const double Kca1 = a == 2 ? Kc02 : Kc01, Kca2 = a == 0 ? Kc02 : Kc12;   // Kcau(a, o1), Kcau(a, o2)
+        double AX[4], AY[4], row[12];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            AX[j] = b[a] * Pxx[j] + c[a] * Pyx[j];
+            AY[j] = b[a] * Pxy[j] + c[a] * Pyy[j];
+        }
+        double MdU = 0, KU = 0;
+#pragma unroll
+        for (int bb = 0; bb < 3; ++bb) {
+            const double Kab = a + bb == 1 ? Kc01 : a + bb == 2 ? Kc02 : Kc12;   // a != bb
+            double Ue[4], dUe[4];
+            quad_all(U[bb], Ue);
+            quad_all(dU[bb], dUe);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool diag = i == j;
+                const double Mpg = C[a][j] * tau;
+                const double m = diag ? (a == bb ? Mg1 : Mg2) + Mpg : Mpg;
+                double k;
+                if (a == bb) {
+                    const double k1v = tau4area * (b[o1] * AX[j] + c[o1] * AY[j]);
+                    const double k2v = tau4area * (b[o2] * AX[j] + c[o2] * AY[j]);
+                    k = C[a][j] - (k1v + k2v);
+                    k = diag ? k - (Kca1 + Kca2) : k;
+                } else {
+                    const double kp = tau4area * (b[bb] * AX[j] + c[bb] * AY[j]);
+                    k = C[bb][j] + kp;
+                    k = diag ? k + Kab : k;
                 }
+                MdU += m * dUe[j];
+                KU += k * Ue[j];
+                row[4 * bb + j] = m + alpha * delta_t * k;
             }
-            R[4 * a + i] = -MdU - KU;
         }
+        if ((l >> 2) < n) Res[12 * static_cast<size_t>(e) + 4 * a + i] = -MdU - KU;
+        // value k of row i of element r at 144 r + 48 a + 12 i + k: turned so that lanes store in order
+        double *dst = Ae + 144 * static_cast<size_t>(ew) + 48 * a;
+#pragma unroll
+        for (int k = 0; k < 12; ++k) turn[l * 13 + k] = row[k];
+        wave_lds_fence();
+        double w[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+            const int q = k * 64 + l, r = q / 12;
+            w[k] = turn[r * 13 + (q - 12 * r)];
+        }
+        wave_lds_fence();   // the next rows reuse the part
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+            const int q = k * 64 + l, r = q / 48;
+            if (r < n) dst[144 * r + (q - 48 * r)] = w[k];
+        }
+        __builtin_amdgcn_sched_barrier(0);   // one vertex's rows at a time: their registers are reused
     }
 }
 
@@ -279,9 +339,10 @@ extern "C" int femgpu_assemble_euler(femgpu_mesh *M, const femgpu_euler_problem 
     in.type = M->type.p;
     in.invP = M->invP.p;
     in.ien = M->ien.p;
+    in.neq = M->neq;
     in.pb = *pb;
     if (M->nel > 0) {
-        k_elem_euler<<<(M->nel + 255) / 256, 256, 0, ctx->stream>>>(M->nel, in, Ae, M->fe.p);
+        k_elem_euler<<<xcd_grid((M->nel + 63) / 64), 256, 0, ctx->stream>>>(M->nel, in, Ae, M->fe.p);
         FG_HIP(hipGetLastError());
     }
     return launch_block_gathers(M, Ae, d_R, d_AA);

@@ -294,7 +294,17 @@ struct femgpu_ebe {
     fg::DevBuf<int> col32v;         // unknowns (NEQ: the sink)
     fg::DevBuf<int> src;            // incidence slot -> e*s*s + ndof*a*s (its rows in element order), -1 padding
     fg::DevBuf<double> val;         // FP64 values in the gathered layout
-    fg::DevBuf<float> val32;        // FP32 copy (mixed-precision inner solver)
+    // FP32 product (mixed-precision inner solver): node block rows -- a group's column nodes, the element
+    // blocks of each summed; slice sl owns block rows [bptr[sl], bptr[sl+1])
+    int nslices = 0, nbrows = 0, maxblk = 0;
+    bool wide_slots = false;        // a node with too many column nodes for the fill kernel's LDS
+    fg::DevBuf<int> bptr;           // slice -> first block row (nslices + 1)
+    fg::DevBuf<int> blen;           // group -> column nodes
+    fg::DevBuf<short> bcol16;       // (block row*64 + lane)*ndof + dof: columns, as col16v
+    fg::DevBuf<int> bcol32;         // or as col32v
+    fg::DevBuf<unsigned> slots;     // incidence slot -> block rows of its three column nodes (8 bits each, 255
+                                    // none; three words per incidence with wide_slots)
+    fg::DevBuf<float> val32;
     bool has_values = false;
 };
 

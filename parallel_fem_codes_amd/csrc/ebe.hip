@@ -99,60 +99,236 @@ __global__ void k_ebe_zero(int n, T *__restrict__ q, const int *__restrict__ ski
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) q[i] = T(0);
 }
 
-// Element matrices (element order, ebe_assembly.c layout) into the gathered layout, FP64 and FP32.
+// The FP32 product, on node block rows: a node's element blocks that share a column node are summed (in
+// FP64, in element order, by the fill kernel below) and rounded to FP32 once, so a node of six triangles
+// reads 7 blocks of ND x ND values instead of 6 x 3 -- the product streams values, so that is what it costs:
+// 801 x 401 nodes, ND = 4, 29 us back to back and 39.6 us from HBM (170 MB; 81 us on the FP32 copy of
+// the element rows, 412 MB). The FP64 product keeps the element rows: its sums are the reference's, bit for bit.
+// Block row r of lane l: ND values of dof row d at ((r*ND + d)*64 + l)*ND, the ND columns at
+// (r*64 + l)*ND.
 template <int ND>
-__global__ __launch_bounds__(256) void k_ebe_fill(int nslots, const int *__restrict__ src, const double *__restrict__ Ae,
-                                                  double *__restrict__ val, float *__restrict__ val32)
+struct NodeVec {
+    float v[ND];
+};
+
+template <typename CT, int ND, int U>
+__global__ __launch_bounds__(256) void k_node_rows(int ngroups, int NEQ, const int *__restrict__ bptr,
+                                                   const int *__restrict__ blen, const int *__restrict__ eq,
+                                                   const int *__restrict__ key, const CT *__restrict__ col,
+                                                   const float *__restrict__ val, const float *__restrict__ P,
+                                                   float *__restrict__ Q, const int *__restrict__ skip)
 {
-    constexpr int S = 3 * ND;
-    const int q = blockIdx.x * 256 + static_cast<int>(threadIdx.x);
-    if (q >= nslots) return;
-    const size_t r = static_cast<size_t>(q >> 6);
-    const int l = q & 63, base = src[q];
+    if (skip && *skip) return;
+    const int g = xcd_block() * 256 + static_cast<int>(threadIdx.x);
+    if (g >= ngroups) return;
+    const int sl = g >> 6, l = g & 63;
+    const int r0 = bptr[sl], n = blen[g];
+    const int kg = key ? key[g] : 0;
+    double acc[ND];   // FP32 products are exact in FP64: one rounding at the end
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+    for (int d = 0; d < ND; ++d) acc[d] = 0.0;
+    for (int j = 0; j < n; j += U) {
+        NodeVec<ND> a[U][ND];
+        float p[U][ND];
 #pragma unroll
-        for (int b = 0; b < S; ++b) {
-            const double v = base >= 0 ? Ae[static_cast<size_t>(base) + d * S + b] : 0.0;
-            const size_t o = ((r * ND + d) * S + b) * 64 + l;
-            val[o] = v;
-            val32[o] = static_cast<float>(v);
+        for (int u = 0; u < U; ++u) {   // block rows past the list re-read the batch's first, not added
+            const size_t r = static_cast<size_t>(r0 + (j + u < n ? j + u : j));
+            CT c[ND];
+#pragma unroll
+            for (int b = 0; b < ND; ++b) c[b] = col[(r * 64 + l) * ND + b];
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                const float *src = val + ((r * ND + d) * 64 + l) * ND;
+                if constexpr (ND == 4) {
+                    const float4 w = *reinterpret_cast<const float4 *>(src);
+                    a[u][d].v[0] = w.x, a[u][d].v[1] = w.y, a[u][d].v[2] = w.z, a[u][d].v[3] = w.w;
+                } else {
+#pragma unroll
+                    for (int b = 0; b < ND; ++b) a[u][d].v[b] = src[b];
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < ND; ++b) {
+                const int idx = ebe_col<CT>(c[b], kg, NEQ);
+                const float pv = P[idx >= 0 ? idx : 0];
+                p[u][b] = idx >= 0 ? pv : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (j + u < n) {
+#pragma unroll
+                for (int d = 0; d < ND; ++d)
+#pragma unroll
+                    for (int b = 0; b < ND; ++b)
+                        acc[d] = fma(static_cast<double>(a[u][d].v[b]), static_cast<double>(p[u][b]), acc[d]);
+            }
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        const int q = eq[(static_cast<size_t>(sl) * ND + d) * 64 + l];
+        if (q < NEQ) Q[q] = static_cast<float>(acc[d]);
+    }
+}
+
+// Element matrices (element order, ebe_assembly.c layout) into the gathered FP64 layout and the FP32 node
+// block rows. One wavefront per (slice, dof row d): per incidence row it reads the 64 element rows in
+// order -- lane l the l-th value of the rows one after the other, so a load covers whole rows instead
+// of 64 strided words -- turns them through LDS, writes them column-major, and adds them to the lane's block
+// row in LDS, which it rounds and writes at the end. Both sides are streams: 401 x 201
+// nodes, ND = 4, 98 us for 410 MB (136 us with a thread per incidence, whose loads and stores were strided, for
+// 470 MB). RB incidence rows have their loads in flight together; 2 for ND > 1: one or three are slower at
+// 61 x 31 nodes or at 801 x 401 (7.7 / 383 us; 8.6 / 374 and 7.6 / 391). Nodes with more
+// than kFillBlocks column nodes (LDS) take k_node_rows_fill for their FP32 rows (ACC = false here).
+constexpr int kFillBlocks = 24;
+
+template <int ND, int RB, bool ACC>
+__global__ __launch_bounds__(64) void k_ebe_fill(const int *__restrict__ iptr, const int *__restrict__ bptr,
+                                                 const int *__restrict__ src, const unsigned *__restrict__ slots,
+                                                 const double *__restrict__ Ae, double *__restrict__ val,
+                                                 float *__restrict__ val32)
+{
+    constexpr int S = 3 * ND, LD = S + 1;
+    extern __shared__ double fill_lds[];
+    double *turn = fill_lds, *acc = fill_lds + RB * 64 * LD;
+    const int sl = blockIdx.x / ND, d = blockIdx.x % ND, l = threadIdx.x;
+    const int nb = ACC ? bptr[sl + 1] - bptr[sl] : 0;
+    if (ACC)
+        for (int k = 0; k < nb * ND; ++k) acc[k * 64 + l] = 0.0;
+    const int r1 = iptr[sl + 1];
+    for (int r = iptr[sl]; r < r1; r += RB) {   // RB incidence rows, their loads issued together
+        int base[RB];
+        unsigned sc[RB];
+        double w[RB][S];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const int ri = r + i < r1 ? r + i : r;
+            base[i] = src[ri * 64 + l];
+            sc[i] = ACC ? slots[ri * 64 + l] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int k = 0; k < S; ++k) {   // value k * 64 + l of the 64 rows
+                const int q = k * 64 + l, inc = q / S, b = q - inc * S;
+                const int ib = __shfl(base[i], inc, 64);
+                w[i][k] = Ae[static_cast<size_t>(ib >= 0 ? ib : 0) + d * S + b];   // padding dropped below
+            }
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int k = 0; k < S; ++k) {
+                const int q = k * 64 + l, inc = q / S, b = q - inc * S;
+                turn[(i * 64 + inc) * LD + b] = w[i][k];
+            }
+        __syncthreads();   // one wavefront: orders its LDS writes before the reads
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            if (r + i >= r1) break;
+            double v[S];
+#pragma unroll
+            for (int b = 0; b < S; ++b) {
+                const double t = turn[(i * 64 + l) * LD + b];
+                v[b] = base[i] >= 0 ? t : 0.0;
+            }
+            double *o = val + (static_cast<size_t>(r + i) * ND + d) * S * 64 + l;
+#pragma unroll
+            for (int b = 0; b < S; ++b) o[b * 64] = v[b];
+            if (ACC && base[i] >= 0) {
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    const unsigned s = (sc[i] >> (8 * a)) & 255u;
+                    if (s == 255u) continue;   // a column node without unknowns
+#pragma unroll
+                    for (int c = 0; c < ND; ++c) acc[(s * ND + c) * 64 + l] += v[ND * a + c];
+                }
+            }
+        }
+        __syncthreads();   // the turned rows have been read
+    }
+    if (ACC)
+        for (int j = 0; j < nb; ++j) {
+            float *o = val32 + ((static_cast<size_t>(bptr[sl] + j) * ND + d) * 64 + l) * ND;
+            if constexpr (ND == 4) {
+                *reinterpret_cast<float4 *>(o) = make_float4(
+                    static_cast<float>(acc[(j * 4) * 64 + l]), static_cast<float>(acc[(j * 4 + 1) * 64 + l]),
+                    static_cast<float>(acc[(j * 4 + 2) * 64 + l]), static_cast<float>(acc[(j * 4 + 3) * 64 + l]));
+            } else {
+#pragma unroll
+                for (int c = 0; c < ND; ++c) o[c] = static_cast<float>(acc[(j * ND + c) * 64 + l]);
+            }
         }
 }
 
-template <typename T, typename CT, int ND, int U>
-static void gather_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const T *vals, const T *P, T *Q, const int *skip)
+// The FP32 node block rows from the gathered FP64 rows, a thread per (block row, lane, dof row), for
+// operators with a node of more than kFillBlocks column nodes.
+template <int ND>
+__global__ __launch_bounds__(256) void k_node_rows_fill(const int *__restrict__ iptr, const int *__restrict__ bptr,
+                                                        const int *__restrict__ src,
+                                                        const unsigned *__restrict__ slots,
+                                                        const double *__restrict__ val, float *__restrict__ val32)
 {
-    const int grid = xcd_grid((E->ngroups + 255) / 256);
-    const CT *col;
-    if constexpr (sizeof(CT) == 2) col = E->col16v.p;
-    else col = E->col32v.p;
-    k_ebe_gather<T, CT, ND, U><<<grid, 256, 0, ctx->stream>>>(E->ngroups, E->NEQ, E->iptr.p, E->len.p, E->eq.p,
-                                                              E->col16 ? E->key.p : nullptr, col, vals, P, Q, skip);
+    constexpr int S = 3 * ND;
+    const int sl = blockIdx.x / ND, d = blockIdx.x % ND, l = threadIdx.x & 63;
+    for (int j = bptr[sl] + static_cast<int>(threadIdx.x >> 6); j < bptr[sl + 1]; j += 4) {
+        double acc[ND];
+#pragma unroll
+        for (int c = 0; c < ND; ++c) acc[c] = 0.0;
+        for (int r = iptr[sl]; r < iptr[sl + 1]; ++r) {
+            if (src[r * 64 + l] < 0) continue;
+            for (int a = 0; a < 3; ++a) {
+                const unsigned s = slots[(static_cast<size_t>(r) * 64 + l) * 3 + a];
+                if (s != static_cast<unsigned>(j - bptr[sl])) continue;
+#pragma unroll
+                for (int c = 0; c < ND; ++c) acc[c] += val[((static_cast<size_t>(r) * ND + d) * S + ND * a + c) * 64 + l];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < ND; ++c)
+            val32[((static_cast<size_t>(j) * ND + d) * 64 + l) * ND + c] = static_cast<float>(acc[c]);
+    }
 }
 
-template <typename T>
-static int ebe_product(femgpu_ctx *ctx, const femgpu_ebe *E, const T *vals, const T *P, T *Q, const int *skip)
+template <typename CT, int ND, int U, int U32>
+static void gather_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const CT *col, const CT *bcol, const double *P, double *Q,
+                          const float *P32, float *Q32, const int *skip)
+{
+    const int grid = xcd_grid((E->ngroups + 255) / 256);
+    const int *key = E->col16 ? E->key.p : nullptr;
+    if (P32)
+        k_node_rows<CT, ND, U32><<<grid, 256, 0, ctx->stream>>>(E->ngroups, E->NEQ, E->bptr.p, E->blen.p, E->eq.p, key, bcol,
+                                                               E->val32.p, P32, Q32, skip);
+    else
+        k_ebe_gather<double, CT, ND, U><<<grid, 256, 0, ctx->stream>>>(E->ngroups, E->NEQ, E->iptr.p, E->len.p, E->eq.p, key,
+                                                                       col, E->val.p, P, Q, skip);
+}
+
+// Q = A P in FP64 (P32 null) or FP32.
+static int ebe_product(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, double *Q, const float *P32, float *Q32,
+                       const int *skip)
 {
     FG_CHECK(E->has_values, FEMGPU_ERR_STATE, "femgpu_ebemv: element matrices not set");
     if (E->zero_q && E->NEQ > 0) {
-        k_ebe_zero<T><<<std::min(4096, (E->NEQ + 255) / 256), 256, 0, ctx->stream>>>(E->NEQ, Q, skip);
+        const int grid = std::min(4096, (E->NEQ + 255) / 256);
+        if (P32) k_ebe_zero<float><<<grid, 256, 0, ctx->stream>>>(E->NEQ, Q32, skip);
+        else k_ebe_zero<double><<<grid, 256, 0, ctx->stream>>>(E->NEQ, Q, skip);
         FG_HIP(hipGetLastError());
     }
     if (E->ngroups == 0) return FEMGPU_OK;
-    const bool c16 = E->col16 != 0;
+    const short *c16 = E->col16v.p, *b16 = E->bcol16.p;
+    const int *c32 = E->col32v.p, *b32 = E->bcol32.p;
     switch (E->ndof) {
     case 1:
-        if (c16) gather_launch<T, short, 1, 6>(ctx, E, vals, P, Q, skip);
-        else gather_launch<T, int, 1, 6>(ctx, E, vals, P, Q, skip);
+        if (E->col16) gather_launch<short, 1, 6, 7>(ctx, E, c16, b16, P, Q, P32, Q32, skip);
+        else gather_launch<int, 1, 6, 7>(ctx, E, c32, b32, P, Q, P32, Q32, skip);
         break;
     case 3:
-        if (c16) gather_launch<T, short, 3, 1>(ctx, E, vals, P, Q, skip);
-        else gather_launch<T, int, 3, 1>(ctx, E, vals, P, Q, skip);
+        if (E->col16) gather_launch<short, 3, 1, 4>(ctx, E, c16, b16, P, Q, P32, Q32, skip);
+        else gather_launch<int, 3, 1, 4>(ctx, E, c32, b32, P, Q, P32, Q32, skip);
         break;
     default:
-        if (c16) gather_launch<T, short, 4, 1>(ctx, E, vals, P, Q, skip);
-        else gather_launch<T, int, 4, 1>(ctx, E, vals, P, Q, skip);
+        if (E->col16) gather_launch<short, 4, 1, 4>(ctx, E, c16, b16, P, Q, P32, Q32, skip);
+        else gather_launch<int, 4, 1, 4>(ctx, E, c32, b32, P, Q, P32, Q32, skip);
         break;
     }
     FG_HIP(hipGetLastError());
@@ -161,12 +337,30 @@ static int ebe_product(femgpu_ctx *ctx, const femgpu_ebe *E, const T *vals, cons
 
 int launch_ebemv(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, double *Q, const int *skip)
 {
-    return ebe_product<double>(ctx, E, E->val.p, P, Q, skip);
+    return ebe_product(ctx, E, P, Q, nullptr, nullptr, skip);
 }
 
 int launch_ebemv32(femgpu_ctx *ctx, const femgpu_ebe *E, const float *P, float *Q, const int *skip)
 {
-    return ebe_product<float>(ctx, E, E->val32.p, P, Q, skip);
+    return ebe_product(ctx, E, nullptr, nullptr, P, Q, skip);
+}
+
+template <int ND>
+static int fill_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const double *Ae)
+{
+    constexpr int S = 3 * ND, RB = ND == 1 ? 6 : 2;
+    const int grid = E->nslices * ND;
+    const size_t turn = sizeof(double) * RB * 64 * (S + 1);
+    if (!E->wide_slots) {
+        k_ebe_fill<ND, RB, true><<<grid, 64, turn + sizeof(double) * 64 * ND * E->maxblk, ctx->stream>>>(
+            E->iptr.p, E->bptr.p, E->src.p, E->slots.p, Ae, E->val.p, E->val32.p);
+    } else {
+        k_ebe_fill<ND, RB, false><<<grid, 64, turn, ctx->stream>>>(E->iptr.p, nullptr, E->src.p, nullptr, Ae, E->val.p, nullptr);
+        FG_HIP(hipGetLastError());
+        k_node_rows_fill<ND><<<grid, 256, 0, ctx->stream>>>(E->iptr.p, E->bptr.p, E->src.p, E->slots.p, E->val.p, E->val32.p);
+    }
+    FG_HIP(hipGetLastError());
+    return FEMGPU_OK;
 }
 
 }  // namespace fg
@@ -242,9 +436,18 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     const size_t nslots = static_cast<size_t>(nrows) * 64;
     FG_CHECK(nslots * s * nd < (size_t{1} << 40) && nslots < static_cast<size_t>(INT_MAX), FEMGPU_ERR_ARG,
              "femgpu_ebe_create: operator too large");
-    std::vector<int> src(nslots, -1), c32(nslots * s, NEQ);
-    std::vector<short> c16(nslots * s, kSink16);
+    // columns as 16-bit offsets from the node's first unknown where every one fits
     bool fits16 = true;
+    for (size_t ea = 0; ea < kinc.size() && fits16; ++ea) {
+        if (kinc[ea] < 0) continue;
+        const int *L = lm + ea / 3 * s;
+        for (int b = 0; b < s; ++b) {
+            const long dlt = static_cast<long>(L[b]) - kinc[ea];
+            fits16 = fits16 && (L[b] >= NEQ || (dlt >= -32767 && dlt <= 32767));
+        }
+    }
+    std::vector<int> src(nslots, -1), c32(fits16 ? 0 : nslots * s, NEQ);
+    std::vector<short> c16(fits16 ? nslots * s : 0, kSink16);
     for (int g = 0; g < ng; ++g) {
         const int sl = g >> 6, l = g & 63;
         for (int j = 0; j < len[g]; ++j) {
@@ -253,17 +456,87 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
             src[r * 64 + l] = e * s * s + nd * a * s;
             for (int b = 0; b < s; ++b) {
                 const int c = lm[static_cast<size_t>(e) * s + b];
-                c32[(r * s + b) * 64 + l] = c;
-                if (c < NEQ) {
-                    const long dlt = static_cast<long>(c) - gkey[g];
-                    if (dlt < -32767 || dlt > 32767) fits16 = false;
-                    else c16[(r * s + b) * 64 + l] = static_cast<short>(dlt);
+                if (c >= NEQ) continue;
+                if (fits16) c16[(r * s + b) * 64 + l] = static_cast<short>(c - gkey[g]);
+                else c32[(r * s + b) * 64 + l] = c;
+            }
+        }
+    }
+    // node block rows of the FP32 product: per group its column nodes (groups) in order of appearance, and
+    // the position of each incidence's three column nodes among them (three 8-bit positions per incidence,
+    // or one word each where a node has too many column nodes)
+    std::vector<int> bptr(static_cast<size_t>(nslices) + 1, 0), blen(ng, 0), cols(static_cast<size_t>(64) * 3 * maxinc);
+    std::vector<int> b32;
+    std::vector<short> b16;
+    const size_t guess = (static_cast<size_t>(nrows) + 2 * nslices) * 64 * nd;
+    if (fits16) b16.reserve(guess);
+    else b32.reserve(guess);
+    int maxblk = 0;
+    const bool packed = maxinc < kFillBlocks;   // n triangles around a node have n + 1 column nodes
+    bool wide = !packed;
+    std::vector<unsigned> slots(packed ? nslots : 3 * nslots, ~0u);
+    for (int sl = 0; sl < nslices; ++sl) {
+        int w = 0;
+        const int g1 = std::min(ng, 64 * sl + 64);
+        for (int g = 64 * sl; g < g1; ++g) {
+            const int l = g & 63;
+            int *cs = cols.data() + static_cast<size_t>(l) * 3 * maxinc, nc = 0;
+            for (int j = 0; j < len[g]; ++j) {
+                const int ea = inc[gptr[g] + j], e3 = ea - ea % 3;
+                const size_t q = static_cast<size_t>(iptr[sl] + j) * 64 + l;
+                unsigned code = ~0u;
+                for (int a = 0; a < 3; ++a) {
+                    const int k = kinc[e3 + a];
+                    if (k < 0) continue;
+                    int at = 0;
+                    while (at < nc && cs[at] != k) ++at;
+                    if (at == nc) cs[nc++] = k;
+                    if (packed) code = (code & ~(255u << (8 * a))) | (static_cast<unsigned>(at) << (8 * a));
+                    else slots[3 * q + a] = static_cast<unsigned>(at);
+                }
+                if (packed) slots[q] = code;
+            }
+            blen[g] = nc;
+            w = std::max(w, nc);
+        }
+        bptr[sl + 1] = bptr[sl] + w;
+        maxblk = std::max(maxblk, w);
+        const size_t first = static_cast<size_t>(bptr[sl]) * 64 * nd, end = static_cast<size_t>(bptr[sl + 1]) * 64 * nd;
+        if (fits16) b16.resize(end, kSink16);
+        else b32.resize(end, NEQ);
+        for (int g = 64 * sl; g < g1; ++g) {
+            const int l = g & 63, *cs = cols.data() + static_cast<size_t>(l) * 3 * maxinc;
+            for (int j = 0; j < blen[g]; ++j) {
+                const int cg = gid[cs[j]];
+                const int *ce = eq.data() + static_cast<size_t>(cg >> 6) * nd * 64 + (cg & 63);
+                for (int d = 0; d < nd; ++d) {
+                    const int c = ce[d * 64];
+                    if (c >= NEQ) continue;
+                    const size_t at = first + (static_cast<size_t>(j) * 64 + l) * nd + d;
+                    if (fits16) b16[at] = static_cast<short>(c - gkey[g]);
+                    else b32[at] = c;
                 }
             }
         }
     }
+    const size_t nbslots = static_cast<size_t>(bptr[nslices]) * 64;
+    FG_CHECK(nbslots < static_cast<size_t>(INT_MAX) / 16, FEMGPU_ERR_ARG, "femgpu_ebe_create: operator too large");
+    if (packed && maxblk > kFillBlocks) {   // nodes whose triangles do not share edges: unpack the positions
+        std::vector<unsigned> s3(3 * nslots, ~0u);
+        for (size_t q = 0; q < nslots; ++q)
+            for (int a = 0; a < 3; ++a) {
+                const unsigned at = (slots[q] >> (8 * a)) & 255u;
+                if (at != 255u) s3[3 * q + a] = at;
+            }
+        slots.swap(s3);
+        wide = true;
+    }
     auto *E = new femgpu_ebe();
     E->ctx = ctx;
+    E->nslices = nslices;
+    E->nbrows = bptr[nslices];
+    E->wide_slots = wide;
+    E->maxblk = maxblk;
     E->nel = nel;
     E->s = s;
     E->ndof = nd;
@@ -283,7 +556,12 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     if (!rc && fits16) rc = E->col16v.upload(c16.data(), c16.size(), st);
     if (!rc && !fits16) rc = E->col32v.upload(c32.data(), c32.size(), st);
     if (!rc) rc = E->val.alloc(nslots * s * nd);
-    if (!rc) rc = E->val32.alloc(nslots * s * nd);
+    if (!rc) rc = E->bptr.upload(bptr.data(), bptr.size(), st);
+    if (!rc) rc = E->blen.upload(blen.data(), blen.size(), st);
+    if (!rc && fits16) rc = E->bcol16.upload(b16.data(), b16.size(), st);
+    if (!rc && !fits16) rc = E->bcol32.upload(b32.data(), b32.size(), st);
+    if (!rc) rc = E->slots.upload(slots.data(), slots.size(), st);
+    if (!rc) rc = E->val32.alloc(nbslots * nd * nd);
     if (!rc && hipStreamSynchronize(st) != hipSuccess) rc = FEMGPU_ERR_HIP;   // host arrays end here
     if (rc) {
         delete E;
@@ -310,16 +588,11 @@ extern "C" int femgpu_ebe_set_values(femgpu_ebe *E, const double *A, int on_devi
         FG_TRY(tmp.upload(A, total, ctx->stream));
         dA = tmp.p;
     }
-    const int nslots = E->nrows * 64;
-    if (nslots > 0) {
-        const int grid = (nslots + 255) / 256;
-        switch (E->ndof) {
-        case 1: k_ebe_fill<1><<<grid, 256, 0, ctx->stream>>>(nslots, E->src.p, dA, E->val.p, E->val32.p); break;
-        case 3: k_ebe_fill<3><<<grid, 256, 0, ctx->stream>>>(nslots, E->src.p, dA, E->val.p, E->val32.p); break;
-        default: k_ebe_fill<4><<<grid, 256, 0, ctx->stream>>>(nslots, E->src.p, dA, E->val.p, E->val32.p); break;
+    if (E->nrows > 0) switch (E->ndof) {
+        case 1: FG_TRY(fill_launch<1>(ctx, E, dA)); break;
+        case 3: FG_TRY(fill_launch<3>(ctx, E, dA)); break;
+        default: FG_TRY(fill_launch<4>(ctx, E, dA)); break;
         }
-        FG_HIP(hipGetLastError());
-    }
     if (!on_device) FG_HIP(hipStreamSynchronize(ctx->stream));
     E->has_values = true;
     return FEMGPU_OK;
@@ -337,7 +610,7 @@ extern "C" int femgpu_ebe_get_info(femgpu_ebe *E, femgpu_ebe_info *info)
     info->column_bytes = E->col16 ? 2 : 4;
     info->pad = 0;
     info->bytes_f64 = slots * nd * s * 8 + cols + meta + 16LL * E->NEQ;
-    info->bytes_f32 = slots * nd * s * 4 + cols + meta + 8LL * E->NEQ;
+    info->bytes_f32 = static_cast<long long>(E->nbrows) * 64 * nd * (4 * nd + (E->col16 ? 2 : 4)) + meta + 8LL * E->NEQ;
     return FEMGPU_OK;
 }
 
