@@ -112,6 +112,7 @@ constexpr int kStreamLongMax = 4096;    // long-lived slots at most
 struct StreamSweep {
     bool ok = false;
     int n = 0, nsteps = 0, steps = 0, K = 0, W = 0, L = 0, depth = 0;   // nsteps: padded, steps: real
+    int threads = kStreamThreads;   // workgroup size: the widest step, in whole wavefronts
     DevBuf<int> stepq;              // step -> first schedule position (nsteps + 2*kStreamPad + 1, tail = n)
     DevBuf<int> row_of;             // schedule position -> row (n)
     DevBuf<unsigned short> slot;    // n*K LDS slots of the dependencies

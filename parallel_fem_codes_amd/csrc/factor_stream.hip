@@ -213,9 +213,8 @@ struct FixedStage {
     int q;
 };
 
-__device__ __forceinline__ void fixed_fetch(FixedStage &g, const FactorArgs &A, const int *sq, int s)
+__device__ __forceinline__ void fixed_fetch(FixedStage &g, const FactorArgs &A, int q)
 {
-    const int q = factor_pos(sq, s);
     g.q = q;
     const unsigned qq = q < 0 ? 0u : static_cast<unsigned>(q);
 #pragma unroll
@@ -259,6 +258,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_factor_fixed(FactorArgs A)
         for (int u = 0; u < D; ++u) {
             __builtin_amdgcn_sched_barrier(0);
             FixedStage &g = st[u];
+            const int qn = factor_pos(sq, s0 + u + D);   // with the ring reads, as in the sweeps
             const bool on = g.q >= 0;
             // a wave past the step's rows (its lane 0 idle) computes, writes and stores nothing;
             // idle lanes of a wave with rows write to slot W + 1 and store past the n positions
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_factor_fixed(FactorArgs A)
                 at32(reinterpret_cast<double2 *>(A.out + 2 * static_cast<size_t>(A.ostride)), qo) =
                     make_double2(out[5], out[6]);
             }
-            fixed_fetch(g, A, sq, s0 + u + D);
+            fixed_fetch(g, A, qn);
             lds_barrier();
         }
     }
@@ -446,13 +446,13 @@ int launch_stream_factor(femgpu_ctx *ctx, femgpu_csr *A)
     a.err = ctx->err.p;
     if (F.compact) {
         if (F.structured)
-            k_factor_fixed<4, kStructAlways, kStructNever><<<1, kStreamThreads, factor_lds_bytes(P), ctx->stream>>>(a);
+            k_factor_fixed<4, kStructAlways, kStructNever><<<1, P.threads, factor_lds_bytes(P), ctx->stream>>>(a);
         else
-            k_factor_fixed<4, 0u, 0u><<<1, kStreamThreads, factor_lds_bytes(P), ctx->stream>>>(a);
+            k_factor_fixed<4, 0u, 0u><<<1, P.threads, factor_lds_bytes(P), ctx->stream>>>(a);
         k_factor_finish<<<grid, 256, 0, ctx->stream>>>(n, n + kStreamThreads, F.meta.p, F.rec.p, A->AA.p, F.out.p,
                                                        A->LU.p, A->Dinv.p);
     } else {
-        k_factor_stream<4><<<1, kStreamThreads, factor_lds_bytes(P), ctx->stream>>>(a);
+        k_factor_stream<4><<<1, P.threads, factor_lds_bytes(P), ctx->stream>>>(a);
         k_factor_scatter<<<grid, 256, 0, ctx->stream>>>(n, n + kStreamThreads, F.meta.p, F.out.p, F.dinv.p, A->LU.p,
                                                         A->Dinv.p);
     }

@@ -705,6 +705,9 @@ int build_stream_plan(femgpu_ctx *ctx, int n, const int *IA, const int *JA, cons
     P.L = L;
     P.nsteps = nsteps;
     P.steps = nsteps_real;
+    int widest = 1;
+    for (int q = 0; q < n; ++q) widest = std::max(widest, step_end[q] - step_beg[q]);
+    P.threads = (widest + 63) / 64 * 64;
     const size_t limit = ctx->lds_limit > 1024 ? ctx->lds_limit - 1024 : ctx->lds_limit;
     if (stream_lds_bytes(P, sizeof(double)) > limit) return FEMGPU_OK;
     // padded row data in schedule order, entries in the serial sweep's order

@@ -311,12 +311,11 @@ __device__ __forceinline__ int stream_pos(const int *sq, int s)
     return q < sq[s + 1] ? q : -1;
 }
 
-// Stage step s into g: entries, slots, pivot and right-hand side by schedule position.
+// Stage schedule position q (-1: idle) into g: entries, slots, pivot and right-hand side.
 template <typename T, bool UPPER, int K, bool LONG>
-__device__ __forceinline__ void stream_fetch(StreamStage<T, K> &g, const StreamArgs &a, const int *sq, int s,
+__device__ __forceinline__ void stream_fetch(StreamStage<T, K> &g, const StreamArgs &a, int q,
                                              const T *__restrict__ val, const T *__restrict__ dinv, const T *b)
 {
-    const int q = stream_pos(sq, s);
     const int qq = q < 0 ? 0 : q;
     load_bytes<K * sizeof(T)>(val + static_cast<size_t>(qq) * K, g.v);
     load_bytes<K * 2>(a.slot + static_cast<size_t>(qq) * K, g.s);
@@ -329,8 +328,8 @@ __device__ __forceinline__ void stream_fetch(StreamStage<T, K> &g, const StreamA
 // UPPER: x = (b - U x) * Dinv; else x = b - L x (ILUp_precond.c:26-44, same operation order,
 // contraction off; padding entries subtract 0 * 0). b and x are in schedule order; b may alias x:
 // a row's b is read D steps before its own result is stored, and no other row reads it.
-template <typename T, bool UPPER, int K, int D, bool LONG>
-__global__ __launch_bounds__(kStreamThreads) void k_sweep_stream(StreamArgs a, const T *__restrict__ val,
+template <typename T, bool UPPER, int K, int D, bool LONG, int MAXT>
+__global__ __launch_bounds__(MAXT) void k_sweep_stream(StreamArgs a, const T *__restrict__ val,
                                                                  const T *__restrict__ dinv, const T *b, T *x,
                                                                  const int *__restrict__ skip)
 {
@@ -361,6 +360,10 @@ __global__ __launch_bounds__(kStreamThreads) void k_sweep_stream(StreamArgs a, c
         st[u].q = -1;
         st[u].ks = static_cast<unsigned short>(a.W + 1);
     }
+    // A step's loads go into the stage the last step has freed, D - 1 steps ahead, in the shadow of the ring
+    // reads; with two stages that would leave one step of lookahead, so they follow the step's own work there.
+    constexpr bool EARLY = D > 2;
+    int qn = stream_pos(sq, EARLY ? D - 1 : D);
     for (int s0 = 0; s0 < a.nsteps; s0 += D) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
@@ -368,16 +371,25 @@ __global__ __launch_bounds__(kStreamThreads) void k_sweep_stream(StreamArgs a, c
             // would make this step wait for that step's loads
             __builtin_amdgcn_sched_barrier(0);
             StreamStage<T, K> &g = st[u];
+            T r[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) r[k] = ring[g.s[k]];
+            const int qnn = stream_pos(sq, s0 + u + (EARLY ? D : D + 1));   // the next step's table entry
+            if constexpr (EARLY) {
+                stream_fetch<T, UPPER, K, LONG>(st[(u + D - 1) % D], a, qn, val, dinv, b);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             T acc = g.b;
 #pragma unroll
-            for (int k = 0; k < K; ++k) acc -= g.v[k] * ring[g.s[k]];
+            for (int k = 0; k < K; ++k) acc -= g.v[k] * r[k];
             if (UPPER) acc *= g.d;
             const bool on = g.q >= 0;
             ring[on ? (g.q & wmask) : a.W + 1] = acc;
             if (LONG) ring[g.ks] = acc;   // read again beyond the ring's reach (else the idle slot)
             // a wave past the step's rows (its lane 0 idle) stores nothing
             if (__builtin_amdgcn_readfirstlane(on ? 1 : 0)) *(on ? x + g.q : sink) = acc;
-            stream_fetch<T, UPPER, K, LONG>(g, a, sq, s0 + u + D, val, dinv, b);
+            if constexpr (!EARLY) stream_fetch<T, UPPER, K, LONG>(g, a, qn, val, dinv, b);
+            qn = qnn;
             lds_barrier();
         }
     }
@@ -422,29 +434,31 @@ static StreamArgs stream_args(const StreamSweep &P)
     return a;
 }
 
-template <typename T>
-constexpr int kD16 = sizeof(T) == 4 ? 4 : 2;
+// The workgroup is as wide as the widest step, in whole wavefronts: a wavefront that never has rows would
+// only take issue slots from the others. Lookahead: the most steps that fit the registers of MAXT threads.
+template <typename T, bool UPPER, int K, int D, int MAXT>
+static void stream_launch_k(femgpu_ctx *ctx, const StreamSweep &P, const T *val, const T *dinv, const T *b, T *x,
+                            const int *skip)
+{
+    const size_t lds = stream_lds_bytes(P, sizeof(T));
+    const StreamArgs a = stream_args(P);
+    if (P.L == 0)
+        k_sweep_stream<T, UPPER, K, D, false, MAXT><<<1, P.threads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
+    else
+        k_sweep_stream<T, UPPER, K, D, true, MAXT><<<1, P.threads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
+}
 
 template <typename T, bool UPPER>
 static int stream_launch(femgpu_ctx *ctx, const StreamSweep &P, const T *val, const T *dinv, const T *b, T *x,
                          const int *skip)
 {
-    const size_t lds = stream_lds_bytes(P, sizeof(T));
-    const StreamArgs a = stream_args(P);
-    if (P.K == 4 && P.L == 0)
-        k_sweep_stream<T, UPPER, 4, 8, false><<<1, kStreamThreads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
-    else if (P.K == 4)
-        k_sweep_stream<T, UPPER, 4, 8, true><<<1, kStreamThreads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
-    else if (P.K == 8 && P.L == 0)
-        k_sweep_stream<T, UPPER, 8, 4, false><<<1, kStreamThreads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
-    else if (P.K == 8)
-        k_sweep_stream<T, UPPER, 8, 4, true><<<1, kStreamThreads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
+    constexpr int F = sizeof(T) == 4 ? 2 : 1;
+    if (P.K == 4) stream_launch_k<T, UPPER, 4, 8, kStreamThreads>(ctx, P, val, dinv, b, x, skip);
+    else if (P.K == 8) stream_launch_k<T, UPPER, 8, 4, kStreamThreads>(ctx, P, val, dinv, b, x, skip);
     // 16-entry rows: 4 steps of lookahead fit the registers in FP32 (6.6 against 7.4 ms per apply on
     // the 513 x 513 cavity), 2 in FP64
-    else if (P.L == 0)
-        k_sweep_stream<T, UPPER, 16, kD16<T>, false><<<1, kStreamThreads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
-    else
-        k_sweep_stream<T, UPPER, 16, kD16<T>, true><<<1, kStreamThreads, lds, ctx->stream>>>(a, val, dinv, b, x, skip);
+    else if (P.threads > 256) stream_launch_k<T, UPPER, 16, 2 * F, kStreamThreads>(ctx, P, val, dinv, b, x, skip);
+    else stream_launch_k<T, UPPER, 16, 4 * F, 256>(ctx, P, val, dinv, b, x, skip);
     FG_HIP(hipGetLastError());
     return FEMGPU_OK;
 }
