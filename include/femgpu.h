@@ -325,7 +325,9 @@ typedef struct {
  * on the current element matrices; the inner solver uses the FP32 element matrices and FP32 inverse
  * blocks, sweep_mode / factor_sweeps ignored, graphs must be 0). X = 0 is returned where it already
  * passes (||F|| = 0 or tol >= 1: status 0), with max_refinements = 0 (status 1 unless ||F|| = 0)
- * and for a non-finite F (status 1). No reference counterpart. */
+ * and for a non-finite F (status 1). CSR systems of at most 4096 rows with factor_sweeps >= 1,
+ * sweep_mode >= 1 and modified Gram-Schmidt run as one workgroup's launch (femgpu_gmres_mixed_wg's
+ * kernel, graphs or not). No reference counterpart. */
 int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *sys, const femgpu_mixed_opts *opt,
                        double tol, const double *d_F, double *d_X, femgpu_solve_info *info);
 
@@ -345,7 +347,10 @@ typedef struct {
  * the inner right-hand side zeroed, so every Krylov vector is exactly zero there) as soon as
  * ||F_s - A_s x_s|| <= tol ||F_s||; active systems enter each inner FP32 GMRES cycle with their
  * residual scaled to unit norm, and the cycle's correction is scaled back per system. One launch
- * sequence serves the whole batch. info: nsys entries. No reference counterpart. */
+ * sequence serves the whole batch. Batches of systems of at most 3072 rows (no more systems than the
+ * GPU has compute units, factor_sweeps >= 1, sweep_mode >= 1) take femgpu_gmres_mixed_wg's kernel: a
+ * workgroup and a Krylov space (modified Gram-Schmidt) per system. info: nsys entries. No reference
+ * counterpart. */
 int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *sys, int nsys, const int *row_off,
                                const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
                                femgpu_batch_info *info);

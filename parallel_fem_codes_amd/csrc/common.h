@@ -425,6 +425,11 @@ void csr_map(int nkeys, const std::vector<std::pair<int, int>> &pairs, std::vect
              std::vector<int> &dst);
 int check_device_error(femgpu_ctx *ctx);
 int wg_threads_for(long long rows, int nsys);   // persistent batched solver: default workgroup size
+bool wg_preferred(const femgpu_ctx *ctx, const femgpu_system *S, const femgpu_mixed_opts *opt, int nsys, int widest);
+int wg_solve_one(femgpu_ctx *ctx, femgpu_csr *A, const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
+                 femgpu_batch_info *info);
+int wg_solve_batch(femgpu_ctx *ctx, femgpu_csr *A, int nsys, const int *row_off, const femgpu_mixed_opts *opt, double tol,
+                   int threads, const double *d_F, double *d_X, femgpu_batch_info *info);
 int csr_autotune(femgpu_csr *A, femgpu_tune_info *info);
 void release_step_graphs(femgpu_ctx *ctx);
 

@@ -1028,6 +1028,23 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
         FG_CHECK(opt->graphs == 0, FEMGPU_ERR_ARG, "femgpu_gmres_mixed: graph replay needs a CSR operator");
     }
     const int kin = opt->inner_kmax;
+    // small systems: the whole solve as one workgroup's launch (modified Gram-Schmidt only; graphs or not, so
+    // that replayed and eager solves stay the same)
+    if (csr && opt->orthogonalization != 1 && tol < 1.0 && wg_preferred(ctx, S, opt, 1, n)) {
+        femgpu_batch_info bi;
+        FG_TRY(wg_solve_one(ctx, S->csr, opt, tol, d_F, d_X, &bi));
+        if (info) {
+            memset(info, 0, sizeof(*info));
+            const bool finite = std::isfinite(bi.normF);
+            info->iterations = info->inner_iterations = bi.inner_iterations;
+            info->cycles = bi.refinements;
+            info->normb = bi.normF;
+            info->true_rel_residual = bi.normF == 0.0 ? 0.0 : finite ? bi.true_rel_residual : bi.normF;
+            info->rho = finite ? bi.true_rel_residual * bi.normF : bi.normF;
+            info->status = finite && bi.status == 0 ? 0 : 1;
+        }
+        return FEMGPU_OK;
+    }
     GDev G{};
     FG_TRY(make_gdev(ctx, kin, G));
     G.prec_mode = opt->sweep_mode;
@@ -1179,6 +1196,11 @@ extern "C" int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *
     FG_CHECK(opt->factor_sweeps > 0 || S->ilu->factored, FEMGPU_ERR_STATE,
              "femgpu_gmres_mixed_batched: ILU(0) not factored");
     const int kin = opt->inner_kmax;
+    // small systems: a workgroup each (its own Krylov space), modified Gram-Schmidt
+    int widest = 0;
+    for (int s = 0; s < nsys; ++s) widest = std::max(widest, row_off[s + 1] - row_off[s]);
+    if (wg_preferred(ctx, S, opt, nsys, widest))
+        return wg_solve_batch(ctx, S->csr, nsys, row_off, opt, tol, wg_threads_for(widest, 1), d_F, d_X, info);
     memset(info, 0, sizeof(*info) * static_cast<size_t>(nsys));
     GDev G{};
     FG_TRY(make_gdev(ctx, kin, G));

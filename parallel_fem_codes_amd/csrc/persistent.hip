@@ -10,6 +10,7 @@
 // outer steps, m - 1 inner steps, the Jacobi iteration count), and every exit decision is taken
 // from values that all threads of the workgroup hold identically, so every wave reaches the end.
 #include <algorithm>
+#include <cstring>
 
 #include "common.h"
 #include "device_util.h"
@@ -20,7 +21,8 @@ namespace {
 constexpr int kWgMaxBasis = 64;   // inner basis size limit: the Hessenberg matrix lives in LDS
 
 struct WgArgs {
-    const int *row_off;
+    const int *row_off;          // null: one system of n rows
+    int n;
     const int *IA, *JA;          // FP64 CSR (outer residual)
     const double *AA;
     const int *sptr, *scol;      // sliced ELL of A (FP32 SpMV) and of the factors
@@ -35,6 +37,18 @@ struct WgArgs {
     double tol, inner_tol;
     femgpu_batch_info *info;
 };
+
+__device__ __forceinline__ void wg_report(const WgArgs &a, int sys, int refinements, int inner, double rn, double normF)
+{
+    femgpu_batch_info inf;
+    inf.refinements = refinements;
+    inf.inner_iterations = inner;
+    inf.status = (rn <= a.tol * normF) ? 0 : 1;
+    inf.pad = 0;
+    inf.normF = normF;
+    inf.true_rel_residual = normF > 0.0 ? rn / normF : 0.0;
+    a.info[sys] = inf;
+}
 
 // Sum over the workgroup, the same value (same order) in every thread. Two barriers: red may be
 // reused by the next call at once.
@@ -110,15 +124,354 @@ __device__ void wg_jacobi(const WgArgs &a, int r0, int r1, float *T0, float *T1,
     }
 }
 
-template <int BS, int QW>
-__global__ __launch_bounds__(BS) void k_gmres_wg(WgArgs a)
+// ---- systems of at most R rows per thread: the vectors a row gathers from are in LDS, its own values in
+// registers. Row r0 + tid + k*BS belongs to thread tid; a Jacobi or product phase gathers from one of two
+// LDS vectors and writes the other, one barrier each. Where they fit, the rows' matrix entries, factors
+// and columns stay in registers for the whole solve (KEEP), so a phase touches no memory; else they are read
+// again (from L2) in every phase. What bounds a step is then its chain of barriers and reductions.
+// Against the path that keeps the vectors in global memory, transient systems of 361 / 1 472 / 3 481 rows:
+// 84 / 181 / 337 us a solve, 139 / 429 / 734 us before (10, 14 and 12 Arnoldi steps).
+
+__device__ __forceinline__ double lane_value(double v, int lane)   // lane: uniform
 {
-    extern __shared__ double sm[];
-    __shared__ int s_done;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane(static_cast<int>(b), lane), hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), lane);
+    return __longlong_as_double(static_cast<long long>(static_cast<unsigned>(lo)) | (static_cast<long long>(hi) << 32));
+}
+
+// Sum over the workgroup in every thread (as wg_sum) with one barrier: successive calls alternate between
+// the two halves of red, and the barrier of a call separates the reads of the call before it from the
+// writes of the call after it.
+template <int BS>
+__device__ __forceinline__ double wg_sum1(double v, double *red, int &half)
+{
+    constexpr int NW = BS / 64;
+    v = wave_sum(v);
+    double *rd = red + half * NW;
+    half ^= 1;
+    if ((threadIdx.x & 63) == 0) rd[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) t += rd[k];
+    return t;
+}
+
+template <int R, int QW, bool KEEP>
+struct WgRows {
+    int p[R], inf[R];              // sliced-ELL position of the row's first entry; strict-lower count | length << 8
+    float dinv[R];
+    float av[KEEP ? R : 1][QW], lv[KEEP ? R : 1][QW];
+    unsigned cc[KEEP ? R : 1][QW / 2];   // columns within the system, two per word
+};
+
+// dot[k] = sum over entries q0[k] <= q < q1[k] of the thread's row k of val * x[col], in order (LU: the
+// factors, else A).
+template <int BS, bool LU, int R, int QW, bool KEEP>
+__device__ __forceinline__ void wg_dots(const WgArgs &a, const WgRows<R, QW, KEEP> &w, const int (&q0)[R], const int (&q1)[R],
+                                        int r0, int n, const float *x, float (&dot)[R])
+{
+#pragma unroll
+    for (int k = 0; k < R; ++k) dot[k] = 0.0f;
+    if constexpr (KEEP) {
+        (void)r0, (void)n;
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int q = 0; q < QW; ++q) {
+                const unsigned c = w.cc[k][q / 2];
+                const float z = (LU ? w.lv[k][q] : w.av[k][q]) * x[q & 1 ? c >> 16 : c & 0xffffu];
+                dot[k] = q >= q0[k] && q < q1[k] ? dot[k] + z : dot[k];
+            }
+    } else {
+        const float *vals = LU ? a.LU : a.sval;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            if (static_cast<int>(threadIdx.x) + k * BS >= n) continue;
+            for (int q = q0[k]; q < q1[k]; q += 4) {   // four entries' loads in flight
+                float v[4];
+                int c[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = w.p[k] + ((q + u < q1[k] ? q + u : q) << 6);
+                    v[u] = vals[e];
+                    c[u] = a.scol[e] - r0;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float z = v[u] * x[c[u]];
+                    dot[k] = q + u < q1[k] ? dot[k] + z : dot[k];
+                }
+            }
+        }
+    }
+}
+
+// out = (U~ L~)^-1 b by jac Jacobi iterations per triangle, as wg_jacobi: b in registers and in S0. The last
+// lower iteration leaves Dinv y, the upper iteration's start, in LDS. Both vectors are free on return.
+template <int BS, int R, int QW, bool KEEP>
+__device__ __forceinline__ void wg_jacobi_lds(const WgArgs &a, const WgRows<R, QW, KEEP> &w, int r0, int n, const float (&b)[R],
+                                              float *S0, float *S1, float (&out)[R])
+{
+    float y[R], d[R];
+    int z[R], nl[R], nu[R], len[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        z[k] = 0;
+        nl[k] = w.inf[k] & 0xff;
+        nu[k] = nl[k] + 1;
+        len[k] = w.inf[k] >> 8;
+    }
+    for (int it = 1; it <= a.jac; ++it) {
+        wg_dots<BS, true>(a, w, z, nl, r0, n, S0, d);
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int i = static_cast<int>(threadIdx.x) + k * BS;
+            y[k] = b[k] - d[k];
+            if (i < n) S1[i] = it == a.jac ? w.dinv[k] * y[k] : y[k];
+        }
+        __syncthreads();
+        float *t = S0;
+        S0 = S1;
+        S1 = t;
+    }
+    for (int it = 1; it <= a.jac; ++it) {
+        wg_dots<BS, true>(a, w, nu, len, r0, n, S0, d);
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int i = static_cast<int>(threadIdx.x) + k * BS;
+            out[k] = i < n ? w.dinv[k] * (y[k] - d[k]) : 0.0f;
+            if (it < a.jac && i < n) S1[i] = out[k];
+        }
+        __syncthreads();
+        float *t = S0;
+        S0 = S1;
+        S1 = t;
+    }
+}
+
+// Givens update of column i by the first wavefront (pgmres.c:118-159): lane j holds rotation j and entry j
+// of the column; the running entry is carried along the rotations.
+__device__ __forceinline__ void wg_givens(int i, int ld, double hn, double eps, int last, double *H, double *cs, double *sn,
+                                          double *e, int *done)
+{
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63, jl = lane < i ? lane : 0;
+    const double c = cs[jl], s = sn[jl], h = H[(lane <= i ? lane : 0) * ld + i], ei = e[i];
+    double run = lane_value(h, 0), mine = 0.0;
+    for (int j = 0; j < i; ++j) {
+        const double cj = lane_value(c, j), sj = lane_value(s, j), hx = lane_value(h, j + 1);
+        const double h1 = cj * run + sj * hx, h2 = -sj * run + cj * hx;
+        mine = lane == j ? h1 : mine;
+        run = h2;
+    }
+    const double rr = sqrt(run * run + hn * hn), ci = run / rr, si = hn / rr, en = -si * ei;
+    if (lane < i) H[lane * ld + i] = mine;
+    if (lane == 0) {
+        cs[i] = ci;
+        sn[i] = si;
+        H[i * ld + i] = rr;
+        H[(i + 1) * ld + i] = 0.0;
+        e[i + 1] = en;
+        e[i] = ci * ei;
+        *done = !(fabs(en) > eps) || last;
+    }
+}
+
+// H y = e over steps columns by the first wavefront, a column at a time: lane j holds e_j.
+__device__ __forceinline__ void wg_back(int steps, int ld, const double *H, const double *e, double *y)
+{
+    const int lane = threadIdx.x & 63;
+    double r = lane < steps ? e[lane] : 0.0, mine = 0.0;
+    for (int k = steps - 1; k >= 0; --k) {
+        const double yk = lane_value(r, k) / H[k * ld + k];
+        const double hk = lane < k ? H[lane * ld + k] : 0.0;
+        mine = lane == k ? yk : mine;
+        r = r - hk * yk;
+    }
+    if (lane < steps) y[lane] = mine;
+}
+
+template <int BS, int QW, int R>
+__device__ __forceinline__ void wg_solve_lds(const WgArgs &a, double *sm, int *s_done)
+{
+    constexpr bool KEEP = R * QW <= (BS == 1024 ? 16 : 32);   // what 128 / 256 registers hold
+    using Rows = WgRows<R, QW, KEEP>;
+    const int ld = a.kin + 1, sys = blockIdx.x, tid = threadIdx.x;
+    double *H = sm, *cs = H + ld * ld, *sn = cs + ld, *e = sn + ld, *y = e + ld, *red = y + ld;
+    double *XS = red + 2 * (BS / 64);                       // the FP64 iterate, in the space of S0 and S1
+    float *S0 = reinterpret_cast<float *>(XS), *S1 = S0 + R * BS;
+    const int r0 = a.row_off ? a.row_off[sys] : 0, n = (a.row_off ? a.row_off[sys + 1] : a.n) - r0;
+    int half = 0;
+    Rows w;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = tid + k * BS, row = r0 + (i < n ? i : 0);   // rows past the system repeat its first, unused
+        w.p[k] = n > 0 ? a.sptr[row >> 6] + (row & 63) : 0;
+        w.inf[k] = n > 0 ? a.rinfo[row] : 0;
+        w.dinv[k] = n > 0 ? a.Dinv[row] : 0.0f;
+        if constexpr (KEEP) {
+            const int ln = w.inf[k] >> 8;
+#pragma unroll
+            for (int q = 0; q < QW; ++q) {
+                const int at = w.p[k] + ((q < ln ? q : 0) << 6);
+                w.av[k][q] = n > 0 ? a.sval[at] : 0.0f;
+                w.lv[k][q] = n > 0 ? a.LU[at] : 0.0f;
+                const unsigned c = n > 0 ? static_cast<unsigned>(a.scol[at] - r0) : 0u;
+                w.cc[k][q / 2] = q & 1 ? w.cc[k][q / 2] | (c << 16) : c;
+            }
+        }
+    }
+    int none[R], len[R];
+    double acc = 0.0, x[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        none[k] = 0;
+        len[k] = w.inf[k] >> 8;
+        const double f = tid + k * BS < n ? a.F[r0 + tid + k * BS] : 0.0;
+        acc += f * f;
+        x[k] = 0.0;
+    }
+    const double normF = sqrt(wg_sum1<BS>(acc, red, half));
+    int refinements = 0, inner = 0;
+    double rn = normF;
+    while (normF > 0.0) {
+        // outer FP64 residual r = F - A X (X = 0 on the first pass), entries in row order, X from LDS
+        double res[R];
+        acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int i = tid + k * BS;
+            res[k] = 0.0;
+            if (i < n) {
+                double v = a.F[r0 + i];
+                if (refinements > 0) {
+                    const int p0 = a.IA[r0 + i];
+                    double s = 0.0;
+                    for (int q = 0; q < len[k]; q += 4) {
+                        double t[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const int at = p0 + (q + u < len[k] ? q + u : q);
+                            t[u] = a.AA[at] * XS[a.JA[at] - r0];
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) s = q + u < len[k] ? s + t[u] : s;
+                    }
+                    v = v - s;
+                }
+                res[k] = v;
+                acc += v * v;
+            }
+        }
+        rn = sqrt(wg_sum1<BS>(acc, red, half));
+        if (!(rn <= 1.7976931348623157e308) || rn <= a.tol * normF || refinements >= a.max_ref) break;
+        ++refinements;
+        // inner FP32 solve of M^-1 A d = M^-1 r / ||r||, started from d = 0
+        const double inv_rn = 1.0 / rn;
+        float b[R], v[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int i = tid + k * BS;
+            b[k] = static_cast<float>(res[k] * inv_rn);
+            if (i < n) S0[i] = b[k];
+        }
+        __syncthreads();
+        wg_jacobi_lds<BS>(a, w, r0, n, b, S0, S1, v);
+        acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) acc += static_cast<double>(v[k]) * v[k];
+        const double e0 = sqrt(wg_sum1<BS>(acc, red, half));
+        if (!(e0 > 0.0)) break;   // preconditioned residual vanished in FP32: nothing left to correct
+        const double eps = a.inner_tol * e0;
+        double scale = 1.0 / e0;
+        if (tid == 0) e[0] = e0;
+        int steps = 0;
+        for (int i = 0; i < a.kin - 1; ++i) {
+            // v_i = w / h into LDS and the basis; b = A v_i; w = M^-1 b
+            const float inv = static_cast<float>(scale);
+            float *Vi = a.V + i * a.ldv + r0;
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const int r = tid + k * BS;
+                v[k] = v[k] * inv;
+                if (r < n) {
+                    S1[r] = v[k];
+                    Vi[r] = v[k];
+                }
+            }
+            __syncthreads();
+            wg_dots<BS, false>(a, w, none, len, r0, n, S1, b);
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                if (tid + k * BS < n) S0[tid + k * BS] = b[k];
+            __syncthreads();
+            float z[R];
+            wg_jacobi_lds<BS>(a, w, r0, n, b, S0, S1, z);
+            // MGS on the thread's own rows: h_j = <v_j, w>, then w -= h_j v_j; the next basis vector is
+            // loaded while the workgroup sums
+            float vj[R];
+#pragma unroll
+            for (int k = 0; k < R; ++k) vj[k] = tid + k * BS < n ? a.V[r0 + tid + k * BS] : 0.0f;
+            for (int j = 0; j <= i; ++j) {
+                acc = 0.0;
+                float vn[R];
+                const float *Vn = a.V + (j < i ? j + 1 : j) * a.ldv + r0;
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    acc += static_cast<double>(vj[k]) * static_cast<double>(z[k]);
+                    vn[k] = tid + k * BS < n ? Vn[tid + k * BS] : 0.0f;
+                }
+                const double h = wg_sum1<BS>(acc, red, half);
+                if (tid == 0) H[j * ld + i] = h;
+                const float hf = static_cast<float>(h);
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    z[k] = z[k] - hf * vj[k];
+                    vj[k] = vn[k];
+                }
+            }
+            acc = 0.0;
+#pragma unroll
+            for (int k = 0; k < R; ++k) acc += static_cast<double>(z[k]) * static_cast<double>(z[k]);
+            const double hn = sqrt(wg_sum1<BS>(acc, red, half));
+            if (tid < 64) wg_givens(i, ld, hn, eps, i + 1 >= a.kin - 1, H, cs, sn, e, s_done);
+            __syncthreads();
+            steps = i + 1;
+            if (*s_done) break;
+            scale = 1.0 / hn;
+#pragma unroll
+            for (int k = 0; k < R; ++k) v[k] = z[k];
+        }
+        inner += steps;
+        if (tid < 64) wg_back(steps, ld, H, e, y);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < R; ++k) {   // X += ||r|| * V y
+            const int r = tid + k * BS;
+            if (r < n) {
+                double d = 0.0;
+                for (int j = 0; j < steps; ++j) d = d + static_cast<double>(a.V[j * a.ldv + r0 + r]) * y[j];
+                x[k] = x[k] + rn * d;
+                XS[r] = x[k];
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+        if (tid + k * BS < n) a.X[r0 + tid + k * BS] = x[k];
+    if (tid == 0) wg_report(a, sys, refinements, inner, rn, normF);
+}
+
+// Systems of any size: vectors in global memory.
+template <int BS, int QW>
+__device__ void wg_solve_global(const WgArgs &a, double *sm, int &s_done)
+{
     const int ld = a.kin + 1;
     double *H = sm, *cs = H + ld * ld, *sn = cs + ld, *e = sn + ld, *y = e + ld, *red = y + ld;
     const int sys = blockIdx.x, tid = threadIdx.x;
-    const int r0 = a.row_off[sys], r1 = a.row_off[sys + 1];
+    const int r0 = a.row_off ? a.row_off[sys] : 0, r1 = a.row_off ? a.row_off[sys + 1] : a.n;
     float *T0 = a.T, *T1 = a.T + a.ldv, *T2 = a.T + 2 * a.ldv;
 
     double acc = 0.0;
@@ -251,26 +604,144 @@ __global__ __launch_bounds__(BS) void k_gmres_wg(WgArgs a)
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        femgpu_batch_info inf;
-        inf.refinements = refinements;
-        inf.inner_iterations = inner;
-        inf.status = (rn <= a.tol * normF) ? 0 : 1;
-        inf.pad = 0;
-        inf.normF = normF;
-        inf.true_rel_residual = normF > 0.0 ? rn / normF : 0.0;
-        a.info[sys] = inf;
+    if (tid == 0) wg_report(a, sys, refinements, inner, rn, normF);
+}
+
+// R rows per thread at most in LDS systems (the size alone decides a system's path, so its answer does not
+// depend on the batch); LARGE: systems of more rows are possible.
+template <int BS, int QW, int R, bool LARGE>
+__global__ __launch_bounds__(BS) void k_gmres_wg(WgArgs a)
+{
+    extern __shared__ double sm[];
+    __shared__ int s_done;
+    if constexpr (LARGE) {
+        if ((a.row_off ? a.row_off[blockIdx.x + 1] - a.row_off[blockIdx.x] : a.n) > R * BS) {
+            wg_solve_global<BS, QW>(a, sm, s_done);
+            return;
+        }
     }
+    wg_solve_lds<BS, QW, R>(a, sm, &s_done);
+}
+
+constexpr int kWgLdsRows = 4;   // most rows per thread of an LDS system
+
+template <int BS, int QW>
+static void wg_launch(femgpu_ctx *ctx, const WgArgs &a, int nsys, int widest)
+{
+    const int ld = a.kin + 1, r = (widest + BS - 1) / BS;
+    const auto lds = [&](int rows) {
+        return sizeof(double) * (static_cast<size_t>(ld) * ld + 4 * ld + 2 * (BS / 64) + static_cast<size_t>(rows) * BS);
+    };
+    if (r > kWgLdsRows) k_gmres_wg<BS, QW, kWgLdsRows, true><<<nsys, BS, lds(kWgLdsRows), ctx->stream>>>(a);
+    else if (r == 4) k_gmres_wg<BS, QW, 4, false><<<nsys, BS, lds(4), ctx->stream>>>(a);
+    else if (r == 3) k_gmres_wg<BS, QW, 3, false><<<nsys, BS, lds(3), ctx->stream>>>(a);
+    else if (r == 2) k_gmres_wg<BS, QW, 2, false><<<nsys, BS, lds(2), ctx->stream>>>(a);
+    else k_gmres_wg<BS, QW, 1, false><<<nsys, BS, lds(1), ctx->stream>>>(a);
+}
+
+template <int QW>
+static void wg_launch_width(femgpu_ctx *ctx, const WgArgs &a, int nsys, int widest, int threads)
+{
+    if (threads == 256) wg_launch<256, QW>(ctx, a, nsys, widest);
+    else if (threads == 512) wg_launch<512, QW>(ctx, a, nsys, widest);
+    else wg_launch<1024, QW>(ctx, a, nsys, widest);
 }
 
 }  // namespace
 
-// Workgroup size from the systems' mean size when the caller leaves it to the library: 4 waves up
-// to 2048 rows, 8 up to 8192, 16 above.
+// Workgroup size from the systems' mean size when the caller leaves it to the library: as few wavefronts as
+// hold the rows with their matrix in registers (steady systems of 500 / 1 000 / 2 000 rows: 512 threads 137 /
+// 477 / 1 427 us, 1 024 threads 194 / 533 / 1 385 us).
 int wg_threads_for(long long rows, int nsys)
 {
     const long long mean = rows / std::max(1, nsys);
-    return mean <= 2048 ? 256 : mean <= 8192 ? 512 : 1024;
+    return mean <= 256 ? 256 : mean <= 1536 ? 512 : 1024;
+}
+
+// One launch over nsys systems (row_off: host offsets; null: the whole matrix is one system) after the
+// parallel factorisation; info: device-visible memory, valid once the stream has passed the launch.
+static int wg_enqueue(femgpu_ctx *ctx, femgpu_csr *A, int nsys, const int *row_off, const femgpu_mixed_opts *opt, double tol,
+                      int threads, const double *d_F, double *d_X, femgpu_batch_info *d_info)
+{
+    const int n = A->n, kin = opt->inner_kmax;
+    FG_TRY(launch_parilu32(ctx, A, opt->factor_sweeps));
+    A->f32_factored = true;
+    const size_t ldv = (static_cast<size_t>(n) + 63) / 64 * 64;
+    FG_TRY(ctx->gm_basis32.alloc(ldv * (kin + 1)));
+    FG_TRY(ctx->gm_w32.alloc(ldv * 3));
+    FG_TRY(ctx->gm_r.alloc(static_cast<size_t>(n) + 64));
+    if (row_off) FG_TRY(ctx->bt_rowoff.upload(row_off, static_cast<size_t>(nsys) + 1, ctx->stream));
+    int widest = row_off ? 0 : n;
+    if (row_off)
+        for (int k = 0; k < nsys; ++k) widest = std::max(widest, row_off[k + 1] - row_off[k]);
+    WgArgs a;
+    a.row_off = row_off ? ctx->bt_rowoff.p : nullptr;
+    a.n = n;
+    a.IA = A->IA.p;
+    a.JA = A->JA.p;
+    a.AA = A->AA.p;
+    a.sptr = A->sell_ptr.p;
+    a.scol = A->sell_col.p;
+    a.sval = A->sell_val.p;
+    a.rinfo = A->par_rinfo.p;
+    a.LU = A->par_a.p;
+    a.Dinv = A->Dinv32.p;
+    a.F = d_F;
+    a.X = d_X;
+    a.R = ctx->gm_r.p;
+    a.V = ctx->gm_basis32.p;
+    a.T = ctx->gm_w32.p;
+    a.ldv = ldv;
+    a.kin = kin;
+    a.jac = opt->sweep_mode;
+    a.max_ref = opt->max_refinements;
+    a.tol = tol;
+    a.inner_tol = opt->inner_tol;
+    a.info = d_info;
+    // row-width bound of the unrolled entry loops: the sliced-ELL layout holds rows of <= 16 entries
+    if (A->par_maxw <= 8) wg_launch_width<8>(ctx, a, nsys, widest, threads);
+    else if (A->par_maxw <= 12) wg_launch_width<12>(ctx, a, nsys, widest, threads);
+    else wg_launch_width<16>(ctx, a, nsys, widest, threads);
+    FG_HIP(hipGetLastError());
+    return FEMGPU_OK;
+}
+
+// Whether the multi-launch mixed solvers hand a solve to the workgroup solver: the same operator and
+// preconditioner, systems small enough for its LDS path, one workgroup each. Their own launches cost about
+// 3 us each whatever the rows, 6 + i of them in Arnoldi step i (4 with classical Gram-Schmidt). Transient
+// systems of 361 / 1 472 / 3 481 rows: 84 / 181 / 337 us against 479 / 669 / 601 us; a steady one of 3 800
+// rows 2.42 ms against 3.97 ms; batches of 16 steady systems of 1 000 / 2 000 / 3 000 rows 0.48 / 1.38 /
+// 2.06 ms against 2.06 / 2.29 / 2.51 ms for the block-diagonal launches.
+bool wg_preferred(const femgpu_ctx *ctx, const femgpu_system *S, const femgpu_mixed_opts *opt, int nsys, int widest)
+{
+    const femgpu_csr *A = S->csr;
+    return A && S->ilu == A && A->sell_ok && A->par_ok && A->n > 0 && opt->factor_sweeps >= 1 && opt->factor_sweeps <= 16 &&
+           opt->sweep_mode >= 1 && opt->sweep_mode <= 16 && opt->inner_kmax >= 2 && opt->inner_kmax <= kWgMaxBasis &&
+           opt->max_refinements >= 1 && nsys <= ctx->num_cus && widest <= (nsys == 1 ? 4096 : 3072);
+}
+
+int wg_solve_one(femgpu_ctx *ctx, femgpu_csr *A, const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
+                 femgpu_batch_info *info)
+{
+    // the result goes to host-mapped memory past the solvers' status words
+    constexpr int kAt = 240;
+    static_assert(kAt % 2 == 0 && kAt * sizeof(int) + sizeof(femgpu_batch_info) <= 256 * sizeof(int), "inside the status words");
+    const int width = A->par_maxw <= 8 ? 8 : A->par_maxw <= 12 ? 12 : 16;
+    const int threads = A->n <= 256 ? 256 : A->n <= 512 * (32 / width) ? 512 : 1024;
+    FG_TRY(wg_enqueue(ctx, A, 1, nullptr, opt, tol, threads, d_F, d_X, reinterpret_cast<femgpu_batch_info *>(ctx->d_status + kAt)));
+    FG_HIP(hipStreamSynchronize(ctx->stream));
+    memcpy(info, const_cast<const int *>(ctx->h_status + kAt), sizeof(*info));
+    return FEMGPU_OK;
+}
+
+int wg_solve_batch(femgpu_ctx *ctx, femgpu_csr *A, int nsys, const int *row_off, const femgpu_mixed_opts *opt, double tol,
+                   int threads, const double *d_F, double *d_X, femgpu_batch_info *info)
+{
+    FG_TRY(ctx->wg_info.alloc(static_cast<size_t>(nsys)));
+    FG_TRY(wg_enqueue(ctx, A, nsys, row_off, opt, tol, threads, d_F, d_X, ctx->wg_info.p));
+    FG_HIP(hipMemcpyAsync(info, ctx->wg_info.p, sizeof(femgpu_batch_info) * nsys, hipMemcpyDeviceToHost, ctx->stream));
+    FG_HIP(hipStreamSynchronize(ctx->stream));
+    return FEMGPU_OK;
 }
 
 }  // namespace fg
@@ -300,58 +771,5 @@ extern "C" int femgpu_gmres_mixed_wg(femgpu_ctx *ctx, const femgpu_system *S, in
              "femgpu_gmres_mixed_wg: the matrix has no sliced-ELL factor layout (rows wider than 16 entries or "
              "created without the mixed-precision plans)");
     if (threads == 0) threads = wg_threads_for(n, nsys);
-    const int kin = opt->inner_kmax;
-    FG_TRY(launch_parilu32(ctx, A, opt->factor_sweeps));
-    A->f32_factored = true;
-    const size_t ldv = (static_cast<size_t>(n) + 63) / 64 * 64;
-    FG_TRY(ctx->gm_basis32.alloc(ldv * (kin + 1)));
-    FG_TRY(ctx->gm_w32.alloc(ldv * 3));
-    FG_TRY(ctx->gm_r.alloc(static_cast<size_t>(n) + 64));
-    FG_TRY(ctx->wg_info.alloc(static_cast<size_t>(nsys)));
-    FG_TRY(ctx->bt_rowoff.upload(row_off, static_cast<size_t>(nsys) + 1, ctx->stream));
-    WgArgs a;
-    a.row_off = ctx->bt_rowoff.p;
-    a.IA = A->IA.p;
-    a.JA = A->JA.p;
-    a.AA = A->AA.p;
-    a.sptr = A->sell_ptr.p;
-    a.scol = A->sell_col.p;
-    a.sval = A->sell_val.p;
-    a.rinfo = A->par_rinfo.p;
-    a.LU = A->par_a.p;
-    a.Dinv = A->Dinv32.p;
-    a.F = d_F;
-    a.X = d_X;
-    a.R = ctx->gm_r.p;
-    a.V = ctx->gm_basis32.p;
-    a.T = ctx->gm_w32.p;
-    a.ldv = ldv;
-    a.kin = kin;
-    a.jac = opt->sweep_mode;
-    a.max_ref = opt->max_refinements;
-    a.tol = tol;
-    a.inner_tol = opt->inner_tol;
-    a.info = ctx->wg_info.p;
-    const int ld = kin + 1;
-    const size_t lds = sizeof(double) * (static_cast<size_t>(ld) * ld + 4 * ld + 16);
-    // row-width bound of the unrolled entry loops: the sliced-ELL layout holds rows of <= 16 entries
-    const bool narrow = A->par_maxw <= 8;
-    switch (threads) {
-    case 256:
-        if (narrow) k_gmres_wg<256, 8><<<nsys, 256, lds, ctx->stream>>>(a);
-        else k_gmres_wg<256, 16><<<nsys, 256, lds, ctx->stream>>>(a);
-        break;
-    case 512:
-        if (narrow) k_gmres_wg<512, 8><<<nsys, 512, lds, ctx->stream>>>(a);
-        else k_gmres_wg<512, 16><<<nsys, 512, lds, ctx->stream>>>(a);
-        break;
-    default:
-        if (narrow) k_gmres_wg<1024, 8><<<nsys, 1024, lds, ctx->stream>>>(a);
-        else k_gmres_wg<1024, 16><<<nsys, 1024, lds, ctx->stream>>>(a);
-        break;
-    }
-    FG_HIP(hipGetLastError());
-    FG_HIP(hipMemcpyAsync(info, ctx->wg_info.p, sizeof(femgpu_batch_info) * nsys, hipMemcpyDeviceToHost, ctx->stream));
-    FG_HIP(hipStreamSynchronize(ctx->stream));
-    return FEMGPU_OK;
+    return wg_solve_batch(ctx, A, nsys, row_off, opt, tol, threads, d_F, d_X, info);
 }

@@ -1,0 +1,96 @@
+"""The small mixed-precision solves that run as one workgroup's launch: sizes where the rows per thread, the
+workgroup or the route change, rows of up to 8, 12 and 16 entries, single systems and batches, and the
+answers that need no solve. Residuals are checked with numpy in 64 bits."""
+import numpy as np
+import pytest
+
+from parallel_fem_codes_amd import fem
+
+pytestmark = pytest.mark.gpu
+
+
+def system(n, width, seed):
+    """A diagonally dominant system with rows of up to `width` entries at random distances up to 40."""
+    rng = np.random.default_rng(seed)
+    rows = []
+    for i in range(n):
+        near = np.arange(max(0, i - 40), min(n, i + 41))
+        near = near[near != i]
+        k = min(len(near), int(rng.integers(width // 2, width)))
+        rows.append(np.sort(np.concatenate([rng.choice(near, k, replace=False), [i]])))
+    if n > 80:
+        rows[40] = np.sort(np.concatenate([np.arange(41 - width, 40), [40]]))   # one row of the full width
+    IA = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    JA = np.concatenate(rows).astype(np.int32)
+    AA = rng.uniform(-1, 1, len(JA))
+    r = np.repeat(np.arange(n), np.diff(IA))
+    AA[JA == r] = 1.5 + 0.6 * np.bincount(r, weights=np.abs(AA), minlength=n)
+    return IA, JA, AA, rng.standard_normal(n)
+
+
+def residual(IA, JA, AA, F, x):
+    return np.linalg.norm(F - np.add.reduceat(AA * x[JA], IA[:-1])) / np.linalg.norm(F)
+
+
+@pytest.mark.parametrize("width", [7, 12, 16])
+@pytest.mark.parametrize("n", [1, 2, 63, 256, 257, 1024, 1025, 1366, 2048, 2049, 4096, 4097])
+def test_single(n, width):
+    import torch
+    IA, JA, AA, F = system(n, min(width, max(n, 2)), n + width)
+    dev = fem.Device(0)
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(AA)
+    Fd = torch.from_numpy(F).cuda()
+    X = torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")
+    for kw in (dict(sweep_mode=2, factor_sweeps=1), dict(sweep_mode=1, factor_sweeps=3, inner_kmax=64),
+               dict(sweep_mode=3, factor_sweeps=2, inner_kmax=4)):
+        info = fem.gmres_mixed(dev, A, Fd, X, tol=1e-10, **kw)
+        res = residual(IA, JA, AA, F, X.cpu().numpy())
+        assert info.status == 0 and res <= 1.01e-10, (kw, res)
+        assert abs(res - info.true_rel_residual) <= 1e-3 * res + 1e-15
+        assert info.iterations == info.inner_iterations > 0 and info.cycles > 0
+        assert np.isclose(info.normb, np.linalg.norm(F), rtol=1e-14)
+
+
+def test_answers_without_a_solve():
+    import torch
+    IA, JA, AA, F = system(300, 7, 5)
+    dev = fem.Device(0)
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(AA)
+    kw = dict(sweep_mode=2, factor_sweeps=1)
+    for Fv, extra, status in ((0 * F, {}, 0), (F, dict(tol=1.0), 0), (F, dict(max_refinements=0), 1),
+                              (np.where(np.arange(300) == 7, np.inf, F), {}, 1),
+                              (np.where(np.arange(300) == 7, np.nan, F), {}, 1)):
+        X = torch.full((300,), 3.0, dtype=torch.float64, device="cuda")
+        info = fem.gmres_mixed(dev, A, torch.from_numpy(Fv).cuda(), X, **{"tol": 1e-8, **kw, **extra})
+        assert info.status == status and (X == 0).all()
+    X = torch.empty(300, dtype=torch.float64, device="cuda")
+    info = fem.gmres_mixed(dev, A, torch.from_numpy(F).cuda(), X, tol=1e-14, max_refinements=1, **kw)
+    assert info.status == 1 and info.cycles == 1 and 0 < info.true_rel_residual < 1
+
+
+@pytest.mark.parametrize("sizes", [[5, 300, 0, 1, 1500], [3072, 40], [3073, 40], [700] * 5])
+def test_batch(sizes):
+    """Systems of one batch, one of them empty, one with a zero right-hand side; each as when alone."""
+    import torch
+    dev = fem.Device(0)
+    syss = [system(n, 9, 100 + k) for k, n in enumerate(sizes) if n] if 0 not in sizes else \
+        [system(n, 9, 100 + k) if n else (np.zeros(1, np.int32), np.zeros(0, np.int32), np.zeros(0), np.zeros(0))
+         for k, n in enumerate(sizes)]
+    syss[0] = syss[0][:3] + (0 * syss[0][3],)
+    IA, JA, off, _ = fem.concat_csr([(s[0], s[1]) for s in syss])
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(np.concatenate([s[2] for s in syss]))
+    X = torch.full((off[-1],), float("nan"), dtype=torch.float64, device="cuda")
+    infos = fem.gmres_mixed_batched(dev, A, off, torch.from_numpy(np.concatenate([s[3] for s in syss])).cuda(), X, tol=1e-9,
+                                    orthogonalization="CGS")
+    x = X.cpu().numpy()
+    for k, (s, i) in enumerate(zip(syss, infos)):
+        xk = x[off[k]:off[k + 1]]
+        assert i.status == 0
+        if not len(xk) or not s[3].any():
+            assert (xk == 0).all() and i.refinements == 0
+            continue
+        assert residual(*s, xk) <= 1.01e-9
+        assert abs(residual(*s, xk) - i.true_rel_residual) <= 1e-3 * i.true_rel_residual + 1e-15
