@@ -407,7 +407,10 @@ bool sell64_active(const femgpu_csr *A);     // the FP64 kernels read sell_val64
 int set_spmv_lanes(femgpu_csr *A, int lanes);   // 0: FP64 sliced ELL (allocates and fills sell_val64)
 int launch_to_f32(femgpu_ctx *ctx, const double *src, float *dst, size_t n);
 int launch_ebemv(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, double *Q, const int *skip = nullptr);
-int launch_ebemv32(femgpu_ctx *ctx, const femgpu_ebe *E, const float *P, float *Q, const int *skip = nullptr);
+// xs, xout: the operand P * *xs, stored to xout on the way (where ebe_scales(E): every unknown in an element)
+int launch_ebemv32(femgpu_ctx *ctx, const femgpu_ebe *E, const float *P, float *Q, const int *skip = nullptr,
+                   const double *xs = nullptr, float *xout = nullptr);
+bool ebe_scales(const femgpu_ebe *E);
 int launch_blockdiag_apply32(femgpu_ctx *ctx, const femgpu_blockdiag *B, const float *p, float *z, const int *skip);
 
 int dot64(femgpu_ctx *ctx, int n, const double *x, const double *y, double *d_out);

@@ -105,7 +105,8 @@ __global__ void k_ebe_zero(int n, T *__restrict__ q, const int *__restrict__ ski
 // 801 x 401 nodes, ND = 4, 29 us back to back and 39.6 us from HBM (170 MB; 81 us on the FP32 copy of
 // the element rows, 412 MB). The FP64 product keeps the element rows: its sums are the reference's, bit for bit.
 // Block row r of lane l: ND values of dof row d at ((r*ND + d)*64 + l)*ND, the ND columns at
-// (r*64 + l)*ND.
+// (r*64 + l)*ND. xs, xout: the operand is P * *xs, and that product is stored to xout (the Arnoldi
+// normalisation, as k_spmv's).
 template <int ND>
 struct NodeVec {
     float v[ND];
@@ -116,6 +117,7 @@ __global__ __launch_bounds__(256) void k_node_rows(int ngroups, int NEQ, const i
                                                    const int *__restrict__ blen, const int *__restrict__ eq,
                                                    const int *__restrict__ key, const CT *__restrict__ col,
                                                    const float *__restrict__ val, const float *__restrict__ P,
+                                                   const double *__restrict__ xs_ptr, float *__restrict__ xout,
                                                    float *__restrict__ Q, const int *__restrict__ skip)
 {
     if (skip && *skip) return;
@@ -123,6 +125,7 @@ __global__ __launch_bounds__(256) void k_node_rows(int ngroups, int NEQ, const i
     if (g >= ngroups) return;
     const int sl = g >> 6, l = g & 63;
     const int r0 = bptr[sl], n = blen[g];
+    const float xs = xs_ptr ? static_cast<float>(*xs_ptr) : 1.0f;
     const int kg = key ? key[g] : 0;
     double acc[ND];   // FP32 products are exact in FP64: one rounding at the end
 #pragma unroll
@@ -150,7 +153,7 @@ __global__ __launch_bounds__(256) void k_node_rows(int ngroups, int NEQ, const i
 #pragma unroll
             for (int b = 0; b < ND; ++b) {
                 const int idx = ebe_col<CT>(c[b], kg, NEQ);
-                const float pv = P[idx >= 0 ? idx : 0];
+                const float pv = P[idx >= 0 ? idx : 0] * xs;
                 p[u][b] = idx >= 0 ? pv : 0.0f;
             }
         }
@@ -167,7 +170,10 @@ __global__ __launch_bounds__(256) void k_node_rows(int ngroups, int NEQ, const i
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
         const int q = eq[(static_cast<size_t>(sl) * ND + d) * 64 + l];
-        if (q < NEQ) Q[q] = static_cast<float>(acc[d]);
+        if (q < NEQ) {
+            Q[q] = static_cast<float>(acc[d]);
+            if (xout) xout[q] = P[q] * xs;
+        }
     }
 }
 
@@ -291,13 +297,13 @@ __global__ __launch_bounds__(256) void k_node_rows_fill(const int *__restrict__ 
 
 template <typename CT, int ND, int U, int U32>
 static void gather_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const CT *col, const CT *bcol, const double *P, double *Q,
-                          const float *P32, float *Q32, const int *skip)
+                          const float *P32, float *Q32, const int *skip, const double *xs, float *xout)
 {
     const int grid = xcd_grid((E->ngroups + 255) / 256);
     const int *key = E->col16 ? E->key.p : nullptr;
     if (P32)
         k_node_rows<CT, ND, U32><<<grid, 256, 0, ctx->stream>>>(E->ngroups, E->NEQ, E->bptr.p, E->blen.p, E->eq.p, key, bcol,
-                                                               E->val32.p, P32, Q32, skip);
+                                                               E->val32.p, P32, xs, xout, Q32, skip);
     else
         k_ebe_gather<double, CT, ND, U><<<grid, 256, 0, ctx->stream>>>(E->ngroups, E->NEQ, E->iptr.p, E->len.p, E->eq.p, key,
                                                                        col, E->val.p, P, Q, skip);
@@ -305,7 +311,7 @@ static void gather_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const CT *col, c
 
 // Q = A P in FP64 (P32 null) or FP32.
 static int ebe_product(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, double *Q, const float *P32, float *Q32,
-                       const int *skip)
+                       const int *skip, const double *xs = nullptr, float *xout = nullptr)
 {
     FG_CHECK(E->has_values, FEMGPU_ERR_STATE, "femgpu_ebemv: element matrices not set");
     if (E->zero_q && E->NEQ > 0) {
@@ -319,16 +325,16 @@ static int ebe_product(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, do
     const int *c32 = E->col32v.p, *b32 = E->bcol32.p;
     switch (E->ndof) {
     case 1:
-        if (E->col16) gather_launch<short, 1, 6, 7>(ctx, E, c16, b16, P, Q, P32, Q32, skip);
-        else gather_launch<int, 1, 6, 7>(ctx, E, c32, b32, P, Q, P32, Q32, skip);
+        if (E->col16) gather_launch<short, 1, 6, 7>(ctx, E, c16, b16, P, Q, P32, Q32, skip, xs, xout);
+        else gather_launch<int, 1, 6, 7>(ctx, E, c32, b32, P, Q, P32, Q32, skip, xs, xout);
         break;
     case 3:
-        if (E->col16) gather_launch<short, 3, 1, 4>(ctx, E, c16, b16, P, Q, P32, Q32, skip);
-        else gather_launch<int, 3, 1, 4>(ctx, E, c32, b32, P, Q, P32, Q32, skip);
+        if (E->col16) gather_launch<short, 3, 1, 4>(ctx, E, c16, b16, P, Q, P32, Q32, skip, xs, xout);
+        else gather_launch<int, 3, 1, 4>(ctx, E, c32, b32, P, Q, P32, Q32, skip, xs, xout);
         break;
     default:
-        if (E->col16) gather_launch<short, 4, 1, 4>(ctx, E, c16, b16, P, Q, P32, Q32, skip);
-        else gather_launch<int, 4, 1, 4>(ctx, E, c32, b32, P, Q, P32, Q32, skip);
+        if (E->col16) gather_launch<short, 4, 1, 4>(ctx, E, c16, b16, P, Q, P32, Q32, skip, xs, xout);
+        else gather_launch<int, 4, 1, 4>(ctx, E, c32, b32, P, Q, P32, Q32, skip, xs, xout);
         break;
     }
     FG_HIP(hipGetLastError());
@@ -340,10 +346,14 @@ int launch_ebemv(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, double *
     return ebe_product(ctx, E, P, Q, nullptr, nullptr, skip);
 }
 
-int launch_ebemv32(femgpu_ctx *ctx, const femgpu_ebe *E, const float *P, float *Q, const int *skip)
+int launch_ebemv32(femgpu_ctx *ctx, const femgpu_ebe *E, const float *P, float *Q, const int *skip, const double *xs,
+                   float *xout)
 {
-    return ebe_product(ctx, E, nullptr, nullptr, P, Q, skip);
+    FG_CHECK(!xout || ebe_scales(E), FEMGPU_ERR_ARG, "EBE product: some unknown has no node row to store its scaled value");
+    return ebe_product(ctx, E, nullptr, nullptr, P, Q, skip, xs, xout);
 }
+
+bool ebe_scales(const femgpu_ebe *E) { return !E->zero_q; }
 
 template <int ND>
 static int fill_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const double *Ae)

@@ -44,8 +44,7 @@ constexpr int kMaxBasis = 150;   // largest GMRES basis (make_gdev)
 // Givens update of column i and the convergence test (pgmres.c:118-159), with h_{i+1,i} = hn.
 // Called by every thread of the block: the block stages the column, the earlier rotations and
 // e[i] in LDS with loads issued together, then one thread applies the rotations -- the operations
-// of a serial update in the same order -- and stores the results (a serial update in global memory
-// would wait for every read after a write to the same column).
+// of a serial update in the same order -- and stores the results.
 __device__ void givens_column(const GDev &G, int i, double hn)
 {
 #pragma clang fp contract(off)
@@ -58,19 +57,34 @@ __device__ void givens_column(const GDev &G, int i, double hn)
     if (threadIdx.x == 0) ei_s = G.e[i];
     __syncthreads();
     if (threadIdx.x != 0) return;
-    col[i + 1] = hn;
-    for (int j = 0; j <= i - 1; ++j) {
-        const double h1 = cs[j] * col[j] + sn[j] * col[j + 1];
-        const double h2 = -sn[j] * col[j] + cs[j] * col[j + 1];
-        col[j] = h1;
-        col[j + 1] = h2;
+    // the entry that the rotations carry along stays in a register and eight rotations' operands are read
+    // ahead: an LDS round trip per rotation would be most of this kernel's time
+    double run = col[0];
+    int j0 = 0;
+    for (; j0 + 8 <= i; j0 += 8) {
+        double cj[8], sj[8], hj[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            cj[u] = cs[j0 + u];
+            sj[u] = sn[j0 + u];
+            hj[u] = col[j0 + u + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            Hat(G, j0 + u, i) = cj[u] * run + sj[u] * hj[u];
+            run = -sj[u] * run + cj[u] * hj[u];
+        }
     }
-    const double a = col[i], b = col[i + 1];
+    for (; j0 < i; ++j0) {
+        const double hj = col[j0 + 1];
+        Hat(G, j0, i) = cs[j0] * run + sn[j0] * hj;
+        run = -sn[j0] * run + cs[j0] * hj;
+    }
+    const double a = run, b = hn;
     const double r = sqrt(a * a + b * b);
     const double ci = a / r, si = b / r;
     G.c[i] = ci;
     G.s[i] = si;
-    for (int k = 0; k < i; ++k) Hat(G, k, i) = col[k];
     Hat(G, i, i) = r;
     Hat(G, i + 1, i) = 0.0;
     const double ei = ei_s;
@@ -228,46 +242,56 @@ __global__ __launch_bounds__(256) void k_mgs_finish(GDev G, int nb, int i)
 // the inner solve of the refinement tolerates; the outer FP64 loop verifies the answer.
 constexpr int kCgsBlocks = kReduceBlocks, kCgsChunk = 8;
 
+// Block row y takes the coefficients 8y .. 8y + 7 (a loop over the chunks in one block made a small system's
+// pass as long as its chunks: 13 us at i = 25 of 80 000 unknowns, TIME_DOTS with the chunks side by side).
 __global__ __launch_bounds__(256) void k_cgs_dots(GDev G, int n, int i, const float *__restrict__ w,
                                                   const float *__restrict__ V, size_t ldv, double *__restrict__ part)
 {
     if (G.flags[0]) return;
     __shared__ double red[4 * kCgsChunk];
-    const int nv = n / 4;
-    for (int j0 = 0; j0 <= i; j0 += kCgsChunk) {
-        double acc[kCgsChunk];
+    const int nv = n / 4, j0 = static_cast<int>(blockIdx.y) * kCgsChunk;
+    double acc[kCgsChunk];
 #pragma unroll
-        for (int c = 0; c < kCgsChunk; ++c) acc[c] = 0.0;
-        for (int k = blockIdx.x * 256 + threadIdx.x; k < nv; k += gridDim.x * 256) {
-            const float4 wv = reinterpret_cast<const float4 *>(w)[k];
-            float4 v[kCgsChunk];
+    for (int c = 0; c < kCgsChunk; ++c) acc[c] = 0.0;
+    for (int k = blockIdx.x * 256 + threadIdx.x; k < nv; k += gridDim.x * 256) {
+        const float4 wv = reinterpret_cast<const float4 *>(w)[k];
+        float4 v[kCgsChunk];
 #pragma unroll
-            for (int c = 0; c < kCgsChunk; ++c)
-                if (j0 + c <= i) v[c] = reinterpret_cast<const float4 *>(V + (j0 + c) * ldv)[k];
+        for (int c = 0; c < kCgsChunk; ++c)
+            if (j0 + c <= i) v[c] = reinterpret_cast<const float4 *>(V + (j0 + c) * ldv)[k];
 #pragma unroll
-            for (int c = 0; c < kCgsChunk; ++c)
-                if (j0 + c <= i)
-                    acc[c] += static_cast<double>(v[c].x) * wv.x + static_cast<double>(v[c].y) * wv.y +
-                              static_cast<double>(v[c].z) * wv.z + static_cast<double>(v[c].w) * wv.w;
-        }
-        if (blockIdx.x == 0)
-            for (int k = nv * 4 + threadIdx.x; k < n; k += 256)
-#pragma unroll
-                for (int c = 0; c < kCgsChunk; ++c)
-                    if (j0 + c <= i) acc[c] += static_cast<double>(V[(j0 + c) * ldv + k]) * w[k];
-        // all coefficients of the chunk reduced together: wave sums, one barrier, then thread c
-        // adds the four wave sums of coefficient c in wave order
-#pragma unroll
-        for (int c = 0; c < kCgsChunk; ++c) acc[c] = wave_sum(acc[c]);
-        __syncthreads();
-        if (threadIdx.x % 64 == 0)
-#pragma unroll
-            for (int c = 0; c < kCgsChunk; ++c) red[c * 4 + threadIdx.x / 64] = acc[c];
-        __syncthreads();
-        if (threadIdx.x < kCgsChunk && j0 + threadIdx.x <= i)
-            part[(j0 + threadIdx.x) * kCgsBlocks + blockIdx.x] =
-                ((red[threadIdx.x * 4] + red[threadIdx.x * 4 + 1]) + red[threadIdx.x * 4 + 2]) + red[threadIdx.x * 4 + 3];
+        for (int c = 0; c < kCgsChunk; ++c)
+            if (j0 + c <= i)
+                acc[c] += static_cast<double>(v[c].x) * wv.x + static_cast<double>(v[c].y) * wv.y +
+                          static_cast<double>(v[c].z) * wv.z + static_cast<double>(v[c].w) * wv.w;
     }
+    if (blockIdx.x == 0)
+        for (int k = nv * 4 + threadIdx.x; k < n; k += 256)
+#pragma unroll
+            for (int c = 0; c < kCgsChunk; ++c)
+                if (j0 + c <= i) acc[c] += static_cast<double>(V[(j0 + c) * ldv + k]) * w[k];
+    // the chunk's eight sums over the wavefront together: three exchanges halve the coefficients a lane
+    // keeps, three more add the remaining lanes (10 exchanges instead of 48)
+    static_assert(kCgsChunk == 8, "three halvings");
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int h = 4; h >= 1; h >>= 1) {
+        const bool up = l & (8 * h);
+#pragma unroll
+        for (int c = 0; c < h; ++c) {
+            const double give = up ? acc[c] : acc[c + h], keep = up ? acc[c + h] : acc[c];
+            acc[c] = keep + __shfl_xor(give, 8 * h, 64);
+        }
+    }
+    double t = acc[0];   // coefficient (l >> 3): bits 5, 4, 3 chose the halves of 4, 2 and 1
+    t += __shfl_xor(t, 4, 64);
+    t += __shfl_xor(t, 2, 64);
+    t += __shfl_xor(t, 1, 64);
+    if ((l & 7) == 0) red[(l >> 3) * 4 + threadIdx.x / 64] = t;
+    __syncthreads();
+    if (threadIdx.x < kCgsChunk && j0 + static_cast<int>(threadIdx.x) <= i)
+        part[(j0 + threadIdx.x) * kCgsBlocks + blockIdx.x] =
+            ((red[threadIdx.x * 4] + red[threadIdx.x * 4 + 1]) + red[threadIdx.x * 4 + 2]) + red[threadIdx.x * 4 + 3];
 }
 
 // Block j: h_{j,i} = the fixed-order sum of the nb partials of coefficient j.
@@ -281,26 +305,52 @@ __global__ __launch_bounds__(256) void k_cgs_reduce(GDev G, int nb, int i, const
 }
 
 // w -= sum_j h_{j,i} V[j] (FP32, j ascending; loads of a chunk of basis vectors issued together) and
-// the partials of ||w||^2.
+// the partials of ||w||^2. nsum > 0: every block first forms the h_{j,i} itself from their nsum partials
+// (four lanes per coefficient, the same order in every block) and block 0 stores them: for few partials that
+// costs less than the launch of k_cgs_reduce.
+constexpr int kCgsLoad = 16;      // basis vectors whose loads an update has in flight
+constexpr int kCgsSumMax = 128;   // partials per coefficient up to which the blocks sum them
 __global__ __launch_bounds__(256) void k_cgs_update(GDev G, int n, int i, float *__restrict__ w,
-                                                    const float *__restrict__ V, size_t ldv, double *__restrict__ part)
+                                                    const float *__restrict__ V, size_t ldv, double *__restrict__ part,
+                                                    int nsum)
 {
     if (G.flags[0]) return;
     __shared__ double red[4];
     __shared__ float h[160];
-    for (int j = threadIdx.x; j <= i; j += 256) h[j] = static_cast<float>(Hat(G, j, i));
+    const int nv = n / 4, kfirst = blockIdx.x * 256 + threadIdx.x;
+    if (nsum > 0) {
+        const int lane4 = threadIdx.x & 3;
+        for (int j = threadIdx.x >> 2; j <= i; j += 64) {
+            const double *p = part + j * kCgsBlocks;
+            double v = 0.0;
+            for (int b0 = lane4; b0 < nsum; b0 += 32) {
+                double t[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) t[u] = b0 + 4 * u < nsum ? p[b0 + 4 * u] : 0.0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v += t[u];
+            }
+            v += __shfl_xor(v, 1, 64);
+            v += __shfl_xor(v, 2, 64);
+            if (lane4 == 0) {
+                h[j] = static_cast<float>(v);
+                if (blockIdx.x == 0) Hat(G, j, i) = v;
+            }
+        }
+    } else {
+        for (int j = threadIdx.x; j <= i; j += 256) h[j] = static_cast<float>(Hat(G, j, i));
+    }
     __syncthreads();
     double acc = 0.0;
-    const int nv = n / 4;
-    for (int k = blockIdx.x * 256 + threadIdx.x; k < nv; k += gridDim.x * 256) {
+    for (int k = kfirst; k < nv; k += gridDim.x * 256) {
         float4 wv = reinterpret_cast<const float4 *>(w)[k];
-        for (int j0 = 0; j0 <= i; j0 += kCgsChunk) {
-            float4 v[kCgsChunk];
+        for (int j0 = 0; j0 <= i; j0 += kCgsLoad) {
+            float4 v[kCgsLoad];
 #pragma unroll
-            for (int c = 0; c < kCgsChunk; ++c)
+            for (int c = 0; c < kCgsLoad; ++c)
                 if (j0 + c <= i) v[c] = reinterpret_cast<const float4 *>(V + (j0 + c) * ldv)[k];
 #pragma unroll
-            for (int c = 0; c < kCgsChunk; ++c)
+            for (int c = 0; c < kCgsLoad; ++c)
                 if (j0 + c <= i) {
                     const float hj = h[j0 + c];
                     wv.x -= hj * v[c].x;
@@ -391,31 +441,39 @@ __global__ __launch_bounds__(256) void k_cycle_start_finish(GDev G, int nb, int 
     }
 }
 
-// Back substitution H y = e over the first i + 1 columns (pgmres.c:159-170) into ys (LDS), the
-// same operations in the same order as the serial loop; called by every thread of the block. For
-// bases up to kStageBasis the block first stages the triangle and e in LDS with loads issued
-// together, so the serial loop of thread 0 does not wait on global memory per step.
-constexpr int kStageBasis = 32;
+// Back substitution H y = e over the first i + 1 columns (pgmres.c:159-170) into ys (LDS), called by every
+// thread of the block. Up to a wavefront's lanes of columns the block stages the triangle in LDS and the
+// first wavefront solves it a column at a time, lane j holding e_j less the columns done: a serial loop
+// would wait for an LDS (for larger bases a memory) round trip per entry, 60 us of the finish of a 40-step
+// cycle.
+constexpr int kStageBasis = 64;
 
 __device__ void back_substitute(const GDev &G, int i, double *ys)
 {
 #pragma clang fp contract(off)
-    __shared__ double hs[kStageBasis * kStageBasis], es[kStageBasis];
+    __shared__ double hs[kStageBasis * (kStageBasis + 1) / 2];   // column c at c (c + 1) / 2
     if (i < kStageBasis) {
         const int m = i + 1;
         for (int q = threadIdx.x; q < m * m; q += blockDim.x) {
             const int r = q / m, c = q - r * m;
-            if (c >= r) hs[q] = Hat(G, r, c);
+            if (c >= r) hs[c * (c + 1) / 2 + r] = Hat(G, r, c);
         }
-        for (int q = threadIdx.x; q < m; q += blockDim.x) es[q] = G.e[q];
         __syncthreads();
-        if (threadIdx.x == 0) {
-            ys[i] = es[i] / hs[i * m + i];
-            for (int j = i - 1; j >= 0; --j) {
-                double soma = 0.0;
-                for (int k = j + 1; k <= i; ++k) soma = soma + hs[j * m + k] * ys[k];
-                ys[j] = (es[j] - soma) / hs[j * m + j];
+        if (threadIdx.x < 64) {
+            const int l = threadIdx.x;
+            double e = l <= i ? G.e[l] : 0.0, mine = 0.0;
+            for (int k = i; k >= 0; --k) {
+                const double *col = hs + k * (k + 1) / 2;
+                const double h = col[l < k ? l : k], d = col[k];
+                const long long eb = __double_as_longlong(e);
+                const int lo = __builtin_amdgcn_readlane(static_cast<int>(eb), k);
+                const int hi = __builtin_amdgcn_readlane(static_cast<int>(eb >> 32), k);
+                const double y = __longlong_as_double(static_cast<long long>(static_cast<unsigned>(lo)) |
+                                                      (static_cast<long long>(hi) << 32)) / d;
+                mine = l == k ? y : mine;
+                e = l < k ? e - h * y : e;
             }
+            if (l <= i) ys[l] = mine;
         }
     } else if (threadIdx.x == 0) {
         ys[i] = G.e[i] / Hat(G, i, i);
@@ -425,6 +483,22 @@ __device__ void back_substitute(const GDev &G, int i, double *ys)
             ys[j] = (G.e[j] - soma) / Hat(G, j, j);
         }
     }
+}
+
+// sum over j of V[j][k] * ys[j], in ascending j from x0, eight loads in flight
+template <typename T, typename A>
+__device__ __forceinline__ A basis_sum(A x0, const T *__restrict__ V, size_t ldv, int k, int i, const double *ys)
+{
+#pragma clang fp contract(off)
+    for (int j0 = 0; j0 <= i; j0 += 8) {
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = V[(j0 + u <= i ? j0 + u : i) * ldv + k];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (j0 + u <= i) x0 = x0 + static_cast<A>(v[u]) * static_cast<A>(ys[j0 + u]);
+    }
+    return x0;
 }
 
 // Back substitution (pgmres.c:159-170) by every block into LDS, then X += scale * sum_j V[j] y[j]
@@ -438,18 +512,15 @@ __global__ __launch_bounds__(256) void k_cycle_finish(GDev G, int n, const T *__
     const int i = G.flags[1] - 1;
     if (i < 0) return;
     back_substitute(G, i, ys);
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        for (int j = 0; j <= i; ++j) G.y[j] = ys[j];
     __syncthreads();
+    if (blockIdx.x == 0)
+        for (int j = threadIdx.x; j <= i; j += 256) G.y[j] = ys[j];
     for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) {
         // assign: X was not initialised (x0 = 0): the sums start from 0 instead of X
         if (scale == 1.0) {
-            TX xv = assign ? TX(0) : X[k];
-            for (int j = 0; j <= i; ++j) xv = xv + static_cast<TX>(V[j * ldv + k]) * static_cast<TX>(ys[j]);
-            X[k] = xv;
+            X[k] = basis_sum<T, TX>(assign ? TX(0) : X[k], V, ldv, k, i, ys);
         } else {
-            double d = 0;
-            for (int j = 0; j <= i; ++j) d = d + static_cast<double>(V[j * ldv + k]) * ys[j];
+            const double d = basis_sum<T, double>(0.0, V, ldv, k, i, ys);
             X[k] = static_cast<TX>((assign ? 0.0 : static_cast<double>(X[k])) + scale * d);
         }
     }
@@ -556,8 +627,7 @@ __global__ __launch_bounds__(256) void k_cycle_finish_seg(GDev G, int n, const f
     back_substitute(G, i, ys);
     __syncthreads();
     for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) {
-        double d = 0;
-        for (int j = 0; j <= i; ++j) d = d + static_cast<double>(V[j * ldv + k]) * ys[j];
+        const double d = basis_sum<float, double>(0.0, V, ldv, k, i, ys);
         X[k] = X[k] + rn[sys[k]] * d;
     }
 }
@@ -743,7 +813,8 @@ __global__ void k_scale_copy(int n, const T *__restrict__ x, const double *__res
 
 // FP32 operator and preconditioner of the inner solver: w = M^-1 A (x * xs), with x * xs stored
 // into xout (the basis vector). CSR: the sliced-ELL SpMV with the scaling fused, then the ILU(0)
-// sweeps; EBE: the scaled copy, the gathered element product, then the nodal block-diagonal blocks.
+// sweeps; EBE: the gathered element product with the scaling
+// fused, then the nodal block-diagonal blocks.
 static int op_prec32(femgpu_ctx *ctx, const femgpu_system *S, int prec_mode, const float *x, const double *xs,
                      float *xout, float *w, const int *skip, const float *dv = nullptr, double *dpart = nullptr)
 {
@@ -751,9 +822,13 @@ static int op_prec32(femgpu_ctx *ctx, const femgpu_system *S, int prec_mode, con
         FG_TRY(launch_spmv32(ctx, S->csr, x, xs, xout, w, skip));
         return prec32(ctx, S->ilu, prec_mode, w, w, skip, dv, dpart);
     }
-    k_scale_copy<float><<<grid_for(S->ebe->NEQ) * 4, 256, 0, ctx->stream>>>(S->ebe->NEQ, x, xs, xout, skip);
-    FG_HIP(hipGetLastError());
-    FG_TRY(launch_ebemv32(ctx, S->ebe, xout, w, skip));
+    if (!ebe_scales(S->ebe)) {
+        k_scale_copy<float><<<grid_for(S->ebe->NEQ) * 4, 256, 0, ctx->stream>>>(S->ebe->NEQ, x, xs, xout, skip);
+        FG_HIP(hipGetLastError());
+        FG_TRY(launch_ebemv32(ctx, S->ebe, xout, w, skip));
+    } else {
+        FG_TRY(launch_ebemv32(ctx, S->ebe, x, w, skip, xs, xout));
+    }
     return launch_blockdiag_apply32(ctx, S->bdiag, w, w, skip);
 }
 
@@ -769,9 +844,10 @@ static int step_kernels32(femgpu_ctx *ctx, const femgpu_system *S, const GDev &G
                      nf ? ctx->jac_partials.p : nullptr));
     if (G.cgs) {
         const int nb = std::max(1, std::min(kCgsBlocks, (n / 4 + 255) / 256));
-        k_cgs_dots<<<nb, 256, 0, ctx->stream>>>(G, n, i, wn, V, ldv, ctx->cgs_partials.p);
-        k_cgs_reduce<<<i + 1, 256, 0, ctx->stream>>>(G, nb, i, ctx->cgs_partials.p);
-        k_cgs_update<<<nb, 256, 0, ctx->stream>>>(G, n, i, wn, V, ldv, ctx->cgs_partials.p);
+        const bool in_update = nb <= kCgsSumMax;
+        k_cgs_dots<<<dim3(nb, i / kCgsChunk + 1), 256, 0, ctx->stream>>>(G, n, i, wn, V, ldv, ctx->cgs_partials.p);
+        if (!in_update) k_cgs_reduce<<<i + 1, 256, 0, ctx->stream>>>(G, nb, i, ctx->cgs_partials.p);
+        k_cgs_update<<<nb, 256, 0, ctx->stream>>>(G, n, i, wn, V, ldv, ctx->cgs_partials.p, in_update ? nb : 0);
         k_cgs_finish<<<1, 256, 0, ctx->stream>>>(G, nb, i, ctx->cgs_partials.p);
     } else {
         mgs_step<float>(ctx, G, n, i, wn, V, ldv, nf, ctx->jac_partials.p);
@@ -982,7 +1058,7 @@ extern "C" int femgpu_pgmres(femgpu_ctx *ctx, const femgpu_system *S, int kmax, 
             (void)hipEventDestroy(ev[0]);
             (void)hipEventDestroy(ev[1]);
         }
-        k_cycle_finish<double, double><<<grid, 256, 0, ctx->stream>>>(G, n, V, ldv, d_X, 1.0, 0);
+        k_cycle_finish<double, double><<<std::min(4 * kReduceBlocks, grid * 4), 256, 0, ctx->stream>>>(G, n, V, ldv, d_X, 1.0, 0);
         FG_HIP(hipGetLastError());
         // device truth: steps and rho of this cycle
         FG_HIP(hipMemcpyAsync(&ctx->h_pinned[0], G.scal + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1148,7 +1224,7 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
                 rn = normF;
                 if (normF == 0.0 || !std::isfinite(normF)) return zero_answer(normF);
             }
-            k_cycle_finish<float, double><<<grid, 256, 0, ctx->stream>>>(G, n, V, ldv, d_X, rn, refinements == 0);
+            k_cycle_finish<float, double><<<std::min(4 * kReduceBlocks, grid * 4), 256, 0, ctx->stream>>>(G, n, V, ldv, d_X, rn, refinements == 0);
             FG_HIP(hipGetLastError());
             // only the level-scheduled sweeps (mode 0) can raise the device error word; otherwise the
             // next residual is enqueued right behind the update, and its norm's wait covers both
