@@ -327,7 +327,7 @@ extern "C" int femgpu_assemble_euler(femgpu_mesh *M, const femgpu_euler_problem 
 {
     FG_CHECK(M && pb && d_u && d_du && d_R, FEMGPU_ERR_ARG, "femgpu_assemble_euler: bad arguments");
     FG_CHECK(M->ndof == 4, FEMGPU_ERR_STATE, "femgpu_assemble_euler: not an Euler mesh");
-    FG_CHECK(!d_AA || M->aa_ptr.p, FEMGPU_ERR_STATE, "femgpu_assemble_euler: mesh created without a CSR slot table");
+    FG_CHECK(!d_AA || M->has_scheme, FEMGPU_ERR_STATE, "femgpu_assemble_euler: mesh created without a CSR slot table");
     femgpu_ctx *ctx = M->ctx;
     double *Ae = d_Ae ? d_Ae : M->ke.p;
     EulerIn in;

@@ -334,6 +334,14 @@ struct femgpu_mesh {
     fg::DevBuf<int4> fz_ent;
     fg::DevBuf<unsigned> fz_inc;
     fg::DevBuf<int4> fz_row;
+    // Fused Navier-Stokes assembly (built with the mesh where it applies, in place of the slot lists): every
+    // node's equations, and per block (a patch of nodes) its (element, vertex) incidences, its nodes' rows
+    // and its (node, neighbour) pairs with their contributions as LDS offsets.
+    bool nf_ok = false;
+    int nf_blocks = 0, nf_slots = 0;
+    fg::DevBuf<int4> nf_bptr, nf_inc, nf_eqs, nf_node;
+    fg::DevBuf<uint2> nf_pair;
+    fg::DevBuf<unsigned short> nf_code;
 };
 
 namespace fg {
