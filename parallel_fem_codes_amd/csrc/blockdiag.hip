@@ -19,6 +19,8 @@ struct femgpu_blockdiag {
     femgpu_ctx *ctx = nullptr;
     int nnodes = 0, nel = 0, ndof = 0, NEQ = 0;
     fg::DevBuf<int> id;                  // nnodes*ndof: equation of the dof, NEQ when prescribed
+    fg::DevBuf<int> node_of;             // NEQ: node of the unknown (-1: none)
+    int nfree = 0;                       // nodes with unknowns (-1: an unknown belongs to two dofs)
     fg::DevBuf<int> ien;                 // nel*3
     fg::DevBuf<int> inc_ptr, inc_src, inc_dst;   // node incidences e*3+a in element order
     fg::DevBuf<double> inv;              // nnodes*ndof^2 inverse blocks (row-major)
@@ -238,6 +240,16 @@ static int bd_apply(femgpu_ctx *ctx, const femgpu_blockdiag *B, const T *inv, co
     return FEMGPU_OK;
 }
 
+const float *blockdiag_inv32(const femgpu_blockdiag *B) { return B->inv32.p; }
+
+bool blockdiag_nodes(const femgpu_blockdiag *B, int ndof, int NEQ, const int **node_of, const int **id, int *nfree)
+{
+    *node_of = B->node_of.p;
+    *id = B->id.p;
+    *nfree = B->nfree;
+    return B->ndof == ndof && B->NEQ == NEQ && B->nfree >= 0;
+}
+
 int launch_blockdiag_apply(femgpu_ctx *ctx, const femgpu_blockdiag *B, const double *p, double *z, const int *skip)
 {
     return bd_apply<double>(ctx, B, B->inv.p, p, z, skip);
@@ -264,6 +276,23 @@ extern "C" int femgpu_blockdiag_create(femgpu_ctx *ctx, int nnodes, int nel, int
                  "femgpu_blockdiag_create: dof %zu has invP_id %d outside [0, NEQ)", k, invP[k]);
         id[k] = type[k] == 0 ? NEQ : invP[k];
     }
+    // node of every unknown; nfree < 0 when an unknown belongs to two dofs
+    std::vector<int> node_of(static_cast<size_t>(NEQ), -1);
+    int nfree = 0;
+    for (int v = 0; v < nnodes && nfree >= 0; ++v) {
+        bool any = false;
+        for (int j = 0; j < ndof; ++j) {
+            const int q = id[static_cast<size_t>(v) * ndof + j];
+            if (q == NEQ) continue;
+            any = true;
+            if (node_of[q] >= 0) {
+                nfree = -1;
+                break;
+            }
+            node_of[q] = v;
+        }
+        if (any && nfree >= 0) ++nfree;
+    }
     std::vector<std::pair<int, int>> pairs;
     pairs.reserve(static_cast<size_t>(nel) * 3);
     for (int e = 0; e < nel; ++e)
@@ -281,7 +310,9 @@ extern "C" int femgpu_blockdiag_create(femgpu_ctx *ctx, int nnodes, int nel, int
     B->ndof = ndof;
     B->NEQ = NEQ;
     hipStream_t s = ctx->stream;
+    B->nfree = nfree;
     int rc = B->id.upload(id.data(), id.size(), s);
+    if (!rc) rc = B->node_of.upload(node_of.data(), node_of.size(), s);
     if (!rc) rc = B->ien.upload(ien, static_cast<size_t>(nel) * 3, s);
     if (!rc) rc = B->inc_ptr.upload(ptr.data(), ptr.size(), s);
     if (!rc) rc = B->inc_src.upload(src.data(), src.size(), s);

@@ -194,6 +194,7 @@ struct femgpu_ctx {
     // Solver workspaces (grown on demand, kept across calls).
     fg::DevBuf<double> gm_basis, gm_small, gm_w, gm_r;
     fg::DevBuf<int> bt_rowoff, bt_sys;        // batched solver: system row offsets, system of each row
+    fg::DevBuf<int> node_match;               // EBE groups' nodes in the block-diagonal preconditioner
     fg::DevBuf<double> cgs_partials;          // classical Gram-Schmidt: per-block partial dot products
     fg::DevBuf<femgpu_batch_info> wg_info;    // persistent batched solver: per-system results
     fg::DevBuf<double> bt_scal;               // batched solver: per-system norms and scales
@@ -417,7 +418,13 @@ int launch_to_f32(femgpu_ctx *ctx, const double *src, float *dst, size_t n);
 int launch_ebemv(femgpu_ctx *ctx, const femgpu_ebe *E, const double *P, double *Q, const int *skip = nullptr);
 // xs, xout: the operand P * *xs, stored to xout on the way (where ebe_scales(E): every unknown in an element)
 int launch_ebemv32(femgpu_ctx *ctx, const femgpu_ebe *E, const float *P, float *Q, const int *skip = nullptr,
-                   const double *xs = nullptr, float *xout = nullptr);
+                   const double *xs = nullptr, float *xout = nullptr, const struct ArnoldiTail *tail = nullptr);
+const float *blockdiag_inv32(const femgpu_blockdiag *B);
+bool blockdiag_nodes(const femgpu_blockdiag *B, int ndof, int NEQ, const int **node_of, const int **id, int *nfree);
+// node of B of every group of E (in ctx scratch), on the stream; {groups with a node, groups without} arrive in
+// ctx->h_pinned[kPinMatch]; *want: the first count when B's nodes with unknowns and E's groups agree
+constexpr int kPinMatch = 8;
+int ebe_match_nodes(femgpu_ctx *ctx, const femgpu_ebe *E, const femgpu_blockdiag *B, const int **gnode, int *want);
 bool ebe_scales(const femgpu_ebe *E);
 int launch_blockdiag_apply32(femgpu_ctx *ctx, const femgpu_blockdiag *B, const float *p, float *z, const int *skip);
 

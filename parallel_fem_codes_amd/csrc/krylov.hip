@@ -16,89 +16,9 @@
 
 #include "common.h"
 #include "device_util.h"
+#include "arnoldi.h"
 
 namespace fg {
-
-struct GDev {
-    double *H;        // (ld x ld) Hessenberg, H[r*ld + c]
-    double *c, *s, *e, *y, *hnorm, *invh;   // ld each
-    double *scal;     // [0] eps  [1] rho  [2] normb
-    int *flags;       // [0] cycle done  [1] steps in cycle
-    int ld, kmax;
-    double *partials;
-    int *h_status;    // host-mapped: per step {done} ; h_rho host-mapped rho per step
-    double *h_rho;
-    int prec_mode;    // FP32 preconditioner (host side only): 0 exact sweeps, k > 0 Jacobi iterations
-    int cgs;          // FP32 inner Arnoldi with classical Gram-Schmidt (host side only)
-    int graphs;       // FP32 inner Arnoldi steps replayed from captured hipGraphs (host side only)
-};
-
-__device__ __forceinline__ double &Hat(const GDev &G, int r, int c) { return G.H[r * G.ld + c]; }
-
-// Host-mapped doubles (G.h_rho): [0, kmax) the residual estimate after each step, kMapE0 / kMapEps
-// the cycle's starting residual and its target, 248..255 norms of the mixed solver.
-constexpr int kMapE0 = 246, kMapEps = 247;
-
-constexpr int kMaxBasis = 150;   // largest GMRES basis (make_gdev)
-
-// Givens update of column i and the convergence test (pgmres.c:118-159), with h_{i+1,i} = hn.
-// Called by every thread of the block: the block stages the column, the earlier rotations and
-// e[i] in LDS with loads issued together, then one thread applies the rotations -- the operations
-// of a serial update in the same order -- and stores the results.
-__device__ void givens_column(const GDev &G, int i, double hn)
-{
-#pragma clang fp contract(off)
-    __shared__ double col[kMaxBasis + 1], cs[kMaxBasis], sn[kMaxBasis], ei_s;
-    for (int k = threadIdx.x; k <= i; k += blockDim.x) col[k] = Hat(G, k, i);
-    for (int k = threadIdx.x; k < i; k += blockDim.x) {
-        cs[k] = G.c[k];
-        sn[k] = G.s[k];
-    }
-    if (threadIdx.x == 0) ei_s = G.e[i];
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    // the entry that the rotations carry along stays in a register and eight rotations' operands are read
-    // ahead: an LDS round trip per rotation would be most of this kernel's time
-    double run = col[0];
-    int j0 = 0;
-    for (; j0 + 8 <= i; j0 += 8) {
-        double cj[8], sj[8], hj[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            cj[u] = cs[j0 + u];
-            sj[u] = sn[j0 + u];
-            hj[u] = col[j0 + u + 1];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            Hat(G, j0 + u, i) = cj[u] * run + sj[u] * hj[u];
-            run = -sj[u] * run + cj[u] * hj[u];
-        }
-    }
-    for (; j0 < i; ++j0) {
-        const double hj = col[j0 + 1];
-        Hat(G, j0, i) = cs[j0] * run + sn[j0] * hj;
-        run = -sn[j0] * run + cs[j0] * hj;
-    }
-    const double a = run, b = hn;
-    const double r = sqrt(a * a + b * b);
-    const double ci = a / r, si = b / r;
-    G.c[i] = ci;
-    G.s[i] = si;
-    Hat(G, i, i) = r;
-    Hat(G, i + 1, i) = 0.0;
-    const double ei = ei_s;
-    G.e[i + 1] = -si * ei;
-    G.e[i] = ci * ei;
-    const double rho = fabs(G.e[i + 1]);
-    const int steps = i + 1;
-    const int done = !(rho > G.scal[0]) || (steps >= G.kmax - 1);
-    G.scal[1] = rho;
-    G.flags[1] = steps;
-    G.flags[0] = done;
-    __hip_atomic_store(&G.h_rho[i], rho, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(&G.h_status[i], done ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 
 // 16-byte vectors of the basis type (the basis and work vectors are 256-byte aligned).
 template <typename T>
@@ -127,27 +47,6 @@ struct Vec16<double> {
 // Grid reductions leave per-block partials (plain stores; the kernel boundary makes them visible)
 // that a later kernel sums in a fixed order, so results do not depend on block timing and need no
 // atomics or device-scope fences.
-
-// Sum of the nb partials in a fixed order by one block of 256 threads (valid in every thread).
-// Each thread adds its entries b, b + 256, ... in order, with four loads issued together.
-__device__ __forceinline__ double sum_partials(const double *partials, int nb, double *red)
-{
-    double v = 0;
-    int b = threadIdx.x;
-    for (; b + 3 * 256 < nb; b += 4 * 256) {
-        const double a0 = partials[b], a1 = partials[b + 256], a2 = partials[b + 512], a3 = partials[b + 768];
-        v += a0;
-        v += a1;
-        v += a2;
-        v += a3;
-    }
-    for (; b < nb; b += 256) v += partials[b];
-    v = block_sum<256>(v, red);
-    __shared__ double total;
-    if (threadIdx.x == 0) total = v;
-    __syncthreads();
-    return total;
-}
 
 constexpr int kMgsVec = 4;
 
@@ -769,13 +668,15 @@ static int prec32_dot_blocks(const femgpu_system *S, int mode)
     return S->csr && S->ilu && mode > 0 ? jacobi_dot_blocks(S->ilu) : 0;
 }
 
+struct NodeMatch;
+
 template <typename T>
 static int run_cycle(femgpu_ctx *ctx, const femgpu_system *S, GDev &G, int n, T *V, size_t ldv, T *wA, T *wB,
-                     int kmax, int *steps_out);
+                     int kmax, int *steps_out, NodeMatch *match = nullptr);
 
 template <>
 int run_cycle<double>(femgpu_ctx *ctx, const femgpu_system *S, GDev &G, int n, double *V, size_t ldv, double *wA,
-                      double *wB, int kmax, int *steps_out)
+                      double *wB, int kmax, int *steps_out, NodeMatch *)
 {
     hipEvent_t ev[2];
     FG_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
@@ -817,7 +718,8 @@ __global__ void k_scale_copy(int n, const T *__restrict__ x, const double *__res
 // sweeps; EBE: the gathered element product with the scaling
 // fused, then the nodal block-diagonal blocks.
 static int op_prec32(femgpu_ctx *ctx, const femgpu_system *S, int prec_mode, const float *x, const double *xs,
-                     float *xout, float *w, const int *skip, const float *dv = nullptr, double *dpart = nullptr)
+                     float *xout, float *w, const int *skip, const float *dv = nullptr, double *dpart = nullptr,
+                     const ArnoldiTail *tail = nullptr)
 {
     if (S->csr) {
         FG_TRY(launch_spmv32(ctx, S->csr, x, xs, xout, w, skip));
@@ -828,28 +730,32 @@ static int op_prec32(femgpu_ctx *ctx, const femgpu_system *S, int prec_mode, con
         FG_HIP(hipGetLastError());
         FG_TRY(launch_ebemv32(ctx, S->ebe, xout, w, skip));
     } else {
-        FG_TRY(launch_ebemv32(ctx, S->ebe, x, w, skip, xs, xout));
+        FG_TRY(launch_ebemv32(ctx, S->ebe, x, w, skip, xs, xout, tail));
+        if (tail && tail->gnode) return FEMGPU_OK;
     }
     return launch_blockdiag_apply32(ctx, S->bdiag, w, w, skip);
 }
 
+static int cgs_blocks(int n) { return std::max(1, std::min(kCgsBlocks, (n / 4 + 255) / 256)); }
+
 // The launches of Arnoldi step i of the FP32 inner solver: w_next = M^-1 A (v_i), v_i = w_cur / h
 // stored on the way, then the orthogonalization and the Givens update of column i. With the Jacobi
 // preconditioner and MGS, the last Jacobi iteration also forms the partials of <V[0], w_next>
-// (the first MGS pass), in ctx->jac_partials.
+// (the first MGS pass), in ctx->jac_partials. tail (EBE operators): the parts of the neighbouring kernels that
+// the product takes over; deferred: the Givens update is left to the next product.
 static int step_kernels32(femgpu_ctx *ctx, const femgpu_system *S, const GDev &G, int n, int i, float *wc,
-                          float *wn, float *V, size_t ldv)
+                          float *wn, float *V, size_t ldv, const ArnoldiTail *tail = nullptr, bool deferred = false)
 {
     const int nf = G.cgs ? 0 : prec32_dot_blocks(S, G.prec_mode);
     FG_TRY(op_prec32(ctx, S, G.prec_mode, wc, G.invh + i, V + i * ldv, wn, G.flags, nf ? V : nullptr,
-                     nf ? ctx->jac_partials.p : nullptr));
+                     nf ? ctx->jac_partials.p : nullptr, tail));
     if (G.cgs) {
-        const int nb = std::max(1, std::min(kCgsBlocks, (n / 4 + 255) / 256));
+        const int nb = cgs_blocks(n);
         const bool in_update = nb <= kCgsSumMax;
         k_cgs_dots<<<dim3(nb, i / kCgsChunk + 1), 256, 0, ctx->stream>>>(G, n, i, wn, V, ldv, ctx->cgs_partials.p);
         if (!in_update) k_cgs_reduce<<<i + 1, 256, 0, ctx->stream>>>(G, nb, i, ctx->cgs_partials.p);
         k_cgs_update<<<nb, 256, 0, ctx->stream>>>(G, n, i, wn, V, ldv, ctx->cgs_partials.p, in_update ? nb : 0);
-        k_cgs_finish<<<1, 256, 0, ctx->stream>>>(G, nb, i, ctx->cgs_partials.p);
+        if (!deferred) k_cgs_finish<<<1, 256, 0, ctx->stream>>>(G, nb, i, ctx->cgs_partials.p);
     } else {
         mgs_step<float>(ctx, G, n, i, wn, V, ldv, nf, ctx->jac_partials.p);
     }
@@ -913,42 +819,91 @@ static int graph_step32(femgpu_ctx *ctx, const femgpu_system *S, const GDev &G, 
     return FEMGPU_OK;
 }
 
+// The nodal preconditioner inside the EBE product: ebe_match_nodes finds the node of every group of the operator
+// at the start of a solve and leaves {groups with a node, groups without} in pinned memory; once a later
+// event of the stream has been waited for, the product applies the blocks if every group has its node and
+// every node its group.
+struct NodeMatch {
+    const int *gnode = nullptr;
+    const volatile int *found = nullptr;
+    int want = 0;
+    bool known = false;
+    const int *use() const { return known && gnode && found[0] == want && found[1] == 0 ? gnode : nullptr; }
+};
+
 // The host keeps one step in flight ahead of the one it checks: step i is enqueued before step
 // i - 1's done word is read, so the device never waits for the host between steps, and the step
 // after the converged one drains (its kernels exit on the done flag). When the last contraction of
 // the residual estimate predicts that the step in flight reaches the target (rho_{i-2}^2 / rho_{i-3}
 // <= eps), the host waits for that step before enqueuing the next: the drained step's launches,
 // about 20 us, are saved, and a wrong prediction costs one host round trip.
+// With an EBE operator and classical Gram-Schmidt over few enough blocks the end of step i - 1 runs inside the product
+// of step i (a launch of 4.7 us and its gap less per step; 8.4 -> 6.6 ms for a step of 245 inner iterations of
+// 80 000 unknowns, with the nodal blocks in the product too): a step's done word then comes one step later,
+// and a step that has to be known at once (predicted to be the last, or the cycle's last) is ended by a
+// launch of its own.
 template <>
 int run_cycle<float>(femgpu_ctx *ctx, const femgpu_system *S, GDev &G, int n, float *V, size_t ldv, float *wA,
-                     float *wB, int kmax, int *steps_out)
+                     float *wB, int kmax, int *steps_out, NodeMatch *match)
 {
     hipEvent_t ev[2];
     FG_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
     FG_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
     const volatile double *hrho = reinterpret_cast<const volatile double *>(ctx->h_status + 256);
+    const bool scales = !S->csr && ebe_scales(S->ebe);
+    const bool deferred = scales && G.cgs && cgs_blocks(n) <= kCgsSumMax;
     float *wc = wA, *wn = wB;
-    int rc = FEMGPU_OK, steps = 0, waited = -1;
+    // known: the last step whose done word the host has seen; ended: the last one with its Givens update enqueued
+    int rc = FEMGPU_OK, steps = 0, known = -1, ended = -1;
+    bool done = false;
+    const auto end_step = [&](int i) {
+        k_cgs_finish<<<1, 256, 0, ctx->stream>>>(G, cgs_blocks(n), i, ctx->cgs_partials.p);
+        ended = i;
+        return hipGetLastError() == hipSuccess && hipEventRecord(ev[i & 1], ctx->stream) == hipSuccess;
+    };
+    const auto wait = [&](int i, int tells) {   // for the event of step i, which tells that of step `tells`
+        if (hipEventSynchronize(ev[i & 1]) != hipSuccess) return false;
+        if (match) match->known = true;
+        for (; known < tells; ++known) done = done || ctx->h_status[known + 1];
+        return true;
+    };
     for (int i = 0; i < kmax - 1; ++i) {
-        if (i >= 2) {   // steps up to i - 2 are known (not done), step i - 1 is in flight
-            const double r1 = hrho[i - 2], r0 = i >= 3 ? hrho[i - 3] : hrho[kMapE0], eps = hrho[kMapEps];
-            if (r0 > 0.0 && r1 > 0.0 && r1 * (r1 / r0) <= eps) {
-                if (hipEventSynchronize(ev[(i - 1) & 1]) != hipSuccess) { rc = FEMGPU_ERR_HIP; break; }
-                waited = i - 1;
-                if (ctx->h_status[i - 1]) break;
+        if (known >= 0 && known < i - 1) {   // steps known + 1 .. i - 1 are in flight
+            const double r1 = hrho[known], r0 = known >= 1 ? hrho[known - 1] : hrho[kMapE0], eps = hrho[kMapEps];
+            const double f = r1 / r0;
+            if (r0 > 0.0 && r1 > 0.0 && r1 * (i - 1 - known == 1 ? f : f * f) <= eps) {
+                if (ended < i - 1 && !end_step(i - 1)) { rc = FEMGPU_ERR_HIP; break; }
+                if (!wait(i - 1, i - 1)) { rc = FEMGPU_ERR_HIP; break; }
+                if (done) break;
             }
         }
         ctx->h_status[i] = 0;
-        rc = G.graphs ? graph_step32(ctx, S, G, n, i, wA, wB, V, ldv) : step_kernels32(ctx, S, G, n, i, wc, wn, V, ldv);
+        if (G.graphs) {
+            rc = graph_step32(ctx, S, G, n, i, wA, wB, V, ldv);
+        } else {
+            ArnoldiTail tail;
+            tail.G = G;
+            tail.gnode = match ? match->use() : nullptr;
+            tail.inv = tail.gnode ? blockdiag_inv32(S->bdiag) : nullptr;
+            if (ended < i - 1) {
+                tail.part = ctx->cgs_partials.p + static_cast<size_t>(i) * kCgsBlocks;
+                tail.nb = cgs_blocks(n);
+                tail.col = i - 1;
+            }
+            rc = step_kernels32(ctx, S, G, n, i, wc, wn, V, ldv, scales && (tail.nb || tail.gnode) ? &tail : nullptr,
+                                deferred);
+        }
         if (rc) break;
         if (hipEventRecord(ev[i & 1], ctx->stream) != hipSuccess) { rc = FEMGPU_ERR_HIP; break; }
         std::swap(wc, wn);
         steps = i + 1;
-        if (i >= 1 && waited != i - 1) {
-            if (hipEventSynchronize(ev[(i - 1) & 1]) != hipSuccess) { rc = FEMGPU_ERR_HIP; break; }
-            if (ctx->h_status[i - 1]) break;
+        ended = deferred ? i - 1 : i;
+        if (i >= 1 && known < i - 1) {
+            if (!wait(i - 1, deferred ? i - 2 : i - 1)) { rc = FEMGPU_ERR_HIP; break; }
+            if (done) break;
         }
     }
+    if (!rc && !done && steps > 0 && ended < steps - 1 && !end_step(steps - 1)) rc = FEMGPU_ERR_HIP;
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
     *steps_out = steps;
@@ -1169,6 +1124,11 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
     // ||F|| is not waited for: the first refinement reads it on the device, and the host reads it
     // from the mapped slot after the first cycle's synchronisation (the cases above and ||F|| = 0 or
     // non-finite, which the first cycle then turns into NaN work, end with X = 0)
+    NodeMatch match;
+    if (!csr && ebe_scales(S->ebe)) {
+        FG_TRY(ebe_match_nodes(ctx, S->ebe, S->bdiag, &match.gnode, &match.want));
+        match.found = reinterpret_cast<const volatile int *>(ctx->h_pinned + kPinMatch);
+    }
     volatile double *hmap_F = nullptr;
     FG_TRY(norm64_async(ctx, n, d_F, d_fn, 0, hmap_F));
     struct Event {
@@ -1177,8 +1137,17 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
     } evF;
     FG_HIP(hipEventCreateWithFlags(&evF.e, hipEventDisableTiming));
     FG_HIP(hipEventRecord(evF.e, ctx->stream));
-    int refinements = 0, inner_total = 0;
+    int refinements = 0, inner_total = 0, last_steps = 0;
     double rn = 0.0;
+    // the device's step count of the last cycle: the first step that reported it done
+    const auto count_steps = [&]() {
+        for (int i = 0; i < last_steps; ++i)
+            if (ctx->h_status[i]) {
+                last_steps = i + 1;
+                break;
+            }
+        inner_total += last_steps;
+    };
     for (;;) {
         // outer FP64 residual r = F - A X; on the first pass X = 0 (not yet written): r = F, ||r|| = ||F||
         const double *rr = d_F, *d_rcur = d_fn;
@@ -1198,6 +1167,7 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
                 }
                 FG_TRY(norm64_sync(ctx, n, r, d_rn, 1, rn));
             }
+            count_steps();   // every step has reported by now
             rr = r;
             d_rcur = d_rn;
         }
@@ -1218,7 +1188,7 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
             cycle_start<float>(ctx, G, n, wA, nullptr, 0, 1, opt->inner_tol, nfz, ctx->jac_partials.p);
             FG_HIP(hipGetLastError());
             int steps = 0;
-            FG_TRY(run_cycle<float>(ctx, S, G, n, V, ldv, wA, wB, kin, &steps));
+            FG_TRY(run_cycle<float>(ctx, S, G, n, V, ldv, wA, wB, kin, &steps, csr ? nullptr : &match));
             if (refinements == 0) {   // ||F|| (run_cycle has normally waited for a later step already)
                 FG_HIP(hipEventSynchronize(evF.e));
                 normF = *hmap_F;
@@ -1233,14 +1203,7 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
                 FG_HIP(hipStreamSynchronize(ctx->stream));
                 FG_TRY(check_device_error(ctx));
             }
-            // the device's step count: the first step that reported the cycle done
-            int dsteps = steps;
-            for (int i = 0; i < steps; ++i)
-                if (ctx->h_status[i]) {
-                    dsteps = i + 1;
-                    break;
-                }
-            inner_total += dsteps;
+            last_steps = steps;
         }
         ++refinements;
     }
