@@ -8,7 +8,8 @@
 // its vertex pair, evaluated in the reference's operation order with contraction off (for the
 // symmetric terms the reference evaluates the (min, max) pair and reuses it, and so does this
 // kernel), so element matrices, residuals, CSR values and right-hand sides are bit-identical.
-// Global accumulation is a gather in element order, as for the transport assembly.
+// Global accumulation is a sum in element order, as for the transport assembly: inside the fused
+// kernel where the mesh has its plan and CSR values are wanted, through slot lists otherwise.
 #include <algorithm>
 #include <cstdint>
 #include <vector>

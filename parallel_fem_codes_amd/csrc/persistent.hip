@@ -6,6 +6,11 @@
 // alone and in any batch. For the small systems of the serving loop, where one launch per kernel
 // step would cost more than the step's memory traffic.
 //
+// Two forms. A system whose vectors fit in the workgroup's LDS runs there, its matrix and factors in
+// registers where the rows per thread allow it (a step then touches memory for the FP64 residual only);
+// larger ones keep the vectors in global memory. femgpu_gmres_mixed and femgpu_gmres_mixed_batched take
+// the first form for small systems, where a chain of launches of 2 to 4 us each was the solve's time.
+//
 // Synchronisation is workgroup-local only (__syncthreads), every loop is bounded (max_refinements
 // outer steps, m - 1 inner steps, the Jacobi iteration count), and every exit decision is taken
 // from values that all threads of the workgroup hold identically, so every wave reaches the end.

@@ -456,7 +456,8 @@ static int stream_launch(femgpu_ctx *ctx, const StreamSweep &P, const T *val, co
     if (P.K == 4) stream_launch_k<T, UPPER, 4, 8, kStreamThreads>(ctx, P, val, dinv, b, x, skip);
     else if (P.K == 8) stream_launch_k<T, UPPER, 8, 4, kStreamThreads>(ctx, P, val, dinv, b, x, skip);
     // 16-entry rows: 4 steps of lookahead fit the registers in FP32 (6.6 against 7.4 ms per apply on
-    // the 513 x 513 cavity), 2 in FP64
+    // the 513 x 513 cavity), 2 in FP64; a workgroup of at most 256 threads has twice the registers and takes twice
+    // that (81 x 81 cavity, FP64 apply 1.45 -> 0.45 ms with the narrower workgroup)
     else if (P.threads > 256) stream_launch_k<T, UPPER, 16, 2 * F, kStreamThreads>(ctx, P, val, dinv, b, x, skip);
     else stream_launch_k<T, UPPER, 16, 4 * F, 256>(ctx, P, val, dinv, b, x, skip);
     FG_HIP(hipGetLastError());
