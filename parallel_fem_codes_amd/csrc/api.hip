@@ -205,6 +205,15 @@ static int csr_setup(femgpu_csr *A, int n, int nnz, const int *IA, const int *JA
     A->nnz = nnz;
     A->hIA.assign(IA, IA + n + 1);
     A->hJA.assign(JA, JA + nnz);
+    A->hsplit.resize(static_cast<size_t>(n) + 1);   // rows are sorted and hold their diagonal
+    for (int r = 0, reach = -1; r <= n; ++r) {
+        A->hsplit[r] = reach < r;
+        if (r < n) reach = std::max(reach, JA[IA[r + 1] - 1]);
+    }
+    for (int r = n, low = n; r >= 0; --r) {
+        A->hsplit[r] = A->hsplit[r] && low >= r;
+        if (r > 0) low = std::min(low, JA[IA[r - 1]]);
+    }
     hipStream_t s = ctx->stream;
     int rc = A->IA.upload(IA, n + 1, s);
     if (!rc) rc = A->JA.upload(JA, nnz, s);

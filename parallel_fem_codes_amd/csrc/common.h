@@ -216,6 +216,7 @@ struct femgpu_csr {
     unsigned long long serial = 0;  // unique per matrix created in the process
     int n = 0, nnz = 0;
     std::vector<int> hIA, hJA;
+    std::vector<bool> hsplit;       // r in [0, n]: no entry couples rows before r with rows from r on
     fg::DevBuf<int> IA, JA, diag;   // diag[i] = position of the diagonal entry of row i
     fg::DevBuf<double> AA;          // nnz+1 (dummy slot nnz)
     fg::DevBuf<float> AA32;         // FP32 CSR values, kept only when sell_ok && par_ok is false
@@ -443,6 +444,7 @@ void csr_map(int nkeys, const std::vector<std::pair<int, int>> &pairs, std::vect
              std::vector<int> &dst);
 int check_device_error(femgpu_ctx *ctx);
 int wg_threads_for(long long rows, int nsys);   // persistent batched solver: default workgroup size
+bool uncoupled_systems(const femgpu_csr *A, int nsys, const int *row_off);
 bool wg_preferred(const femgpu_ctx *ctx, const femgpu_system *S, const femgpu_mixed_opts *opt, int nsys, int widest);
 int wg_solve_one(femgpu_ctx *ctx, femgpu_csr *A, const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
                  femgpu_batch_info *info);

@@ -1236,10 +1236,10 @@ extern "C" int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *
     FG_CHECK(opt->factor_sweeps > 0 || S->ilu->factored, FEMGPU_ERR_STATE,
              "femgpu_gmres_mixed_batched: ILU(0) not factored");
     const int kin = opt->inner_kmax;
-    // small systems: a workgroup each (its own Krylov space), modified Gram-Schmidt
+    // small systems that share no entry: a workgroup each (its own Krylov space), modified Gram-Schmidt
     int widest = 0;
     for (int s = 0; s < nsys; ++s) widest = std::max(widest, row_off[s + 1] - row_off[s]);
-    if (wg_preferred(ctx, S, opt, nsys, widest))
+    if (wg_preferred(ctx, S, opt, nsys, widest) && uncoupled_systems(S->csr, nsys, row_off))
         return wg_solve_batch(ctx, S->csr, nsys, row_off, opt, tol, wg_threads_for(widest, 1), d_F, d_X, info);
     memset(info, 0, sizeof(*info) * static_cast<size_t>(nsys));
     GDev G{};

@@ -725,6 +725,15 @@ bool wg_preferred(const femgpu_ctx *ctx, const femgpu_system *S, const femgpu_mi
            opt->max_refinements >= 1 && nsys <= ctx->num_cus && widest <= (nsys == 1 ? 4096 : 3072);
 }
 
+// The workgroup of a system reads no other system's rows (its vectors in LDS hold its own only): whether no
+// entry of A lies between two systems.
+bool uncoupled_systems(const femgpu_csr *A, int nsys, const int *row_off)
+{
+    for (int s = 0; s <= nsys; ++s)
+        if (!A->hsplit[row_off[s]]) return false;
+    return true;
+}
+
 int wg_solve_one(femgpu_ctx *ctx, femgpu_csr *A, const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
                  femgpu_batch_info *info)
 {
@@ -775,6 +784,8 @@ extern "C" int femgpu_gmres_mixed_wg(femgpu_ctx *ctx, const femgpu_system *S, in
     FG_CHECK(A->sell_ok && A->par_ok, FEMGPU_ERR_ARG,
              "femgpu_gmres_mixed_wg: the matrix has no sliced-ELL factor layout (rows wider than 16 entries or "
              "created without the mixed-precision plans)");
+    FG_CHECK(uncoupled_systems(A, nsys, row_off), FEMGPU_ERR_ARG,
+             "femgpu_gmres_mixed_wg: an entry of the matrix couples two of the systems");
     if (threads == 0) threads = wg_threads_for(n, nsys);
     return wg_solve_batch(ctx, A, nsys, row_off, opt, tol, threads, d_F, d_X, info);
 }

@@ -94,3 +94,32 @@ def test_batch(sizes):
             continue
         assert residual(*s, xk) <= 1.01e-9
         assert abs(residual(*s, xk) - i.true_rel_residual) <= 1e-3 * i.true_rel_residual + 1e-15
+
+
+@pytest.mark.parametrize("at", [0, 1])
+def test_batch_of_coupled_rows(at):
+    """An entry between two "systems" (in the rows before or after their boundary): their rows are solved
+    together, as one matrix, and the solver of one workgroup per system refuses them."""
+    import torch
+    n = [300, 200]
+    a, b = system(n[0], 9, 7), system(n[1], 9, 8)
+    IA, JA, off, _ = fem.concat_csr([a[:2], b[:2]])
+    AA, F = np.concatenate([a[2], b[2]]), np.concatenate([a[3], b[3]])
+    r, c = [(n[0] - 2, n[0] + 5), (n[0] + 3, 20)][at]
+    p = IA[r] + int(np.searchsorted(JA[IA[r]:IA[r + 1]], c))
+    JA, AA = np.insert(JA, p, c), np.insert(AA, p, 0.5)
+    IA[r + 1:] += 1
+    dev = fem.Device(0)
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(AA)
+    Fd = torch.from_numpy(F).cuda()
+    X = torch.full((sum(n),), float("nan"), dtype=torch.float64, device="cuda")
+    infos = fem.gmres_mixed_batched(dev, A, off, Fd, X, tol=1e-9)
+    res = np.add.reduceat(AA * X.cpu().numpy()[JA], IA[:-1]) - F
+    for k, i in enumerate(infos):
+        rows = slice(off[k], off[k + 1])
+        assert i.status == 0 and np.linalg.norm(res[rows]) <= 1.01e-9 * np.linalg.norm(F[rows])
+    with pytest.raises(Exception, match="couples two"):
+        fem.gmres_mixed_wg(dev, A, off, Fd, X, tol=1e-9)
+    infos = fem.gmres_mixed_wg(dev, A, [0, 0, sum(n)], Fd, X, tol=1e-9)   # one system and an empty one
+    assert all(i.status == 0 for i in infos)
