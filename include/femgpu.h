@@ -314,7 +314,9 @@ typedef struct {
                               orthogonalization) is captured once into a hipGraph and replayed;
                               the graphs are kept by the context and re-captured when the matrix
                               or the workspace changes. Same kernels, same results. */
-    int pad;
+    int multi_launch;      /* 1: small systems too take the solvers of many launches over the whole
+                              GPU (a batch then shares one Krylov space) instead of the launch of
+                              one workgroup per system; else the size decides */
 } femgpu_mixed_opts;
 
 /* Mixed precision: FP64 iterative refinement (residual F - A x, update x += d, Givens and least
@@ -327,7 +329,7 @@ typedef struct {
  * passes (||F|| = 0 or tol >= 1: status 0), with max_refinements = 0 (status 1 unless ||F|| = 0)
  * and for a non-finite F (status 1). CSR systems of at most 4096 rows with factor_sweeps >= 1,
  * sweep_mode >= 1 and modified Gram-Schmidt run as one workgroup's launch (femgpu_gmres_mixed_wg's
- * kernel, graphs or not). No reference counterpart. */
+ * kernel, graphs or not) unless multi_launch is 1. No reference counterpart. */
 int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *sys, const femgpu_mixed_opts *opt,
                        double tol, const double *d_F, double *d_X, femgpu_solve_info *info);
 
@@ -348,9 +350,9 @@ typedef struct {
  * ||F_s - A_s x_s|| <= tol ||F_s||; active systems enter each inner FP32 GMRES cycle with their
  * residual scaled to unit norm, and the cycle's correction is scaled back per system. One launch
  * sequence serves the whole batch. Batches of systems of at most 3072 rows (no more systems than the
- * GPU has compute units, factor_sweeps >= 1, sweep_mode >= 1) take femgpu_gmres_mixed_wg's kernel: a
- * workgroup and a Krylov space (modified Gram-Schmidt) per system. info: nsys entries. No reference
- * counterpart. */
+ * GPU has compute units, factor_sweeps >= 1, sweep_mode >= 1) take femgpu_gmres_mixed_wg's kernel
+ * unless multi_launch is 1: a workgroup and a Krylov space per system, whose Gram-Schmidt is the
+ * modified one whatever orthogonalization says. info: nsys entries. No reference counterpart. */
 int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *sys, int nsys, const int *row_off,
                                const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
                                femgpu_batch_info *info);
@@ -536,7 +538,7 @@ typedef struct {
     int max_batch;         /* requests per batch; 0: tuned online among 4, 8, 16, 32, 64 */
     int kmax;              /* inner GMRES basis size */
     int small_solver;      /* batches of small requests: 0 the block-diagonal shared-Krylov solver
-                              (femgpu_gmres_mixed_batched), 1 the persistent launch with a workgroup
+                              (femgpu_gmres_mixed_batched with multi_launch), 1 the persistent launch with a workgroup
                               per system (femgpu_gmres_mixed_wg) when every system of the batch has
                               at most 3072 rows, else 0, 2 always the persistent launch; the
                               persistent launch needs kmax <= 64 */

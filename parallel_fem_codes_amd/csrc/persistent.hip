@@ -720,7 +720,7 @@ static int wg_enqueue(femgpu_ctx *ctx, femgpu_csr *A, int nsys, const int *row_o
 bool wg_preferred(const femgpu_ctx *ctx, const femgpu_system *S, const femgpu_mixed_opts *opt, int nsys, int widest)
 {
     const femgpu_csr *A = S->csr;
-    return A && S->ilu == A && A->sell_ok && A->par_ok && A->n > 0 && opt->factor_sweeps >= 1 && opt->factor_sweeps <= 16 &&
+    return opt->multi_launch != 1 && A && S->ilu == A && A->sell_ok && A->par_ok && A->n > 0 && opt->factor_sweeps >= 1 && opt->factor_sweeps <= 16 &&
            opt->sweep_mode >= 1 && opt->sweep_mode <= 16 && opt->inner_kmax >= 2 && opt->inner_kmax <= kWgMaxBasis &&
            opt->max_refinements >= 1 && nsys <= ctx->num_cus && widest <= (nsys == 1 ? 4096 : 3072);
 }

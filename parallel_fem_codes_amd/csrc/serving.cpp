@@ -13,8 +13,8 @@
 //               the GPU start as soon as an executor and memory free up, and the executors' work
 //               overlaps on the device
 //   wait     -> the caller collects the nodal solution and the timings
-// Batches of small requests run through the block-diagonal solver, whose kernels spread the batch
-// over the whole GPU, or (small_solver 1 or 2) as one persistent launch with a workgroup per system
+// Batches of small requests run through the block-diagonal solver (femgpu_gmres_mixed_batched with
+// multi_launch), whose kernels spread the batch over the whole GPU, or (small_solver 1 or 2) as one persistent launch with a workgroup per system
 // (femgpu_gmres_mixed_wg: each request's answer is the same alone and in any batch). A solve alone
 // is faster on one compute unit below about 3000 rows (measured: 2x at 300-1000 rows, equal near
 // 3000, 3-8x slower at 10000-20000), so mode 1 takes the persistent launch only when every system
@@ -353,6 +353,7 @@ void run_unit(femgpu_server *S, Executor &E, std::vector<Req> &unit, long long b
         mo.inner_kmax = S->o.kmax;
         if (rc == FEMGPU_OK) {
             const bool wg = threads >= 0 && A->sell_ok && A->par_ok;
+            mo.multi_launch = 1;   // read by the batched entry point only: the shared Krylov space at any size
             used_threads = wg ? (threads > 0 ? threads : fg::wg_threads_for(N, K)) : 0;
             const int st = wg ? femgpu_gmres_mixed_wg(ctx, &sys, K, row_off.data(), &mo, S->o.tol, used_threads, dF, dX,
                                                       binfo.data())

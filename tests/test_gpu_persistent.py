@@ -54,7 +54,7 @@ def systems(dev, torch_cuda):
     return [assemble(dev, torch_cuda, r) for r in reqs]
 
 
-def batch_solve(dev, torch, syss, threads=256, solver="wg"):
+def batch_solve(dev, torch, syss, threads=256, solver="wg", **kw):
     IA, JA, row_off, nnz_off = fem.concat_csr([(s["IA"], s["JA"]) for s in syss])
     A = fem.CsrMatrix(dev, IA, JA)
     A.set_values(np.concatenate([s["AA"] for s in syss]))
@@ -64,7 +64,7 @@ def batch_solve(dev, torch, syss, threads=256, solver="wg"):
     if solver == "wg":
         infos = fem.gmres_mixed_wg(dev, A, row_off, F, X, tol=1e-8, inner_kmax=30, threads=threads)
     else:
-        infos = fem.gmres_mixed_batched(dev, A, row_off, F, X, tol=1e-8, inner_kmax=30)
+        infos = fem.gmres_mixed_batched(dev, A, row_off, F, X, tol=1e-8, inner_kmax=30, **kw)
     x = X.cpu().numpy()
     return [x[row_off[k]:row_off[k + 1]] for k in range(len(syss))], infos
 
@@ -111,12 +111,22 @@ def test_wg_workgroup_sizes(dev, torch_cuda, systems, threads):
     assert max(host_rel_residual(s, x) for s, x in zip(systems, xs)) <= 1.01e-8
 
 
-def test_wg_matches_shared_krylov_batched_solver(dev, torch_cuda, systems):
-    a, ia = batch_solve(dev, torch_cuda, systems)
-    b, ib = batch_solve(dev, torch_cuda, systems, solver="batched")
-    for s, x, y in zip(systems, a, b):
-        assert np.linalg.norm(x - y) / np.linalg.norm(y) < 1e-5
-    assert all(i.status == 0 for i in ib)
+@pytest.mark.parametrize("orth", ["MGS", "CGS"])
+def test_wg_matches_shared_krylov_batched_solver(dev, torch_cuda, systems, orth):
+    small = [s for s in systems if s["n"] <= 3072]
+    assert len(small) >= 3
+    for syss, kw in ((systems, {"multi_launch": True}), (small, {"multi_launch": True}), (small, {})):
+        a, ia = batch_solve(dev, torch_cuda, syss, threads=1024)
+        b, ib = batch_solve(dev, torch_cuda, syss, solver="batched", orthogonalization=orth, **kw)
+        for s, x, y in zip(syss, a, b):
+            assert np.linalg.norm(x - y) / np.linalg.norm(y) < 1e-5
+        assert all(i.status == 0 for i in ib)
+        # the shared Krylov space: the systems that stay active as long took the same steps
+        steps = {}
+        for i in ib:
+            steps.setdefault(i.refinements, set()).add(i.inner_iterations)
+        same = all(len(v) == 1 for v in steps.values())
+        assert same == bool(kw), steps
 
 
 def test_wg_rejects_unsupported_options(dev, torch_cuda, systems):

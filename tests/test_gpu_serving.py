@@ -42,6 +42,10 @@ def test_server_results_alone_in_the_mix_and_fp64(reqs, small_solver):
         assert all(i.wg_threads == (512 if s else 0) for i, s in zip(infos, small))
     else:
         assert all(i.wg_threads == 0 for i in infos)
+        steps = {}   # one Krylov space: requests of a batch that stay active as long took the same steps
+        for i in infos:
+            steps.setdefault((i.batch_id, i.refinements), set()).add(i.iterations)
+        assert all(len(v) == 1 for v in steps.values()), steps
     assert all(i.status == 0 for i in infos)
     assert max(i.true_rel_residual for i in infos) <= 1e-8
     assert all(i.t_end >= i.t_start >= i.t_submit for i in infos)
