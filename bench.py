@@ -435,12 +435,12 @@ def main():
                           "column_bytes": A.sweep_info()["jacobi_column_bytes"]}))
         return
 
-    # kernel of the FP64 products (csrmv, pgmres operator, FP64 residual): CSR lanes per row or
-    # sliced ELL (0), tuned on the assembled matrix before any timed region
+    # kernel of the FP64 products (csrmv, pgmres operator, FP64 residual): CSR lanes per row, staged CSR
+    # (-1) or sliced ELL (0), tuned on the assembled matrix before any timed region
     M.Build_M_K_R_SUPG(pb, alpha, dt, u, du, R, AA_ptr=aa)
     A.values_changed()
     lanes, lane_us = A.autotune()
-    print(f"# FP64 product kernel (lanes per row, 0 = sliced ELL): {lanes} (" +
+    print(f"# FP64 product kernel (lanes per row, -1 = staged, 0 = sliced ELL): {lanes} (" +
           ", ".join(f"{k}: {v:.1f} us" for k, v in lane_us.items()) + ")", file=sys.stderr, flush=True)
 
     if a.profile_step:
@@ -547,14 +547,15 @@ def main():
     # 16-bit distances from the row, else 4 (int32, as in CSR)
     si = A.sweep_info()
     cbs, cbj = si["sell_column_bytes"] or 4, si["jacobi_column_bytes"] or 4
-    bytes_spmv = (8 + (cbs if lanes == 0 else 4)) * nnz + 4 * (n + 1) + 16 * n
+    bytes_spmv = (8 + (cbs if lanes <= 0 else 4)) * nnz + 4 * (n + 1) + 16 * n
     bytes_spmv32 = (4 + cbs) * nnz + 4 * (n + 1) + 8 * n
     bytes_ilu = 12 * (nnz - n) + 8 * (n + 1) + 8 * n + 16 * n
     bytes_jac = a.jacobi * ((4 + cbj) * (nnz - n) + 44 * n)
     kernels = {
         "column_bytes": {"sliced_ell": cbs, "jacobi_triangles": cbj},
         "csrmv_f64": dict(us=t_spmv * 1e6, GBs=bytes_spmv / t_spmv / 1e9, lanes_per_row=lanes,
-                          kernel="k_spmv_sell<double> (sliced ELL)" if lanes == 0 else f"k_spmv<double,{lanes}> (CSR)"),
+                          kernel={0: "k_spmv_sell<double> (sliced ELL)", -1: "k_spmv_staged (CSR)"}.get(
+                              lanes, f"k_spmv<double,{lanes}> (CSR)")),
         "csrmv_f64_cold": dict(us=t_spmv_cold * 1e6, GBs=bytes_spmv / t_spmv_cold / 1e9),
         "csrmv_f32": dict(us=t_spmv32 * 1e6, GBs=bytes_spmv32 / t_spmv32 / 1e9),
         "csrmv_f32_cold": dict(us=t_spmv32_cold * 1e6, GBs=bytes_spmv32 / t_spmv32_cold / 1e9),

@@ -163,17 +163,19 @@ int femgpu_csrmv_f32(femgpu_csr *A, const float *d_P, float *d_Q);
  * L = 1, 2, 4, 8, 16 lanes per row of the CSR kernel (64 / L rows per wavefront), or L = 0: one row
  * per thread on the 64-row sliced-ELL copy, with an FP64 copy of the values in that layout (kept,
  * and refreshed by femgpu_csr_values_changed, only while L = 0; needs the sliced-ELL copy with
- * slices at most 16 wide, else FEMGPU_ERR_ARG). femgpu_csr_autotune times every candidate on A's
- * structure and current values (20 launches each, HIP events) and keeps the fastest; us[] =
- * microseconds per launch for L = 1, 2, 4, 8, 16, us_sell for L = 0 (0 where not possible).
- * Synchronises the context's stream. Until one of the two is called, a kernel chosen from the
- * matrix's size and row length reads the CSR arrays. No reference counterpart (the reference's
- * csrmv is one loop per row). */
+ * slices at most 16 wide, else FEMGPU_ERR_ARG), or L = -1, the default: a kernel that reads the CSR arrays,
+ * chosen from the matrix's size and row length (for large matrices one that stages 64 rows through
+ * LDS, which no other L names). femgpu_csr_autotune times every candidate on A's structure and current
+ * values (20 launches each, HIP events) and keeps the fastest; us[] = microseconds per launch for
+ * L = 1, 2, 4, 8, 16, us_sell for L = 0 and us_staged for the staged kernel (0 where not possible).
+ * Synchronises the context's stream. No reference counterpart (the reference's csrmv is one loop per
+ * row). */
 typedef struct {
-    int lanes;             /* the L chosen */
+    int lanes;             /* the L chosen (-1: the staged kernel, or a matrix without rows) */
     int pad;
     double us[5];          /* per-launch time of L = 1, 2, 4, 8, 16 */
     double us_sell;        /* per-launch time of L = 0 */
+    double us_staged;      /* per-launch time of L = -1 where that is the staged kernel */
 } femgpu_tune_info;
 int femgpu_csr_autotune(femgpu_csr *A, femgpu_tune_info *info);
 int femgpu_csr_set_lanes(femgpu_csr *A, int lanes);

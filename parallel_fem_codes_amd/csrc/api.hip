@@ -358,8 +358,8 @@ extern "C" int femgpu_csr_autotune(femgpu_csr *A, femgpu_tune_info *info)
 
 extern "C" int femgpu_csr_set_lanes(femgpu_csr *A, int lanes)
 {
-    FG_CHECK(A && (lanes == 0 || lanes == 1 || lanes == 2 || lanes == 4 || lanes == 8 || lanes == 16),
-             FEMGPU_ERR_ARG, "femgpu_csr_set_lanes: lanes per row must be 1, 2, 4, 8 or 16 (0: sliced ELL)");
+    FG_CHECK(A && (lanes == -1 || lanes == 0 || lanes == 1 || lanes == 2 || lanes == 4 || lanes == 8 || lanes == 16),
+             FEMGPU_ERR_ARG, "femgpu_csr_set_lanes: lanes per row must be 1, 2, 4, 8 or 16 (0: sliced ELL, -1: the default)");
     return set_spmv_lanes(A, lanes);
 }
 

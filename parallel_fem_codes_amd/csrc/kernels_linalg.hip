@@ -531,16 +531,17 @@ __global__ void k_fill(int n, double v, double *__restrict__ x)
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) x[k] = v;
 }
 
-// Rows-per-wavefront autotuning of the FP64 CSR kernels (SpMV and residual share the choice): each
-// candidate lanes-per-row L (64 / L rows per wavefront) is timed with HIP events over 20 launches on
+// Autotuning of the FP64 CSR kernels (SpMV and residual share the choice): each candidate lanes-per-row L
+// (64 / L rows per wavefront), sliced ELL and the staged kernel, where it is the default, are timed with HIP events over 20 launches on
 // the matrix's own structure and values, after two warm-up launches; the fastest is kept.
 int csr_autotune(femgpu_csr *A, femgpu_tune_info *info)
 {
     femgpu_ctx *ctx = A->ctx;
-    // candidates: CSR with 1, 2, 4, 8, 16 lanes per row, then FP64 sliced ELL (lanes 0) where possible
-    static constexpr int kLanes[6] = {1, 2, 4, 8, 16, 0};
+    // candidates: CSR with 1, 2, 4, 8, 16 lanes per row, then the staged kernel (lanes -1, where the default is
+    // none of these) and FP64 sliced ELL (lanes 0) where possible
+    static constexpr int kLanes[7] = {1, 2, 4, 8, 16, -1, 0};
     femgpu_tune_info out{};
-    out.lanes = A->spmv_lanes < 0 ? 8 : A->spmv_lanes;
+    out.lanes = A->spmv_lanes;
     if (A->n == 0) {
         if (info) *info = out;
         return FEMGPU_OK;
@@ -554,10 +555,10 @@ int csr_autotune(femgpu_csr *A, femgpu_tune_info *info)
     FG_HIP(hipEventCreate(&e0));
     FG_HIP(hipEventCreate(&e1));
     const int saved = A->spmv_lanes;
-    const int ncand = sell64_possible(A) ? 6 : 5;
     int best = saved, rc = FEMGPU_OK;
     float best_ms = 0.0f;
-    for (int c = 0; c < ncand && rc == FEMGPU_OK; ++c) {
+    for (int c = 0; c < 7 && rc == FEMGPU_OK; ++c) {
+        if (kLanes[c] == 0 ? !sell64_possible(A) : kLanes[c] < 0 && A->staged_cap == 0) continue;
         if (kLanes[c] == 0) rc = set_spmv_lanes(A, 0);   // allocates and fills the FP64 sliced-ELL values
         else A->spmv_lanes = kLanes[c];
         for (int w = 0; w < 2 && rc == FEMGPU_OK; ++w) rc = launch_spmv64(ctx, A, x.p, nullptr, nullptr, y.p, nullptr);
@@ -568,7 +569,7 @@ int csr_autotune(femgpu_csr *A, femgpu_tune_info *info)
                                 hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
             rc = FEMGPU_ERR_HIP;
         if (rc != FEMGPU_OK) break;
-        (kLanes[c] == 0 ? out.us_sell : out.us[c]) = 1e3 * ms / 20.0;
+        (kLanes[c] == 0 ? out.us_sell : kLanes[c] < 0 ? out.us_staged : out.us[c]) = 1e3 * ms / 20.0;
         if (c == 0 || ms < best_ms) {
             best_ms = ms;
             best = kLanes[c];

@@ -276,18 +276,21 @@ class CsrMatrix:
         N.check(N.lib().femgpu_csr_rebuild(self.h, self.n, self.nnz, _i32(IA), _i32(JA)))
 
     def autotune(self):
-        """Times the FP64 product kernels (CSR at 1, 2, 4, 8 and 16 lanes per row; sliced ELL, lanes
-        0, where the structure allows it) and keeps the fastest; returns (lanes chosen, {lanes:
-        microseconds per launch})."""
+        """Times the FP64 product kernels (CSR at 1, 2, 4, 8 and 16 lanes per row; the staged CSR kernel,
+        lanes -1, where the matrix is large enough to have it as its default; sliced ELL, lanes 0, where
+        the structure allows it) and keeps the fastest; returns (lanes chosen, {lanes: microseconds per
+        launch})."""
         t = N.TuneInfo()
         N.check(N.lib().femgpu_csr_autotune(self.h, C.byref(t)))
         us = {L: t.us[k] for k, L in enumerate((1, 2, 4, 8, 16))}
         if t.us_sell > 0:
             us[0] = t.us_sell
+        if t.us_staged > 0:
+            us[-1] = t.us_staged
         return t.lanes, us
 
     def set_lanes(self, lanes):
-        """Lanes per row of the FP64 CSR kernels (1, 2, 4, 8, 16) or 0 for FP64 sliced ELL."""
+        """Lanes per row of the FP64 CSR kernels (1, 2, 4, 8, 16), 0 for FP64 sliced ELL, -1 for the default."""
         N.check(N.lib().femgpu_csr_set_lanes(self.h, int(lanes)))
 
     def sweep_info(self):

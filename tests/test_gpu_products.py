@@ -64,6 +64,31 @@ def test_large_csr_products(torch_cuda, n, offsets, keep, dense):
     assert (np.abs(q.cpu().numpy() - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("offsets", [list(range(-12, 13)), [-600, -599, -1, 1, 599, 600]])
+def test_autotune_times_the_default(torch_cuda, offsets):
+    """A large matrix, with and without sliced ELL: the default is among the candidates, the kept kernel is
+    the fastest measured, and -1 brings the default back (its sums, bit for bit)."""
+    torch = torch_cuda
+    n = 120000 if len(offsets) > 16 else 320001
+    rng = np.random.default_rng(n)
+    IA, JA = banded(n, offsets, 1.0, rng)
+    dev = fem.Device(0)
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(rng.standard_normal(len(JA)))
+    p = torch.from_numpy(rng.standard_normal(n)).cuda()
+    default, q = torch.empty_like(p), torch.empty_like(p)
+    A.csrmv(p, default)
+    lanes, us = A.autotune()
+    assert set(us) == {-1, 1, 2, 4, 8, 16} | ({0} if len(offsets) <= 16 else set())
+    assert us[lanes] == min(us.values())
+    A.set_lanes(16)
+    A.set_lanes(-1)
+    A.csrmv(p, q)
+    assert torch.equal(q, default)
+    empty = fem.CsrMatrix(dev, np.zeros(1, np.int32), np.zeros(0, np.int32))
+    assert empty.autotune()[0] == -1   # nothing to time: the default stays
+
+
 def test_large_residual(torch_cuda):
     """The mixed solver on a diagonally dominant matrix of that size: its FP64 residual (the staged
     kernel with the fused norm) is the one numpy computes."""
