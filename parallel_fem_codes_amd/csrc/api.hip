@@ -229,7 +229,8 @@ static int csr_setup(femgpu_csr *A, int n, int nnz, const int *IA, const int *JA
         if (!rc) rc = build_stream_plan(ctx, n, IA, JA, diag.data(), true, A->sup);
         if (!rc) rc = build_stream_maps(ctx, A);
         if (!rc) rc = build_stream_factor(ctx, A, IA, JA, diag.data());
-        if (!rc) rc = build_rows_factor(ctx, A, IA, JA, diag.data());
+        if (A->sfac.ok && A->factor_kernel == 0) A->rfac.release();
+        else if (!rc) rc = build_rows_factor(ctx, A);
     }
     if (!rc) rc = build_sell(ctx, A, IA, JA);
     if (!rc) rc = build_staged(ctx, A, IA, JA);
@@ -333,6 +334,8 @@ extern "C" int femgpu_csr_sweep_info(femgpu_csr *A, femgpu_sweep_info *info)
 extern "C" int femgpu_csr_set_factor_kernel(femgpu_csr *A, int kernel)
 {
     FG_CHECK(A && (kernel == 0 || kernel == 1), FEMGPU_ERR_ARG, "femgpu_csr_set_factor_kernel: bad arguments");
+    // a matrix whose factorisation is streamed has no plan of the level-synchronous one until it is asked for
+    if (kernel == 1 && (A->plans & FEMGPU_PLANS_FP64) && !A->rfac.ok) FG_TRY(build_rows_factor(A->ctx, A));
     A->factor_kernel = kernel;
     return FEMGPU_OK;
 }

@@ -158,7 +158,8 @@ struct StreamFactor {
     DevBuf<double> dinv;     // general, n + kStreamThreads: inverse pivots in schedule order
 };
 
-// Level-synchronous ILU(0) factorisation of rows of at most 32 entries, 16 lanes per row (factor_rows.hip).
+// Level-synchronous ILU(0) factorisation of rows of at most 32 entries, 16 lanes per row (factor_rows.hip):
+// 400 bytes a row, so only for matrices whose factorisation is not streamed, or on demand.
 struct RowsFactor {
     bool ok = false;
     bool wide = false;       // rows with more than 16 L or 15 U entries: 8-bit codes, two passes
@@ -166,6 +167,12 @@ struct RowsFactor {
     DevBuf<int4> info;       // schedule position -> {first entry, length, L count, row}
     DevBuf<int2> dep;        // per L entry: {first U entry of its row, its row}
     DevBuf<unsigned long long> code;   // U columns of the (entry, L entry) pairs
+    void release() {
+        ok = false;
+        info.release();
+        dep.release();
+        code.release();
+    }
 };
 
 // Update lists of the parallel factorisation: for every row its CSR position, length, number of L
@@ -365,7 +372,7 @@ int build_stream_maps(femgpu_ctx *ctx, femgpu_csr *A);
 int build_stream_factor(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag);
 size_t factor_lds_bytes(const StreamSweep &P);
 int launch_stream_factor(femgpu_ctx *ctx, femgpu_csr *A);
-int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag);
+int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A);
 int launch_rows_factor(femgpu_ctx *ctx, femgpu_csr *A);
 int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, FactorPlan &F);
 // LDS bytes one workgroup of the packed sweep needs for T-typed values.

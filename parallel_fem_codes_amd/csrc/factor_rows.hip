@@ -203,12 +203,14 @@ __global__ __launch_bounds__(THREADS) void k_ilu0_factor_rows(RowsArgs A)
     }
 }
 
-int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag)
+int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A)
 {
     RowsFactor &F = A->rfac;
     F.ok = false;
-    const int n = A->n;
+    const int n = A->n, *IA = A->hIA.data(), *JA = A->hJA.data();
     if (n == 0) return FEMGPU_OK;
+    std::vector<int> diag(n);
+    for (int i = 0; i < n; ++i) diag[i] = static_cast<int>(std::lower_bound(JA + IA[i], JA + IA[i + 1], i) - JA);
     int maxrow = 0, maxL = 0, maxU = 0;
     for (int i = 0; i < n; ++i) {
         maxrow = std::max(maxrow, IA[i + 1] - IA[i]);

@@ -62,6 +62,40 @@ def test_factor_rows_bit_exact(oracle, case):
         assert np.array_equal(LU, LUo[:-1]) and np.array_equal(Di, Dio)
 
 
+def test_factor_rows_plan_on_demand(oracle):
+    """A matrix with the streamed factorisation holds no plan of the level-synchronous one (400 bytes a row) until
+    it is asked for; a rebuilt matrix keeps the kernel asked for."""
+    import torch
+    dev = fem.Device(0)
+    IA, JA = block_pattern(600, 1)
+    n = len(IA) - 1
+    A = fem.CsrMatrix(dev, IA, JA)
+    assert A.sweep_info()["factor_kernel"] == 0
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    A.set_factor_kernel("lists")
+    assert free - torch.cuda.mem_get_info()[0] >= 350 * n
+    rng = np.random.default_rng(4)
+    for m in (40, 55):
+        IA, JA = block_pattern(m, 1)
+        n = len(IA) - 1
+        A.rebuild(IA, JA)
+        AA = rng.uniform(-1, 1, len(JA))
+        AA[JA == np.repeat(np.arange(n), np.diff(IA))] = 9.0
+        A.set_values(AA)
+        A.ilu0_factor()
+        assert A.sweep_info()["factor_kernel"] == 1
+        LUo, Dio, rc = oracle.ilu0_factor(IA, JA, np.append(AA, 0.0))
+        LU, Di = A.ilu0_factors()
+        assert rc == 0 and np.array_equal(LU, LUo[:-1]) and np.array_equal(Di, Dio)
+        A.set_factor_kernel("stream")
+        A.set_values(2 * AA)
+        A.ilu0_factor()
+        assert np.array_equal(A.ilu0_factors()[0][JA >= np.repeat(np.arange(n), np.diff(IA))],
+                              2 * LU[JA >= np.repeat(np.arange(n), np.diff(IA))])
+        A.set_factor_kernel("lists")
+
+
 def test_factor_rows_zero_pivot():
     """A zero pivot in the middle of the schedule is reported."""
     IA, JA = block_pattern(12, 3)
