@@ -147,12 +147,14 @@ typedef struct femgpu_sweep_info {
     int factor_compact;        /* streamed factorisation: 1 for the compact row shape (every row at most
                                   7 entries, 3 L and 3 U), 2 for the compact shape on the pair pattern
                                   of the structured triangle meshes, 0 for the general one */
+    int factor_row_lanes;      /* level-synchronous factorisation: lanes per row, 16, or 1 for short rows in
+                                  wide levels (streamed: 0) */
 } femgpu_sweep_info;
 int femgpu_csr_sweep_info(femgpu_csr *A, femgpu_sweep_info *info);
 /* Select the sweep kernel: 0 = streamed when the plan allows it (default), 1 = packed. */
 int femgpu_csr_set_sweep_kernel(femgpu_csr *A, int kernel);
 /* Select the numeric factorisation kernel: 0 = streamed when the plan allows it (default),
- * 1 = level-synchronous, 16 lanes per row. Both give the same factors. */
+ * 1 = level-synchronous. Both give the same factors. */
 int femgpu_csr_set_factor_kernel(femgpu_csr *A, int kernel);
 
 /* csrmv (CSR/csrmv.c:4-65), local block: Q = A P. FP64 and FP32 (FP32 copy of the values). */

@@ -235,7 +235,7 @@ static int csr_setup(femgpu_csr *A, int n, int nnz, const int *IA, const int *JA
     if (!rc) rc = build_sell(ctx, A, IA, JA);
     if (!rc) rc = build_staged(ctx, A, IA, JA);
     if (plans & FEMGPU_PLANS_MIXED) {   // parallel FP32 ILU(0) and Jacobi iterations
-        if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), A->fplan_nat);
+        if (!rc) rc = build_factor_plan(ctx, A, IA, JA, diag.data(), true, A->fplan_nat);
         if (!rc) rc = build_jacobi_ell(ctx, A, IA, JA, diag.data());
         if (!rc) rc = build_parilu_sell(ctx, A, IA, JA, diag.data());
     }
@@ -324,6 +324,7 @@ extern "C" int femgpu_csr_sweep_info(femgpu_csr *A, femgpu_sweep_info *info)
     info->rows_per_chunk = A->plo.R;
     info->lds_limit = static_cast<int>(A->ctx->lds_limit);
     info->factor_kernel = (A->factor_kernel == 0 && A->sfac.ok) ? 0 : 1;
+    info->factor_row_lanes = info->factor_kernel == 0 || !A->rfac.ok ? 0 : A->rfac.lists ? 1 : 16;
     info->jacobi_column_bytes = A->ell_kl > 0 ? (A->ell16 ? 2 : 4) : 0;
     info->sell_column_bytes = A->sell_ok ? (A->sell16 ? 2 : 4) : 0;
     info->long_slots = std::max(A->slo.L, A->sup.L);

@@ -158,10 +158,22 @@ struct StreamFactor {
     DevBuf<double> dinv;     // general, n + kStreamThreads: inverse pivots in schedule order
 };
 
-// Level-synchronous ILU(0) factorisation of rows of at most 32 entries, 16 lanes per row (factor_rows.hip):
-// 400 bytes a row, so only for matrices whose factorisation is not streamed, or on demand.
+// Update lists of a factorisation: for every row (in row order, or of the lower sweep's schedule) its CSR
+// position, length, number of L entries, and its update list -- (U entry position k of a dependency row,
+// target slot in this row, index t of the L entry it belongs to) -- in the serial factorisation's order.
+struct FactorPlan {
+    int maxrow = 0, nupd = 0, maxupd = 0;
+    DevBuf<int4> rowinfo;   // per row: {p0, len, nL, first update}
+    DevBuf<int2> upd;       // {k, dest | t << 16}; dest == nL marks the pivot
+};
+
+// Level-synchronous ILU(0) factorisation of rows of at most 32 entries (factor_rows.hip): 16 lanes per row, or
+// a thread per row where the rows are short and the levels wide. 400 bytes a row in the first form, so only for
+// matrices whose factorisation is not streamed, or on demand.
 struct RowsFactor {
     bool ok = false;
+    bool lists = false;      // a thread per row, along its update list
+    FactorPlan plan;         // lists: by schedule position
     bool wide = false;       // rows with more than 16 L or 15 U entries: 8-bit codes, two passes
     int maxlevel = 0;        // most rows of a level
     DevBuf<int4> info;       // schedule position -> {first entry, length, L count, row}
@@ -169,19 +181,12 @@ struct RowsFactor {
     DevBuf<unsigned long long> code;   // U columns of the (entry, L entry) pairs
     void release() {
         ok = false;
+        plan.rowinfo.release();
+        plan.upd.release();
         info.release();
         dep.release();
         code.release();
     }
-};
-
-// Update lists of the parallel factorisation: for every row its CSR position, length, number of L
-// entries, and its update list -- (U entry position k of a dependency row, target slot in this row,
-// index t of the L entry it belongs to) -- in the serial factorisation's order.
-struct FactorPlan {
-    int maxrow = 0, nupd = 0, maxupd = 0;
-    DevBuf<int4> rowinfo;   // per row: {p0, len, nL, first update}
-    DevBuf<int2> upd;       // {k, dest | t << 16}; dest == nL marks the pivot
 };
 
 }  // namespace fg
@@ -374,7 +379,9 @@ size_t factor_lds_bytes(const StreamSweep &P);
 int launch_stream_factor(femgpu_ctx *ctx, femgpu_csr *A);
 int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A);
 int launch_rows_factor(femgpu_ctx *ctx, femgpu_csr *A);
-int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, FactorPlan &F);
+// natural: rows in index order (the parallel factorisation); else the lower sweep's level schedule.
+int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, bool natural,
+                      FactorPlan &F);
 // LDS bytes one workgroup of the packed sweep needs for T-typed values.
 template <typename T>
 inline size_t packed_lds_bytes(const PackedSweep &P)

@@ -203,6 +203,82 @@ __global__ __launch_bounds__(THREADS) void k_ilu0_factor_rows(RowsArgs A)
     }
 }
 
+// Short rows in wide levels: a thread per row, 512 rows of a level at a time. A row first issues all of its loads
+// together (its update list, the finished U values and pivots it reads, its own values); its values and
+// multipliers then live in LDS while the list is applied one by one. That chain is longer than the 16
+// lanes', but a level of several hundred rows takes one round of it, where those take a round per 64 rows.
+// Same operations in the same order, contraction off.
+constexpr int kListRow = 8, kListUpd = 24, kListThreads = 512;
+
+__global__ __launch_bounds__(kListThreads) void k_ilu0_factor_lists(int depth, const int *__restrict__ lvl_ptr,
+                                                                    const int4 *__restrict__ rowinfo,
+                                                                    const int2 *__restrict__ upd,
+                                                                    const int *__restrict__ JA,
+                                                                    const double *__restrict__ AA, double *LU,
+                                                                    double *Dinv, int *err)
+{
+#pragma clang fp contract(off)
+    __shared__ double scratch[2 * kListRow * kListThreads];
+    double *v = scratch + threadIdx.x;                                 // row value e at v[e * kListThreads]
+    double *dj = scratch + kListRow * kListThreads + threadIdx.x;      // pivot inverse of L entry t, likewise
+    for (int l = 0; l < depth; ++l) {
+        const int q1 = lvl_ptr[l + 1];
+        for (int q = lvl_ptr[l] + static_cast<int>(threadIdx.x); q < q1; q += kListThreads) {
+            const int4 ri = rowinfo[q];
+            const int p0 = ri.x, len = ri.y, nL = ri.z, ub = ri.w;
+            const int nu = rowinfo[q + 1].w - ub;   // rowinfo has a sentinel entry after the last row
+            const int i = JA[p0 + nL];
+            int jr[kListRow];
+#pragma unroll
+            for (int t = 0; t < kListRow; ++t)
+                if (t < nL) jr[t] = JA[p0 + t];
+#pragma unroll
+            for (int e = 0; e < kListRow; ++e)
+                if (e < len) v[e * kListThreads] = AA[p0 + e];
+#pragma unroll
+            for (int t = 0; t < kListRow; ++t)
+                if (t < nL) dj[t * kListThreads] = Dinv[jr[t]];
+            int sc = 0;   // L entries [0, sc) already turned into multipliers
+            for (int u0 = 0; u0 < nu; u0 += kListUpd) {   // a chunk's list entries and U values loaded together
+                int2 U[kListUpd];
+                double Uv[kListUpd];
+#pragma unroll
+                for (int u = 0; u < kListUpd; ++u)
+                    if (u0 + u < nu) U[u] = upd[ub + u0 + u];
+#pragma unroll
+                for (int u = 0; u < kListUpd; ++u)
+                    if (u0 + u < nu) Uv[u] = LU[U[u].x];
+#pragma unroll
+                for (int u = 0; u < kListUpd; ++u) {
+                    if (u0 + u < nu) {
+                        const int t = U[u].y >> 16, dest = U[u].y & 0xffff;
+                        for (; sc <= t; ++sc) v[sc * kListThreads] = v[sc * kListThreads] * dj[sc * kListThreads];
+                        v[dest * kListThreads] -= v[t * kListThreads] * Uv[u];
+                    }
+                }
+            }
+            for (; sc < nL; ++sc) v[sc * kListThreads] = v[sc * kListThreads] * dj[sc * kListThreads];
+#pragma unroll
+            for (int e = 0; e < kListRow; ++e)
+                if (e < len) LU[p0 + e] = v[e * kListThreads];
+            const double piv = v[nL * kListThreads];
+            if (piv == 0.0) {
+                __hip_atomic_store(err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                Dinv[i] = 0.0;
+            } else {
+                Dinv[i] = 1.0 / piv;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Rows per level, on average, from which rows of at most 8 entries take a thread each. Seven-point matrices,
+// a thread per row against 16 lanes: 133 rows 7.4 / 5.5 ms, 167 9.7 / 8.4, 200 12.4 / 13.5, 333 30 / 38 (400 x 400 to
+// 1000 x 1000 squares, SYMRCM); in random order 700 rows 0.22 / 0.38 ms (n = 9 801), 24 000 rows 12.3 / 18.4
+// (n = 4.9e5).
+constexpr int kListLevel = 192;
+
 int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A)
 {
     RowsFactor &F = A->rfac;
@@ -218,6 +294,12 @@ int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A)
         maxU = std::max(maxU, IA[i + 1] - diag[i] - 1);
     }
     if (maxrow > 32) return FEMGPU_OK;
+    F.lists = maxrow <= kListRow && n / std::max(1, A->plo.depth) >= kListLevel;
+    if (F.lists) {
+        FG_TRY(build_factor_plan(ctx, A, IA, JA, diag.data(), false, F.plan));
+        F.ok = true;
+        return FEMGPU_OK;
+    }
     F.wide = maxL > 16 || maxU > 15;
     const int np = F.wide ? 2 : 1, nw = F.wide ? 2 : 1;
     std::vector<int> row_of(n), slot(n, -1);
@@ -262,6 +344,13 @@ int build_rows_factor(femgpu_ctx *ctx, femgpu_csr *A)
 int launch_rows_factor(femgpu_ctx *ctx, femgpu_csr *A)
 {
     const RowsFactor &F = A->rfac;
+    if (F.lists) {
+        k_ilu0_factor_lists<<<1, kListThreads, 0, ctx->stream>>>(A->plo.depth, A->plo.lvl_ptr.p, F.plan.rowinfo.p,
+                                                                 F.plan.upd.p, A->JA.p, A->AA.p, A->LU.p, A->Dinv.p,
+                                                                 ctx->err.p);
+        FG_HIP(hipGetLastError());
+        return FEMGPU_OK;
+    }
     RowsArgs a;
     a.depth = A->plo.depth;
     a.lvl_ptr = A->plo.lvl_ptr.p;

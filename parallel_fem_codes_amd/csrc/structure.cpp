@@ -857,16 +857,20 @@ int build_stream_factor(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int
     return FEMGPU_OK;
 }
 
-int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, FactorPlan &F)
+int build_factor_plan(femgpu_ctx *ctx, femgpu_csr *A, const int *IA, const int *JA, const int *diag, bool natural,
+                      FactorPlan &F)
 {
     const int n = A->n;
+    std::vector<int> row_of(n);
+    std::iota(row_of.begin(), row_of.end(), 0);
+    if (!natural) FG_HIP(hipMemcpy(row_of.data(), A->plo.row_of.p, sizeof(int) * n, hipMemcpyDeviceToHost));
     std::vector<int4> info(static_cast<size_t>(n) + 1);
     std::vector<int2> upd;
     upd.reserve(static_cast<size_t>(IA[n]) * 2);
     std::vector<int> slot(n, -1);
     int maxrow = 0, maxupd = 0;
     for (int q = 0; q < n; ++q) {
-        const int i = q, p0 = IA[i], len = IA[i + 1] - p0, nL = diag[i] - p0;
+        const int i = row_of[q], p0 = IA[i], len = IA[i + 1] - p0, nL = diag[i] - p0;
         const size_t u0 = upd.size();
         maxrow = std::max(maxrow, len);
         info[q] = make_int4(p0, len, nL, static_cast<int>(upd.size()));

@@ -300,7 +300,7 @@ class CsrMatrix:
 
     def set_factor_kernel(self, kind):
         """"stream" (single-workgroup streamed factorisation, the default where its plan exists) or
-        "lists" (level-synchronous, 16 lanes per row)."""
+        "lists" (level-synchronous)."""
         N.check(N.lib().femgpu_csr_set_factor_kernel(self.h, {"stream": 0, "lists": 1}[kind]))
 
     def set_sweep_kernel(self, kind):

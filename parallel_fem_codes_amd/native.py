@@ -60,7 +60,7 @@ class SweepInfo(C.Structure):
     _fields_ = [(f, C.c_int) for f in ("kernel", "depth_lower", "depth_upper", "steps_lower", "steps_upper",
                                         "ring", "entries_per_row", "chunks_lower", "rows_per_chunk", "lds_limit",
                                         "factor_kernel", "jacobi_column_bytes", "sell_column_bytes", "long_slots",
-                                        "factor_compact")]
+                                        "factor_compact", "factor_row_lanes")]
 
 
 class MixedOpts(C.Structure):

@@ -1,5 +1,5 @@
-"""The level-synchronous ILU(0) factorisation (16 lanes per row) at the edges of its row shapes: factors
-bit-identical to the CPU oracle's serial elimination."""
+"""The level-synchronous ILU(0) factorisation (16 lanes per row, or a thread per short row of wide levels) at the
+edges of its row shapes: factors bit-identical to the CPU oracle's serial elimination."""
 import numpy as np
 import pytest
 
@@ -30,15 +30,19 @@ def block_pattern(m, ndof):
 
 
 @pytest.mark.parametrize("case", ["n1", "diag300", "l16u15", "l17u14", "l15u16", "l31", "u31", "wide_level", "ns24",
-                                  "euler16", "euler40"])
+                                  "euler16", "euler40", "diag191", "diag192", "short8", "short8_deep", "short9"])
 def test_factor_rows_bit_exact(oracle, case):
     rng = np.random.default_rng(len(case) * 7 + ord(case[-1]))
     if case == "n1":
         IA, JA = np.array([0, 1], np.int32), np.array([0], np.int32)
-    elif case == "diag300":
-        IA, JA = np.arange(301, dtype=np.int32), np.arange(300, dtype=np.int32)   # one level
+    elif case.startswith("diag"):
+        n = int(case[4:])
+        IA, JA = np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32)   # one level
     elif case == "wide_level":
         IA, JA = random_pattern(3000, 1500, 9, 9, rng)      # levels of several hundred rows
+    elif case.startswith("short"):   # rows of up to 8 or 9 entries: a few levels of thousands of rows, or 7 L entries
+        size, l, u = {"short8": (9000, 1, 6), "short8_deep": (16000, 7, 0), "short9": (9000, 1, 7)}[case]
+        IA, JA = random_pattern(size, size, l, u, rng)
     elif case.startswith("ns"):
         IA, JA = block_pattern(24, 3)
     elif case.startswith("euler"):
@@ -54,6 +58,10 @@ def test_factor_rows_bit_exact(oracle, case):
     A = fem.CsrMatrix(dev, IA, JA)
     A.set_factor_kernel("lists")
     A.set_values(AA)
+    if case.startswith(("diag", "short")):   # a thread per row from 192 rows a level on, for at most 8 entries
+        info = A.sweep_info()
+        lists = n // info["depth_lower"] >= 192 and np.diff(IA).max() <= 8
+        assert info["factor_row_lanes"] == (1 if lists else 16) and lists == (case not in ("diag191", "short9"))
     LUo, Dio, rc = oracle.ilu0_factor(IA, JA, np.append(AA, 0.0))
     assert rc == 0
     for _ in range(2):
@@ -67,7 +75,7 @@ def test_factor_rows_plan_on_demand(oracle):
     it is asked for; a rebuilt matrix keeps the kernel asked for."""
     import torch
     dev = fem.Device(0)
-    IA, JA = block_pattern(600, 1)
+    IA, JA = block_pattern(500, 1)
     n = len(IA) - 1
     A = fem.CsrMatrix(dev, IA, JA)
     assert A.sweep_info()["factor_kernel"] == 0
@@ -96,9 +104,10 @@ def test_factor_rows_plan_on_demand(oracle):
         A.set_factor_kernel("lists")
 
 
-def test_factor_rows_zero_pivot():
+@pytest.mark.parametrize("short", [False, True])
+def test_factor_rows_zero_pivot(short):
     """A zero pivot in the middle of the schedule is reported."""
-    IA, JA = block_pattern(12, 3)
+    IA, JA = random_pattern(3000, 1500, 1, 6, np.random.default_rng(3)) if short else block_pattern(12, 3)
     n = len(IA) - 1
     rows = np.repeat(np.arange(n), np.diff(IA))
     AA = np.where(JA == rows, 4.0, 0.0)
@@ -106,5 +115,6 @@ def test_factor_rows_zero_pivot():
     dev = fem.Device(0)
     A = fem.CsrMatrix(dev, IA, JA)
     A.set_values(AA)
+    A.set_factor_kernel("lists")
     with pytest.raises(Exception, match="zero pivot"):
         A.ilu0_factor()
