@@ -507,15 +507,17 @@ __global__ __launch_bounds__(256) void k_seg_norm2(const int *__restrict__ off, 
 }
 
 // r32 = r * scale[system]: every active system's residual normalised to unit norm, finished
-// systems zeroed (their blocks of every Krylov vector then stay exactly zero).
+// systems zeroed, whatever is in their residual (their blocks of every Krylov vector then stay exactly zero).
 __global__ void k_scale_to_f32_seg(int n, const int *__restrict__ sys, const double *__restrict__ r,
                                    const double *__restrict__ scale, float *__restrict__ r32)
 {
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x)
-        r32[k] = static_cast<float>(r[k] * scale[sys[k]]);
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const double s = scale[sys[k]];
+        r32[k] = s == 0.0 ? 0.0f : static_cast<float>(r[k] * s);
+    }
 }
 
-// X += rn[system] * (V y): the cycle's correction of each system scaled back by its residual norm.
+// X += rn[system] * (V y): the cycle's correction of each system scaled back by its residual norm (0: finished).
 __global__ __launch_bounds__(256) void k_cycle_finish_seg(GDev G, int n, const float *__restrict__ V, size_t ldv,
                                                           double *__restrict__ X, const int *__restrict__ sys,
                                                           const double *__restrict__ rn)
@@ -528,7 +530,8 @@ __global__ __launch_bounds__(256) void k_cycle_finish_seg(GDev G, int n, const f
     __syncthreads();
     for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) {
         const double d = basis_sum<float, double>(0.0, V, ldv, k, i, ys);
-        X[k] = X[k] + rn[sys[k]] * d;
+        const double g = rn[sys[k]];
+        X[k] = g == 0.0 ? X[k] : X[k] + g * d;
     }
 }
 
@@ -1067,13 +1070,12 @@ extern "C" int femgpu_gmres_mixed(femgpu_ctx *ctx, const femgpu_system *S, const
         FG_TRY(wg_solve_one(ctx, S->csr, opt, tol, d_F, d_X, &bi));
         if (info) {
             memset(info, 0, sizeof(*info));
-            const bool finite = std::isfinite(bi.normF);
             info->iterations = info->inner_iterations = bi.inner_iterations;
             info->cycles = bi.refinements;
             info->normb = bi.normF;
-            info->true_rel_residual = bi.normF == 0.0 ? 0.0 : finite ? bi.true_rel_residual : bi.normF;
-            info->rho = finite ? bi.true_rel_residual * bi.normF : bi.normF;
-            info->status = finite && bi.status == 0 ? 0 : 1;
+            info->true_rel_residual = bi.true_rel_residual;
+            info->rho = std::isfinite(bi.normF) ? bi.true_rel_residual * bi.normF : bi.normF;
+            info->status = bi.status;
         }
         return FEMGPU_OK;
     }
@@ -1271,7 +1273,7 @@ extern "C" int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *
     const int grid = grid_for(n);
     if (n > 0) k_sys_of_row<<<grid * 4, 256, 0, ctx->stream>>>(n, nsys, ctx->bt_rowoff.p, ctx->bt_sys.p);
     FG_HIP(hipMemsetAsync(d_X, 0, sizeof(double) * n, ctx->stream));
-    std::vector<double> normF(nsys), rn(nsys), scale(nsys);
+    std::vector<double> normF(nsys), rn(nsys), scale(nsys), gain(nsys);
     std::vector<int> refin(nsys, 0), done(nsys, 0);
     int inner_total = 0, refinements = 0;
     auto seg_norms = [&](const double *v, std::vector<double> &out) -> int {
@@ -1292,14 +1294,17 @@ extern "C" int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *
         FG_TRY(seg_norms(r, rn));
         int active = 0;
         for (int s = 0; s < nsys; ++s) {
-            if (!done[s] && (rn[s] <= tol * normF[s] || refin[s] >= opt->max_refinements)) done[s] = 1;
+            // a system with a non-finite residual cannot be continued and must not reach the shared basis
+            if (!done[s] && (!std::isfinite(rn[s]) || rn[s] <= tol * normF[s] || refin[s] >= opt->max_refinements))
+                done[s] = 1;
             scale[s] = done[s] ? 0.0 : 1.0 / rn[s];
+            gain[s] = done[s] ? 0.0 : rn[s];
             active += !done[s];
         }
         if (active == 0) break;
         for (int s = 0; s < nsys; ++s) refin[s] += !done[s];
         FG_HIP(hipMemcpyAsync(d_scale, scale.data(), sizeof(double) * nsys, hipMemcpyHostToDevice, ctx->stream));
-        FG_HIP(hipMemcpyAsync(d_rn, rn.data(), sizeof(double) * nsys, hipMemcpyHostToDevice, ctx->stream));
+        FG_HIP(hipMemcpyAsync(d_rn, gain.data(), sizeof(double) * nsys, hipMemcpyHostToDevice, ctx->stream));
         k_scale_to_f32_seg<<<grid * 4, 256, 0, ctx->stream>>>(n, ctx->bt_sys.p, r, d_scale, wA);
         FG_HIP(hipGetLastError());
         FG_TRY(prec32(ctx, S->ilu, G.prec_mode, wA, wA, nullptr, nullptr, nfz ? ctx->jac_partials.p : nullptr));
@@ -1322,8 +1327,8 @@ extern "C" int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *
     for (int s = 0; s < nsys; ++s) {
         info[s].refinements = refin[s];
         info[s].normF = normF[s];
-        info[s].true_rel_residual = normF[s] > 0 ? rn[s] / normF[s] : 0.0;
-        info[s].status = (rn[s] <= tol * normF[s]) ? 0 : 1;
+        info[s].true_rel_residual = normF[s] == 0.0 ? 0.0 : std::isfinite(normF[s]) ? rn[s] / normF[s] : normF[s];
+        info[s].status = std::isfinite(rn[s]) && rn[s] <= tol * normF[s] ? 0 : 1;
     }
     (void)inner_total;
     return FEMGPU_OK;

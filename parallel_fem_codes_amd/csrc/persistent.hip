@@ -43,15 +43,17 @@ struct WgArgs {
     femgpu_batch_info *info;
 };
 
+__device__ __forceinline__ bool finite_norm(double v) { return v <= 1.7976931348623157e308; }
+
 __device__ __forceinline__ void wg_report(const WgArgs &a, int sys, int refinements, int inner, double rn, double normF)
 {
     femgpu_batch_info inf;
     inf.refinements = refinements;
     inf.inner_iterations = inner;
-    inf.status = (rn <= a.tol * normF) ? 0 : 1;
+    inf.status = finite_norm(rn) && rn <= a.tol * normF ? 0 : 1;
     inf.pad = 0;
     inf.normF = normF;
-    inf.true_rel_residual = normF > 0.0 ? rn / normF : 0.0;
+    inf.true_rel_residual = normF == 0.0 ? 0.0 : finite_norm(normF) ? rn / normF : normF;
     a.info[sys] = inf;
 }
 
@@ -370,7 +372,7 @@ __device__ __forceinline__ void wg_solve_lds(const WgArgs &a, double *sm, int *s
             }
         }
         rn = sqrt(wg_sum1<BS>(acc, red, half));
-        if (!(rn <= 1.7976931348623157e308) || rn <= a.tol * normF || refinements >= a.max_ref) break;
+        if (!finite_norm(rn) || rn <= a.tol * normF || refinements >= a.max_ref) break;
         ++refinements;
         // inner FP32 solve of M^-1 A d = M^-1 r / ||r||, started from d = 0
         const double inv_rn = 1.0 / rn;
@@ -510,7 +512,7 @@ __device__ void wg_solve_global(const WgArgs &a, double *sm, int &s_done)
             acc += v * v;
         }
         rn = sqrt(wg_sum<BS>(acc, red));
-        if (rn <= a.tol * normF || refinements >= a.max_ref) break;
+        if (!finite_norm(rn) || rn <= a.tol * normF || refinements >= a.max_ref) break;
         ++refinements;
         // inner FP32 solve of M^-1 A d = M^-1 r / ||r||, started from d = 0
         const double inv_rn = 1.0 / rn;

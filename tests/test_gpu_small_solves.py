@@ -123,3 +123,30 @@ def test_batch_of_coupled_rows(at):
         fem.gmres_mixed_wg(dev, A, off, Fd, X, tol=1e-9)
     infos = fem.gmres_mixed_wg(dev, A, [0, 0, sum(n)], Fd, X, tol=1e-9)   # one system and an empty one
     assert all(i.status == 0 for i in infos)
+
+
+@pytest.mark.parametrize("solver", ["batched", "shared", "wg"])
+@pytest.mark.parametrize("sizes", [[400, 300, 700, 200], [400, 5000, 300, 200]])
+def test_batch_with_infinite_and_nan_loads(solver, sizes):
+    """A system whose right-hand side holds an Inf or a NaN is reported unsolved with X = 0; its neighbours converge."""
+    import torch
+    dev = fem.Device(0)
+    syss = [system(n, 9, 300 + k) for k, n in enumerate(sizes)]
+    IA, JA, off, _ = fem.concat_csr([(s[0], s[1]) for s in syss])
+    A = fem.CsrMatrix(dev, IA, JA)
+    A.set_values(np.concatenate([s[2] for s in syss]))
+    F = np.concatenate([s[3] for s in syss])
+    F[off[0] + 5], F[off[2] + 17] = np.inf, np.nan
+    X = torch.full((off[-1],), 7.0, dtype=torch.float64, device="cuda")
+    if solver == "wg":
+        infos = fem.gmres_mixed_wg(dev, A, off, torch.from_numpy(F).cuda(), X, tol=1e-9)
+    else:
+        infos = fem.gmres_mixed_batched(dev, A, off, torch.from_numpy(F).cuda(), X, tol=1e-9, multi_launch=solver == "shared")
+    x = X.cpu().numpy()
+    for k, i in enumerate(infos):
+        xk, fk = x[off[k]:off[k + 1]], F[off[k]:off[k + 1]]
+        if k in (0, 2):
+            assert i.status == 1 and (xk == 0).all() and i.refinements == 0
+            assert not np.isfinite(i.normF) and not np.isfinite(i.true_rel_residual)
+        else:
+            assert i.status == 0 and residual(*syss[k][:3], fk, xk) <= 1.01e-9
