@@ -604,21 +604,30 @@ void csr_map(int nkeys, const std::vector<std::pair<int, int>> &pairs, std::vect
     for (auto &p : pairs) src[fill[rank[p.first]]++] = p.second;
 }
 
-// The lists ptr/src of keys 0 .. n - 1 (each in element order) reordered by their first source (empty
-// lists last), as csr_map orders them.
-static void order_lists(int n, std::vector<int> &ptr, std::vector<int> &src, std::vector<int> &dst)
+// csr_map of the incidences 3 e + a by the row of their vertex (eq: equation of every node, -1: prescribed).
+static void incidence_map(int nel, int neq, const int *ien, const std::vector<int> &eq, std::vector<int> &ptr,
+                          std::vector<int> &src, std::vector<int> &dst)
 {
-    std::vector<int> key(static_cast<size_t>(n));
-    for (int i = 0; i < n; ++i) key[i] = ptr[i] < ptr[i + 1] ? src[ptr[i]] : INT32_MAX;
-    std::stable_sort(dst.begin(), dst.end(), [&](int a, int b) { return key[a] < key[b]; });
-    std::vector<int> p2(static_cast<size_t>(n) + 1, 0), s2;
-    s2.reserve(src.size());
-    for (int k = 0; k < n; ++k) {
-        s2.insert(s2.end(), src.begin() + ptr[dst[k]], src.begin() + ptr[dst[k] + 1]);
-        p2[k + 1] = static_cast<int>(s2.size());
+    const int n3 = 3 * nel;
+    std::vector<int> rank(static_cast<size_t>(neq), -1), fill(static_cast<size_t>(neq) + 1, 0);
+    dst.clear();
+    dst.reserve(static_cast<size_t>(neq));
+    for (int q = 0; q < n3; ++q) {
+        const int i = eq[ien[q]];
+        if (i < 0) continue;
+        if (rank[i] < 0) {
+            rank[i] = static_cast<int>(dst.size());
+            dst.push_back(i);
+        }
+        ++fill[rank[i] + 1];
     }
-    ptr.swap(p2);
-    src.swap(s2);
+    for (int i = 0; i < neq; ++i)
+        if (rank[i] < 0) dst.push_back(i);
+    for (int k = 0; k < neq; ++k) fill[k + 1] += fill[k];
+    ptr = fill;
+    src.resize(static_cast<size_t>(ptr[neq]));
+    for (int q = 0; q < n3; ++q)
+        if (const int i = eq[ien[q]]; i >= 0) src[fill[rank[i]]++] = q;
 }
 
 // A row's incidences 3 e + a in element order, from the equation of every node (-1: prescribed).
@@ -861,23 +870,31 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     if (lm) up(M->lm, lm, static_cast<size_t>(nel) * 3);
     // unknown -> element-vertex incidences in element order (Type-1 vertices only)
     std::vector<int> eq(static_cast<size_t>(nnodes)), rptr, rinc, rdst, ptr, src, dst;
-    for (int v = 0; v < nnodes; ++v) eq[v] = type[v] == 1 ? invP_id[v] : -1;
+    bool in_range = true;
+    for (int v = 0; v < nnodes; ++v) {
+        eq[v] = type[v] == 1 ? invP_id[v] : -1;
+        in_range = in_range && (type[v] != 1 || (eq[v] >= 0 && eq[v] < neq));
+    }
     const size_t n3 = static_cast<size_t>(nel) * 3;
-    for (size_t q = 0; q < n3; ++q)
+    for (size_t q = 0; q < n3 && !in_range; ++q)   // only the vertices of elements matter
         if (type[ien[q]] == 1 && (eq[ien[q]] < 0 || eq[ien[q]] >= neq)) rc = FEMGPU_ERR_ARG;
     if (rc == FEMGPU_ERR_ARG) set_error("femgpu_mesh_create: invP_id out of range");
-    if (rc == FEMGPU_OK) row_incidences(nel, neq, ien, eq, rptr, rinc);
     M->fz_state = -1;
     M->has_scheme = false;
     if (rc == FEMGPU_OK && scheme) {
         for (size_t q = 0; q < 3 * n3; ++q)
             if (scheme[q] < 0 || scheme[q] > nnz) rc = FEMGPU_ERR_ARG;
         if (rc == FEMGPU_ERR_ARG) set_error("femgpu_mesh_create: scheme slot out of range");
-        if (rc == FEMGPU_OK && one_off) M->fz_state = 0;
-        else if (rc == FEMGPU_OK) rc = build_fused_plan(M, ien, scheme, eq, rptr, rinc);
+        if (rc == FEMGPU_OK && one_off) {
+            M->fz_state = 0;
+        } else if (rc == FEMGPU_OK) {
+            row_incidences(nel, neq, ien, eq, rptr, rinc);
+            rc = build_fused_plan(M, ien, scheme, eq, rptr, rinc);
+        }
         M->has_scheme = rc == FEMGPU_OK;
         if (rc == FEMGPU_OK && M->fz_state != 1) {   // slot lists, where the fused assembly does not apply
             std::vector<std::pair<int, int>> pairs;
+            pairs.reserve(3 * n3);
             for (size_t q = 0; q < 3 * n3; ++q)
                 if (scheme[q] < nnz) pairs.emplace_back(scheme[q], static_cast<int>(q));
             csr_map(nnz, pairs, ptr, src, dst);
@@ -889,9 +906,12 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     if (rc == FEMGPU_OK) {
         // the right-hand side's lists, in order of first element where the gather is the only path (next to
         // the fused assembly it serves calls without CSR values: the rows' own order, not sorted)
-        rdst.resize(static_cast<size_t>(neq));
-        for (int i = 0; i < neq; ++i) rdst[i] = i;
-        if (M->fz_state != 1) order_lists(neq, rptr, rinc, rdst);
+        if (M->fz_state != 1) {
+            incidence_map(nel, neq, ien, eq, rptr, rinc, rdst);
+        } else {
+            rdst.resize(static_cast<size_t>(neq));
+            for (int i = 0; i < neq; ++i) rdst[i] = i;
+        }
         up(M->rhs_ptr, rptr.data(), rptr.size());
         up(M->rhs_src, rinc.data(), rinc.size());
         up(M->rhs_dst, rdst.data(), rdst.size());
