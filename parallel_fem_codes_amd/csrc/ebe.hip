@@ -626,7 +626,6 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
         }
     }
     const size_t nbslots = static_cast<size_t>(bptr[nslices]) * 64;
-    FG_CHECK(nbslots < static_cast<size_t>(INT_MAX) / 16, FEMGPU_ERR_ARG, "femgpu_ebe_create: operator too large");
     if (packed && maxblk > kFillBlocks) {   // nodes whose triangles do not share edges: unpack the positions
         std::vector<unsigned> s3(3 * nslots, ~0u);
         for (size_t q = 0; q < nslots; ++q)

@@ -65,3 +65,31 @@ def test_ebe_layouts(oracle, ndof, mesh):
         E.ebemv(torch.from_numpy(p).cuda().float(), q32)
         scale = oracle.ebemv_block(lm, np.abs(Ah), np.abs(p), neq, s)
         assert (np.abs(q32.cpu().numpy().astype(np.float64) - ref) <= 2.1 * 2.0 ** -24 * scale + 1e-300).all()
+
+
+def test_ebe_many_block_rows():
+    """2 048 hubs of 1 024 triangles: 140 million slots of block rows (a slice is as long as its longest node)."""
+    import torch
+    hubs, deg = 2048, 1024
+    k = np.arange(deg)
+    one = np.stack([0 * k, 1 + k, 1 + (k + 1) % deg], 1)
+    lm = ((deg + 1) * np.arange(hubs)[:, None, None] + one).astype(np.int32)
+    neq = hubs * (deg + 1)
+    rng = np.random.default_rng(1)
+    A = rng.standard_normal((hubs * deg, 3, 3))
+    p = rng.standard_normal(neq).astype(np.float32).astype(np.float64)
+    E = fem.EbeMatrix(fem.Device(0), lm.ravel(), 3, neq)
+    E.set_values(torch.from_numpy(A).cuda())
+    tri = lm.reshape(-1, 3)
+
+    def product(A, p):
+        return np.bincount(tri.ravel(), weights=(A * p[tri][:, None, :]).sum(2).ravel(), minlength=neq)
+
+    ref, scale = product(A, p), product(np.abs(A), np.abs(p))
+    q = torch.full((neq,), float("nan"), dtype=torch.float32, device="cuda")
+    E.ebemv(torch.from_numpy(p).cuda().float(), q)
+    assert (np.abs(q.cpu().numpy() - ref) <= 2.1 * 2.0 ** -24 * scale).all()
+    q = torch.full((neq,), float("nan"), dtype=torch.float64, device="cuda")
+    E.ebemv(torch.from_numpy(p).cuda(), q)
+    # sums of 3 * 1024 terms in two orders
+    assert (np.abs(q.cpu().numpy() - ref) <= 3 * deg * 2.0 ** -52 * scale).all()
