@@ -13,6 +13,7 @@
 // load of a wavefront is one contiguous run; the element rows of prescribed dofs are not stored.
 // Columns are kept as int16 offsets from the node's first unknown when the mesh numbering allows
 // (2 bytes per entry), else as int32 unknowns.
+#include <atomic>
 #include <climits>
 #include <vector>
 
@@ -542,89 +543,127 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     const size_t nslots = static_cast<size_t>(nrows) * 64;
     FG_CHECK(nslots * s * nd < (size_t{1} << 40) && nslots < static_cast<size_t>(INT_MAX), FEMGPU_ERR_ARG,
              "femgpu_ebe_create: operator too large");
+    // The passes below are independent from slice to slice and run on several host threads: they are most of
+    // the time of a creation (800 x 400 squares, ndof = 4: 59 ms on one thread, 31 on eight).
+    constexpr size_t kElems = 1 << 13, kSlices = 1 << 6;   // least pieces worth a thread
     // columns as 16-bit offsets from the node's first unknown where every one fits
-    bool fits16 = true;
-    for (size_t ea = 0; ea < kinc.size() && fits16; ++ea) {
-        if (kinc[ea] < 0) continue;
-        const int *L = lm + ea / 3 * s;
-        for (int b = 0; b < s; ++b) {
-            const long dlt = static_cast<long>(L[b]) - kinc[ea];
-            fits16 = fits16 && (L[b] >= NEQ || (dlt >= -32767 && dlt <= 32767));
-        }
-    }
-    std::vector<int> src(nslots, -1), c32(fits16 ? 0 : nslots * s, NEQ);
-    std::vector<short> c16(fits16 ? nslots * s : 0, kSink16);
-    for (int g = 0; g < ng; ++g) {
-        const int sl = g >> 6, l = g & 63;
-        for (int j = 0; j < len[g]; ++j) {
-            const int ea = inc[gptr[g] + j], e = ea / 3, a = ea % 3;
-            const size_t r = static_cast<size_t>(iptr[sl] + j);
-            src[r * 64 + l] = e * s * s + nd * a * s;
-            for (int b = 0; b < s; ++b) {
-                const int c = lm[static_cast<size_t>(e) * s + b];
-                if (c >= NEQ) continue;
-                if (fits16) c16[(r * s + b) * 64 + l] = static_cast<short>(c - gkey[g]);
-                else c32[(r * s + b) * 64 + l] = c;
+    std::atomic<bool> fits{true};
+    host_pieces(static_cast<size_t>(nel), kElems, [&](size_t e0, size_t e1) {
+        bool ok = true;
+        for (size_t e = e0; e < e1 && ok; ++e) {
+            const int *L = lm + e * s;
+            int lo = INT_MAX, hi = -1;   // the element's unknowns
+            for (int b = 0; b < s; ++b)
+                if (L[b] < NEQ) {
+                    lo = std::min(lo, L[b]);
+                    hi = std::max(hi, L[b]);
+                }
+            for (int a = 0; a < 3; ++a) {
+                const int k = kinc[3 * e + a];
+                ok = ok && (k < 0 || (static_cast<long>(lo) - k >= -32767 && static_cast<long>(hi) - k <= 32767));
             }
         }
-    }
+        if (!ok) fits = false;
+    });
+    const bool fits16 = fits;
+    std::vector<int> src(nslots, -1), c32(fits16 ? 0 : nslots * s, NEQ);
+    std::vector<short> c16(fits16 ? nslots * s : 0, kSink16);
+    host_pieces(static_cast<size_t>(nslices), kSlices, [&](size_t s0, size_t s1) {
+        for (int g = static_cast<int>(64 * s0); g < std::min(ng, static_cast<int>(64 * s1)); ++g) {
+            const int sl = g >> 6, l = g & 63, key = gkey[g];
+            for (int j = 0; j < len[g]; ++j) {
+                const int ea = inc[gptr[g] + j], e = ea / 3, a = ea % 3;
+                const size_t r = static_cast<size_t>(iptr[sl] + j);
+                src[r * 64 + l] = e * s * s + nd * a * s;
+                const int *L = lm + static_cast<size_t>(e) * s;
+                if (fits16) {
+                    short *o = c16.data() + r * s * 64 + l;
+                    for (int b = 0; b < s; ++b) o[b * 64] = L[b] < NEQ ? static_cast<short>(L[b] - key) : kSink16;
+                } else {
+                    int *o = c32.data() + r * s * 64 + l;
+                    for (int b = 0; b < s; ++b) o[b * 64] = L[b];
+                }
+            }
+        }
+    });
     // node block rows of the FP32 product: per group its column nodes (groups) in order of appearance, and
     // the position of each incidence's three column nodes among them (three 8-bit positions per incidence,
     // or one word each where a node has too many column nodes)
-    std::vector<int> bptr(static_cast<size_t>(nslices) + 1, 0), blen(ng, 0), cols(static_cast<size_t>(64) * 3 * maxinc);
-    std::vector<int> b32;
-    std::vector<short> b16;
-    const size_t guess = (static_cast<size_t>(nrows) + 2 * nslices) * 64 * nd;
-    if (fits16) b16.reserve(guess);
-    else b32.reserve(guess);
-    int maxblk = 0;
+    std::vector<int> bptr(static_cast<size_t>(nslices) + 1, 0), blen(ng, 0);
     const bool packed = maxinc < kFillBlocks;   // n triangles around a node have n + 1 column nodes
     bool wide = !packed;
     std::vector<unsigned> slots(packed ? nslots : 3 * nslots, ~0u);
+    const auto set_slot = [&](size_t q, int a, int at) {
+        if (packed) slots[q] = (slots[q] & ~(255u << (8 * a))) | (static_cast<unsigned>(at) << (8 * a));
+        else slots[3 * q + a] = static_cast<unsigned>(at);
+    };
+    std::vector<int> pos(packed ? 0 : static_cast<size_t>(NEQ), -1);   // hubs: a column node's position by its key
+    const auto block_cols = [&](size_t s0, size_t s1) {
+        int cs[3 * kFillBlocks];
+        for (size_t sl = s0; sl < s1; ++sl) {
+            int w = 0;
+            for (int g = static_cast<int>(64 * sl); g < std::min(ng, static_cast<int>(64 * sl) + 64); ++g) {
+                int nc = 0;
+                for (int j = 0; j < len[g]; ++j) {
+                    const int ea = inc[gptr[g] + j], e3 = ea - ea % 3;
+                    const size_t q = static_cast<size_t>(iptr[sl] + j) * 64 + (g & 63);
+                    for (int a = 0; a < 3; ++a) {
+                        const int k = kinc[e3 + a];
+                        if (k < 0) continue;
+                        int at = 0;
+                        if (packed) {
+                            while (at < nc && cs[at] != k) ++at;
+                            if (at == nc) cs[nc++] = k;
+                        } else {
+                            if (pos[k] < 0) pos[k] = nc++;
+                            at = pos[k];
+                        }
+                        set_slot(q, a, at);
+                    }
+                }
+                if (!packed)
+                    for (int j = 0; j < len[g]; ++j)
+                        for (int ea = inc[gptr[g] + j], a = 0; a < 3; ++a)
+                            if (const int k = kinc[ea - ea % 3 + a]; k >= 0) pos[k] = -1;
+                blen[g] = nc;
+                w = std::max(w, nc);
+            }
+            bptr[sl + 1] = w;
+        }
+    };
+    if (packed) host_pieces(static_cast<size_t>(nslices), kSlices, block_cols);
+    else block_cols(0, static_cast<size_t>(nslices));
+    int maxblk = 0;
     for (int sl = 0; sl < nslices; ++sl) {
-        int w = 0;
-        const int g1 = std::min(ng, 64 * sl + 64);
-        for (int g = 64 * sl; g < g1; ++g) {
-            const int l = g & 63;
-            int *cs = cols.data() + static_cast<size_t>(l) * 3 * maxinc, nc = 0;
-            for (int j = 0; j < len[g]; ++j) {
-                const int ea = inc[gptr[g] + j], e3 = ea - ea % 3;
-                const size_t q = static_cast<size_t>(iptr[sl] + j) * 64 + l;
-                unsigned code = ~0u;
-                for (int a = 0; a < 3; ++a) {
-                    const int k = kinc[e3 + a];
-                    if (k < 0) continue;
-                    int at = 0;
-                    while (at < nc && cs[at] != k) ++at;
-                    if (at == nc) cs[nc++] = k;
-                    if (packed) code = (code & ~(255u << (8 * a))) | (static_cast<unsigned>(at) << (8 * a));
-                    else slots[3 * q + a] = static_cast<unsigned>(at);
-                }
-                if (packed) slots[q] = code;
-            }
-            blen[g] = nc;
-            w = std::max(w, nc);
-        }
-        bptr[sl + 1] = bptr[sl] + w;
-        maxblk = std::max(maxblk, w);
-        const size_t first = static_cast<size_t>(bptr[sl]) * 64 * nd, end = static_cast<size_t>(bptr[sl + 1]) * 64 * nd;
-        if (fits16) b16.resize(end, kSink16);
-        else b32.resize(end, NEQ);
-        for (int g = 64 * sl; g < g1; ++g) {
-            const int l = g & 63, *cs = cols.data() + static_cast<size_t>(l) * 3 * maxinc;
-            for (int j = 0; j < blen[g]; ++j) {
-                const int cg = gid[cs[j]];
-                const int *ce = eq.data() + static_cast<size_t>(cg >> 6) * nd * 64 + (cg & 63);
-                for (int d = 0; d < nd; ++d) {
-                    const int c = ce[d * 64];
-                    if (c >= NEQ) continue;
-                    const size_t at = first + (static_cast<size_t>(j) * 64 + l) * nd + d;
-                    if (fits16) b16[at] = static_cast<short>(c - gkey[g]);
-                    else b32[at] = c;
-                }
-            }
-        }
+        maxblk = std::max(maxblk, bptr[sl + 1]);
+        bptr[sl + 1] += bptr[sl];
     }
+    // their columns, at the first incidence that has the node
+    const size_t ncols = static_cast<size_t>(bptr[nslices]) * 64 * nd;
+    std::vector<int> b32(fits16 ? 0 : ncols, NEQ);
+    std::vector<short> b16(fits16 ? ncols : 0, kSink16);
+    host_pieces(static_cast<size_t>(nslices), kSlices, [&](size_t s0, size_t s1) {
+        for (int g = static_cast<int>(64 * s0); g < std::min(ng, static_cast<int>(64 * s1)); ++g) {
+            const int sl = g >> 6, l = g & 63;
+            int seen = 0;
+            for (int j = 0; j < len[g] && seen < blen[g]; ++j) {
+                const int ea = inc[gptr[g] + j];
+                const size_t q = static_cast<size_t>(iptr[sl] + j) * 64 + l;
+                for (int a = 0; a < 3; ++a) {
+                    const unsigned at = packed ? (slots[q] >> (8 * a)) & 255u : slots[3 * q + a];
+                    if (at != static_cast<unsigned>(seen)) continue;   // seen before, or without unknowns
+                    ++seen;
+                    const int *L = lm + static_cast<size_t>(ea / 3) * s + nd * a;
+                    const size_t o = ((static_cast<size_t>(bptr[sl]) + at) * 64 + l) * nd;
+                    for (int d = 0; d < nd; ++d) {
+                        if (L[d] >= NEQ) continue;
+                        if (fits16) b16[o + d] = static_cast<short>(L[d] - gkey[g]);
+                        else b32[o + d] = L[d];
+                    }
+                }
+            }
+        }
+    });
     const size_t nbslots = static_cast<size_t>(bptr[nslices]) * 64;
     if (packed && maxblk > kFillBlocks) {   // nodes whose triangles do not share edges: unpack the positions
         std::vector<unsigned> s3(3 * nslots, ~0u);
