@@ -341,8 +341,9 @@ struct femgpu_ebe {
     fg::DevBuf<int> blen;           // group -> column nodes
     fg::DevBuf<short> bcol16;       // (block row*64 + lane)*ndof + dof: columns, as col16v
     fg::DevBuf<int> bcol32;         // or as col32v
-    fg::DevBuf<unsigned> slots;     // incidence slot -> block rows of its three column nodes (8 bits each, 255
-                                    // none; three words per incidence with wide_slots)
+    fg::DevBuf<unsigned> slots;     // incidence slot -> block rows of its three column nodes (8 bits each, 255 none)
+    fg::DevBuf<int> wptr, wsrc;     // with wide_slots instead: block slot -> its element blocks, 3 * incidence row +
+                                    // vertex, in element order
     fg::DevBuf<float> val32;
     bool has_values = false;
 };

@@ -341,27 +341,26 @@ __global__ __launch_bounds__(64) void k_ebe_fill(const int *__restrict__ iptr, c
 }
 
 // The FP32 node block rows from the gathered FP64 rows, a thread per (block row, lane, dof row), for
-// operators with a node of more than kFillBlocks column nodes.
+// operators with a node of more than kFillBlocks column nodes: block slot q sums the element blocks
+// wsrc[wptr[q] .. wptr[q + 1]) = 3 * incidence row + vertex, in element order. (A search of the node's incidences
+// by every block row takes quadratic time at a hub.)
 template <int ND>
-__global__ __launch_bounds__(256) void k_node_rows_fill(const int *__restrict__ iptr, const int *__restrict__ bptr,
-                                                        const int *__restrict__ src,
-                                                        const unsigned *__restrict__ slots,
-                                                        const double *__restrict__ val, float *__restrict__ val32)
+__global__ __launch_bounds__(256) void k_node_rows_fill(const int *__restrict__ bptr, const int *__restrict__ wptr,
+                                                        const int *__restrict__ wsrc, const double *__restrict__ val,
+                                                        float *__restrict__ val32)
 {
     constexpr int S = 3 * ND;
     const int sl = blockIdx.x / ND, d = blockIdx.x % ND, l = threadIdx.x & 63;
     for (int j = bptr[sl] + static_cast<int>(threadIdx.x >> 6); j < bptr[sl + 1]; j += 4) {
+        const size_t q = static_cast<size_t>(j) * 64 + l;
         double acc[ND];
 #pragma unroll
         for (int c = 0; c < ND; ++c) acc[c] = 0.0;
-        for (int r = iptr[sl]; r < iptr[sl + 1]; ++r) {
-            if (src[r * 64 + l] < 0) continue;
-            for (int a = 0; a < 3; ++a) {
-                const unsigned s = slots[(static_cast<size_t>(r) * 64 + l) * 3 + a];
-                if (s != static_cast<unsigned>(j - bptr[sl])) continue;
+        for (int k = wptr[q]; k < wptr[q + 1]; ++k) {
+            const int r = wsrc[k] / 3, a = wsrc[k] % 3;
+            const double *v = val + ((static_cast<size_t>(r) * ND + d) * S + ND * a) * 64 + l;
 #pragma unroll
-                for (int c = 0; c < ND; ++c) acc[c] += val[((static_cast<size_t>(r) * ND + d) * S + ND * a + c) * 64 + l];
-            }
+            for (int c = 0; c < ND; ++c) acc[c] += v[c * 64];
         }
 #pragma unroll
         for (int c = 0; c < ND; ++c)
@@ -464,7 +463,7 @@ static int fill_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const double *Ae)
     } else {
         k_ebe_fill<ND, RB, false><<<grid, 64, turn, ctx->stream>>>(E->iptr.p, nullptr, E->src.p, nullptr, Ae, E->val.p, nullptr);
         FG_HIP(hipGetLastError());
-        k_node_rows_fill<ND><<<grid, 256, 0, ctx->stream>>>(E->iptr.p, E->bptr.p, E->src.p, E->slots.p, E->val.p, E->val32.p);
+        k_node_rows_fill<ND><<<grid, 256, 0, ctx->stream>>>(E->bptr.p, E->wptr.p, E->wsrc.p, E->val.p, E->val32.p);
     }
     FG_HIP(hipGetLastError());
     return FEMGPU_OK;
@@ -591,7 +590,6 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     // or one word each where a node has too many column nodes)
     std::vector<int> bptr(static_cast<size_t>(nslices) + 1, 0), blen(ng, 0);
     const bool packed = maxinc < kFillBlocks;   // n triangles around a node have n + 1 column nodes
-    bool wide = !packed;
     std::vector<unsigned> slots(packed ? nslots : 3 * nslots, ~0u);
     const auto set_slot = [&](size_t q, int a, int at) {
         if (packed) slots[q] = (slots[q] & ~(255u << (8 * a))) | (static_cast<unsigned>(at) << (8 * a));
@@ -665,15 +663,28 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
         }
     });
     const size_t nbslots = static_cast<size_t>(bptr[nslices]) * 64;
-    if (packed && maxblk > kFillBlocks) {   // nodes whose triangles do not share edges: unpack the positions
-        std::vector<unsigned> s3(3 * nslots, ~0u);
-        for (size_t q = 0; q < nslots; ++q)
-            for (int a = 0; a < 3; ++a) {
-                const unsigned at = (slots[q] >> (8 * a)) & 255u;
-                if (at != 255u) s3[3 * q + a] = at;
-            }
-        slots.swap(s3);
-        wide = true;
+    // a node with too many column nodes for the fill kernel's LDS: the element blocks of every block slot instead
+    const bool wide = !packed || maxblk > kFillBlocks;
+    std::vector<int> wptr, wsrc;
+    if (wide) {
+        const auto each_block = [&](const auto &f) {   // f(block slot, 3 * incidence row + vertex), in element order
+            for (int g = 0; g < ng; ++g)
+                for (int j = 0; j < len[g]; ++j) {
+                    const size_t r = static_cast<size_t>(iptr[g >> 6] + j), q = r * 64 + (g & 63);
+                    for (int a = 0; a < 3; ++a) {
+                        const unsigned at = packed ? (slots[q] >> (8 * a)) & 255u : slots[3 * q + a];
+                        if (at != (packed ? 255u : ~0u))
+                            f((static_cast<size_t>(bptr[g >> 6]) + at) * 64 + (g & 63), static_cast<int>(3 * r) + a);
+                    }
+                }
+        };
+        wptr.assign(nbslots + 1, 0);
+        each_block([&](size_t q, int) { ++wptr[q + 1]; });
+        for (size_t q = 0; q < nbslots; ++q) wptr[q + 1] += wptr[q];
+        wsrc.resize(static_cast<size_t>(wptr[nbslots]));
+        each_block([&](size_t q, int ra) { wsrc[wptr[q]++] = ra; });
+        for (size_t q = nbslots; q > 0; --q) wptr[q] = wptr[q - 1];
+        wptr[0] = 0;
     }
     auto *E = new femgpu_ebe();
     E->ctx = ctx;
@@ -704,7 +715,9 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     if (!rc) rc = E->blen.upload(blen.data(), blen.size(), st);
     if (!rc && fits16) rc = E->bcol16.upload(b16.data(), b16.size(), st);
     if (!rc && !fits16) rc = E->bcol32.upload(b32.data(), b32.size(), st);
-    if (!rc) rc = E->slots.upload(slots.data(), slots.size(), st);
+    if (!rc && !wide) rc = E->slots.upload(slots.data(), slots.size(), st);
+    if (!rc && wide) rc = E->wptr.upload(wptr.data(), wptr.size(), st);
+    if (!rc && wide) rc = E->wsrc.upload(wsrc.data(), wsrc.size(), st);
     if (!rc) rc = E->val32.alloc(nbslots * nd * nd);
     if (!rc && hipStreamSynchronize(st) != hipSuccess) rc = FEMGPU_ERR_HIP;   // host arrays end here
     if (rc) {

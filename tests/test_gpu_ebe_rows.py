@@ -31,7 +31,7 @@ def delaunay(n):
 
 
 @pytest.mark.parametrize("ndof", [1, 3, 4])
-@pytest.mark.parametrize("mesh", ["strip31", "strip32", "delaunay300", "fan22", "fan23", "fan24", "fan70", "bowties11",
+@pytest.mark.parametrize("mesh", ["strip31", "strip32", "delaunay300", "fan22", "fan23", "fan24", "fan70", "fan20000", "bowties11",
                                   "bowties13", "bowties90", "spread", "strip20000"])
 def test_ebe_layouts(oracle, ndof, mesh):
     import torch
