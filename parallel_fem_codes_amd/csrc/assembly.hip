@@ -8,7 +8,9 @@
 // with no atomics. Contraction is off in this file: the element arithmetic follows the
 // reference's expression order operation for operation.
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "common.h"
@@ -604,9 +606,14 @@ void csr_map(int nkeys, const std::vector<std::pair<int, int>> &pairs, std::vect
     for (auto &p : pairs) src[fill[rank[p.first]]++] = p.second;
 }
 
-// csr_map of the incidences 3 e + a by the row of their vertex (eq: equation of every node, -1: prescribed).
+struct RowList {
+    int first, end;
+};
+
+// csr_map of the incidences 3 e + a by the row of their vertex (eq: equation of every node, -1: prescribed);
+// rows: each row's part of src, its incidences in element order.
 static void incidence_map(int nel, int neq, const int *ien, const std::vector<int> &eq, std::vector<int> &ptr,
-                          std::vector<int> &src, std::vector<int> &dst)
+                          std::vector<int> &src, std::vector<int> &dst, std::vector<RowList> &rows)
 {
     const int n3 = 3 * nel;
     std::vector<int> rank(static_cast<size_t>(neq), -1), fill(static_cast<size_t>(neq) + 1, 0);
@@ -625,61 +632,62 @@ static void incidence_map(int nel, int neq, const int *ien, const std::vector<in
         if (rank[i] < 0) dst.push_back(i);
     for (int k = 0; k < neq; ++k) fill[k + 1] += fill[k];
     ptr = fill;
+    rows.resize(static_cast<size_t>(neq));
+    for (int k = 0; k < neq; ++k) rows[dst[k]] = {ptr[k], ptr[k + 1]};
     src.resize(static_cast<size_t>(ptr[neq]));
     for (int q = 0; q < n3; ++q)
         if (const int i = eq[ien[q]]; i >= 0) src[fill[rank[i]]++] = q;
 }
 
-// A row's incidences 3 e + a in element order, from the equation of every node (-1: prescribed).
-static void row_incidences(int nel, int neq, const int *ien, const std::vector<int> &eq, std::vector<int> &rptr,
-                           std::vector<int> &rinc)
-{
-    const size_t n3 = static_cast<size_t>(nel) * 3;
-    rptr.assign(static_cast<size_t>(neq) + 1, 0);
-    for (size_t q = 0; q < n3; ++q)
-        if (eq[ien[q]] >= 0) ++rptr[eq[ien[q]] + 1];
-    for (int i = 0; i < neq; ++i) rptr[i + 1] += rptr[i];
-    rinc.resize(static_cast<size_t>(rptr[neq]));
-    std::vector<int> fill(rptr.begin(), rptr.end() - 1);
-    for (size_t q = 0; q < n3; ++q)
-        if (eq[ien[q]] >= 0) rinc[fill[eq[ien[q]]]++] = static_cast<int>(q);
-}
+constexpr size_t kPlanPiece = 1 << 13;   // least rows or elements worth a host thread
 
 // The fused assembly's plan from the mesh's host arrays: rows grouped into compact patches by
 // breadth-first growth over the mesh graph (up to kFzRows rows and kFzMaxSlots incidences), each
 // patch's elements in order of first touch, its incidences numbered row by row as LDS slots. eq:
-// equation of every node (-1: prescribed); rptr, rinc: a row's incidences 3 e + a in element order. fz_state 1 when every
+// equation of every node (-1: prescribed); rows, rinc: a row's incidences 3 e + a in element order. fz_state 1 when every
 // slot of the CSR values is an entry of exactly one row (its slots contiguous, the three of an element
 // row distinct), rows have at most 15 entries and 16 incidences, and no prescribed row has slots; else
 // -1, and the assembly takes the slot lists.
 static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, const std::vector<int> &eq,
-                            const std::vector<int> &rptr, const std::vector<int> &rinc)
+                            const std::vector<RowList> &rows, const std::vector<int> &rinc)
 {
     M->fz_state = -1;
     const int nel = M->nel, neq = M->neq, nnz = M->nnz;
     if (neq == 0 || nel == 0 || nnz == 0) return FEMGPU_OK;
     hipStream_t st = M->ctx->stream;
     int ki = 0;
-    for (int i = 0; i < neq; ++i) ki = std::max(ki, rptr[i + 1] - rptr[i]);
+    for (int i = 0; i < neq; ++i) ki = std::max(ki, rows[i].end - rows[i].first);
     if (ki > kFzMaxInc) return FEMGPU_OK;
     // every row's first and last CSR slot
-    std::vector<int> rfirst(neq, INT32_MAX), rlast(neq, -1);
-    for (size_t ea = 0; ea < static_cast<size_t>(nel) * 3; ++ea) {
-        const int i = eq[ien[ea]], *sc = scheme + 3 * ea;
-        if (i < 0) {
-            if (sc[0] < nnz || sc[1] < nnz || sc[2] < nnz) return FEMGPU_OK;
-            continue;
+    std::vector<int> rfirst(neq), rlast(neq);
+    std::atomic<bool> plain{true};   // no slots in prescribed rows, an element row's slots distinct
+    host_pieces(static_cast<size_t>(neq), kPlanPiece, [&](size_t i0, size_t i1) {
+        bool ok = true;
+        for (size_t i = i0; i < i1; ++i) {
+            int lo = INT32_MAX, hi = -1;
+            for (int q = rows[i].first; q < rows[i].end; ++q) {
+                const int *sc = scheme + 3 * static_cast<size_t>(rinc[q]);
+                for (int b = 0; b < 3; ++b) {
+                    if (sc[b] >= nnz) continue;
+                    ok = ok && sc[b] != sc[(b + 1) % 3];
+                    lo = std::min(lo, sc[b]);
+                    hi = std::max(hi, sc[b]);
+                }
+            }
+            rfirst[i] = lo;
+            rlast[i] = hi;
         }
-        int lo = rfirst[i], hi = rlast[i];
-        for (int b = 0; b < 3; ++b) {
-            if (sc[b] >= nnz) continue;
-            if (sc[b] == sc[(b + 1) % 3]) return FEMGPU_OK;
-            lo = std::min(lo, sc[b]);
-            hi = std::max(hi, sc[b]);
+        if (!ok) plain = false;
+    });
+    host_pieces(static_cast<size_t>(nel), kPlanPiece, [&](size_t e0, size_t e1) {
+        bool ok = true;
+        for (size_t ea = 3 * e0; ea < 3 * e1; ++ea) {
+            const int *sc = scheme + 3 * ea;
+            ok = ok && (eq[ien[ea]] >= 0 || (sc[0] >= nnz && sc[1] >= nnz && sc[2] >= nnz));
         }
-        rfirst[i] = lo;
-        rlast[i] = hi;
-    }
+        if (!ok) plain = false;
+    });
+    if (!plain) return FEMGPU_OK;
     int maxlen = 0;
     long long covered = 0;
     std::vector<char> seen(static_cast<size_t>(nnz), 0);
@@ -699,18 +707,18 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     for (int seed = 0; seed < neq; ++seed) {
         if (blk[seed] >= 0) continue;
         const int b = static_cast<int>(bptr.size()) - 1;
-        int tail = nord + 1, slots = rptr[seed + 1] - rptr[seed];   // order[nord ..] doubles as the queue
+        int tail = nord + 1, slots = rows[seed].end - rows[seed].first;   // order[nord ..] doubles as the queue
         const int full = nord + kFzRows;
         order[nord] = seed;
         blk[seed] = b;
         for (int h = nord; h < tail; ++h) {
             const int i = order[h];
-            for (int q = rptr[i]; q < rptr[i + 1] && tail < full; ++q) {
+            for (int q = rows[i].first; q < rows[i].end && tail < full; ++q) {
                 const int *v = ien + 3 * static_cast<size_t>(rinc[q] / 3);
                 for (int c = 0; c < 3 && tail < full; ++c) {
                     const int j = eq[v[c]];
                     if (j < 0 || blk[j] >= 0) continue;
-                    const int sj = rptr[j + 1] - rptr[j];
+                    const int sj = rows[j].end - rows[j].first;
                     if (slots + sj > kFzMaxSlots) continue;
                     blk[j] = b;
                     order[tail++] = j;
@@ -722,57 +730,83 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
         bptr.push_back(nord);
     }
     const int nb = static_cast<int>(bptr.size()) - 1;
-    std::vector<int> eptr(static_cast<size_t>(nb) + 1, 0);
-    std::vector<int4> ent;
-    ent.reserve(static_cast<size_t>(nel) * 5 / 2 + 16);
-    // every block's incidence codes: ki rows of kFzRows (padding 0xffffffff)
-    std::vector<unsigned> inc(static_cast<size_t>(nb) * ki * kFzRows, 0xffffffffu);
+    // The blocks are independent and planned on several host threads (creating a mesh of 641 x 502 nodes:
+    // 39 ms, 64 on one thread; of 301 x 262 nodes 7.5, where slot lists take 5.5). An element belongs
+    // to the blocks of its rows, at the place of its first row there.
+    std::vector<int> eptr(static_cast<size_t>(nb) + 1, 0), at(static_cast<size_t>(neq)), slots(static_cast<size_t>(nb), 0);
+    std::vector<int> place(static_cast<size_t>(M->nnodes), -1);   // node -> place of its row in order (-1: prescribed)
+    for (int h = 0; h < neq; ++h) at[order[h]] = h;
+    for (int v = 0; v < M->nnodes; ++v)
+        if (eq[v] >= 0 && eq[v] < neq) place[v] = at[eq[v]];
+    // every block's incidence codes: ki rows of kFzRows (padding 0xffffffff). The large arrays are first touched by
+    // the threads that fill them.
+    const size_t ninc = static_cast<size_t>(nb) * ki * kFzRows;
+    std::unique_ptr<unsigned[]> inc(new unsigned[ninc]);
     std::vector<int4> rinfo(static_cast<size_t>(nb) * kFzRows, make_int4(-1, 0, 0, 0));
-    std::vector<unsigned short> qof(static_cast<size_t>(nel) * 3, 0);   // LDS slot of a vertex row in its row's block
-    std::vector<int> mark(static_cast<size_t>(nel), -1), touched;
+    // LDS slot of a vertex row in its row's block, kFirst: the element's first row there
+    constexpr unsigned kFirst = 0x8000u;
+    static_assert(kFzMaxSlots + 3 * kFzMaxInc < static_cast<int>(kFirst), "a slot and the mark in 16 bits");
+    std::unique_ptr<unsigned short[]> qof(new unsigned short[static_cast<size_t>(nel) * 3]);
+    constexpr size_t kBlocks = 64;   // least blocks worth a thread
+    host_pieces(static_cast<size_t>(nb), kBlocks, [&](size_t b0, size_t b1) {
+        for (int b = static_cast<int>(b0); b < static_cast<int>(b1); ++b) {
+            const int r0 = bptr[b], nr = bptr[b + 1] - r0;
+            const size_t base = static_cast<size_t>(b) * ki * kFzRows;
+            int nslot = 0, ne = 0;
+            std::fill(inc.get() + base, inc.get() + base + static_cast<size_t>(ki) * kFzRows, 0xffffffffu);
+            for (int t = 0; t < nr; ++t) {
+                const int i = order[r0 + t], rf = rfirst[i];
+                unsigned *ic = inc.get() + base + t;
+                for (int q = rows[i].first; q < rows[i].end; ++q, ic += kFzRows) {
+                    const int ea = rinc[q], a = ea % 3, *v = ien + (ea - a), *sc = scheme + 3 * static_cast<size_t>(ea);
+                    bool first = true;
+                    for (int c = 0; c < 3; ++c) {
+                        const int h = place[v[c]];
+                        first = first && !(h >= r0 && (h < r0 + t || (h == r0 + t && c < a)));
+                    }
+                    unsigned code = static_cast<unsigned>(nslot);
+                    for (int c = 0; c < 3; ++c)
+                        code |= (sc[c] < nnz ? static_cast<unsigned>(sc[c] - rf) : 15u) << (16 + 4 * c);
+                    *ic = code;
+                    qof[ea] = static_cast<unsigned short>(static_cast<unsigned>(nslot++) | (first ? kFirst : 0u));
+                    ne += first;
+                }
+                rinfo[static_cast<size_t>(b) * kFzRows + t] = make_int4(i, rf, rlast[i] - rf + 1, rows[i].end - rows[i].first);
+            }
+            slots[b] = nslot;
+            eptr[b + 1] = ne;
+        }
+    });
     int slots_max = 0;
     for (int b = 0; b < nb; ++b) {
-        const int r0 = bptr[b], nr = bptr[b + 1] - r0;
-        const size_t base = static_cast<size_t>(b) * ki * kFzRows;
-        int nslot = 0;
-        touched.clear();
-        for (int t = 0; t < nr; ++t) {
-            const int i = order[r0 + t], rf = rfirst[i];
-            unsigned *ic = inc.data() + base + t;
-            for (int q = rptr[i]; q < rptr[i + 1]; ++q, ic += kFzRows) {
-                const int ea = rinc[q], e = ea / 3, *sc = scheme + 3 * static_cast<size_t>(ea);
-                unsigned code = static_cast<unsigned>(nslot);
-                for (int c = 0; c < 3; ++c)
-                    code |= (sc[c] < nnz ? static_cast<unsigned>(sc[c] - rf) : 15u) << (16 + 4 * c);
-                *ic = code;
-                qof[ea] = static_cast<unsigned short>(nslot++);
-                if (mark[e] != b) {
-                    mark[e] = b;
-                    touched.push_back(e);
-                }
-            }
-            rinfo[static_cast<size_t>(b) * kFzRows + t] = make_int4(i, rf, rlast[i] - rf + 1, rptr[i + 1] - rptr[i]);
-        }
-        slots_max = std::max(slots_max, nslot);
-        for (int e : touched) {
-            const size_t e3 = 3 * static_cast<size_t>(e);
-            int qn[3];
-            unsigned sl[3];
-            for (int a = 0; a < 3; ++a) {
-                qn[a] = eq[ien[e3 + a]];
-                sl[a] = qn[a] >= 0 && blk[qn[a]] == b ? qof[e3 + a] : 0xffffu;
-            }
-            ent.push_back(make_int4(ien[e3], ien[e3 + 1], ien[e3 + 2], qn[0]));
-            ent.push_back(make_int4(qn[1], qn[2], static_cast<int>(sl[0] | (sl[1] << 16)),
-                                    static_cast<int>(sl[2] | 0xffff0000u)));
-        }
-        eptr[b + 1] = static_cast<int>(ent.size() / 2);
+        slots_max = std::max(slots_max, slots[b]);
+        eptr[b + 1] += eptr[b];
     }
-    if (inc.empty()) inc.push_back(0xffffffffu);
-    if (ent.empty()) ent.push_back(make_int4(0, 0, 0, 0));
+    const size_t nent = 2 * static_cast<size_t>(eptr[nb]);
+    std::unique_ptr<int4[]> ent(new int4[nent]);
+    host_pieces(static_cast<size_t>(nb), kBlocks, [&](size_t b0, size_t b1) {
+        for (int b = static_cast<int>(b0); b < static_cast<int>(b1); ++b) {
+            int4 *o = ent.get() + 2 * static_cast<size_t>(eptr[b]);
+            for (int h = bptr[b]; h < bptr[b + 1]; ++h)
+                for (int q = rows[order[h]].first; q < rows[order[h]].end; ++q) {
+                    if (!(qof[rinc[q]] & kFirst)) continue;
+                    const int e3 = rinc[q] / 3 * 3;
+                    int qn[3];
+                    unsigned sl[3];
+                    for (int a = 0; a < 3; ++a) {
+                        qn[a] = eq[ien[e3 + a]];
+                        const int h2 = place[ien[e3 + a]];
+                        sl[a] = h2 >= bptr[b] && h2 < bptr[b + 1] ? qof[e3 + a] & (kFirst - 1u) : 0xffffu;
+                    }
+                    *o++ = make_int4(ien[e3], ien[e3 + 1], ien[e3 + 2], qn[0]);
+                    *o++ = make_int4(qn[1], qn[2], static_cast<int>(sl[0] | (sl[1] << 16)),
+                                     static_cast<int>(sl[2] | 0xffff0000u));
+                }
+        }
+    });
     FG_TRY(M->fz_eptr.upload(eptr.data(), eptr.size(), st));
-    FG_TRY(M->fz_ent.upload(ent.data(), ent.size(), st));
-    FG_TRY(M->fz_inc.upload(inc.data(), inc.size(), st));
+    FG_TRY(M->fz_ent.upload(ent.get(), nent, st));
+    FG_TRY(M->fz_inc.upload(inc.get(), ninc, st));
     FG_TRY(M->fz_row.upload(rinfo.data(), rinfo.size(), st));
     FG_HIP(hipStreamSynchronize(st));   // the host arrays end here
     M->fz_nblocks = nb;
@@ -791,7 +825,7 @@ static int fused_plan_from_lists(femgpu_mesh *M)
     const int nn = M->nnodes, nel = M->nel, neq = M->neq, nnz = M->nnz;
     if (neq == 0 || nel == 0 || nnz == 0) return FEMGPU_OK;
     hipStream_t st = M->ctx->stream;
-    std::vector<int> ien(static_cast<size_t>(nel) * 3), eq(nn), invP(nn), rptr(static_cast<size_t>(neq) + 1, 0);
+    std::vector<int> ien(static_cast<size_t>(nel) * 3), eq(nn), invP(nn), rptr, rinc, rdst;
     std::vector<int> aptr(static_cast<size_t>(nnz) + 1), adst(nnz);
     auto down = [&](auto &h, const auto &d) {
         return hipMemcpyAsync(h.data(), d.p, h.size() * sizeof(int), hipMemcpyDeviceToHost, st);
@@ -809,9 +843,9 @@ static int fused_plan_from_lists(femgpu_mesh *M)
     std::vector<int> scheme(static_cast<size_t>(nel) * 9, nnz);
     for (int k = 0; k < nnz; ++k)
         for (int q = aptr[k]; q < aptr[k + 1]; ++q) scheme[asrc[q]] = adst[k];
-    std::vector<int> rinc;
-    row_incidences(nel, neq, ien.data(), eq, rptr, rinc);
-    return build_fused_plan(M, ien.data(), scheme.data(), eq, rptr, rinc);
+    std::vector<RowList> rows;
+    incidence_map(nel, neq, ien.data(), eq, rptr, rinc, rdst, rows);
+    return build_fused_plan(M, ien.data(), scheme.data(), eq, rows, rinc);
 }
 
 template <bool STEADY>
@@ -870,6 +904,7 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     if (lm) up(M->lm, lm, static_cast<size_t>(nel) * 3);
     // unknown -> element-vertex incidences in element order (Type-1 vertices only)
     std::vector<int> eq(static_cast<size_t>(nnodes)), rptr, rinc, rdst, ptr, src, dst;
+    std::vector<RowList> rows;
     bool in_range = true;
     for (int v = 0; v < nnodes; ++v) {
         eq[v] = type[v] == 1 ? invP_id[v] : -1;
@@ -879,17 +914,27 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     for (size_t q = 0; q < n3 && !in_range; ++q)   // only the vertices of elements matter
         if (type[ien[q]] == 1 && (eq[ien[q]] < 0 || eq[ien[q]] >= neq)) rc = FEMGPU_ERR_ARG;
     if (rc == FEMGPU_ERR_ARG) set_error("femgpu_mesh_create: invP_id out of range");
+    if (rc == FEMGPU_OK) {
+        // the right-hand side's lists, next to the fused assembly too: it serves calls without CSR values, whose
+        // gather needs neighbouring threads on neighbouring elements (641 x 502 nodes with shock capture, element
+        // matrices and load 65 us, 94 with the rows in their own order)
+        incidence_map(nel, neq, ien, eq, rptr, rinc, rdst, rows);
+    }
     M->fz_state = -1;
     M->has_scheme = false;
     if (rc == FEMGPU_OK && scheme) {
-        for (size_t q = 0; q < 3 * n3; ++q)
-            if (scheme[q] < 0 || scheme[q] > nnz) rc = FEMGPU_ERR_ARG;
+        std::atomic<bool> slots_ok{true};
+        host_pieces(3 * n3, 9 * kPlanPiece, [&](size_t q0, size_t q1) {
+            bool ok = true;
+            for (size_t q = q0; q < q1; ++q) ok = ok && scheme[q] >= 0 && scheme[q] <= nnz;
+            if (!ok) slots_ok = false;
+        });
+        if (!slots_ok) rc = FEMGPU_ERR_ARG;
         if (rc == FEMGPU_ERR_ARG) set_error("femgpu_mesh_create: scheme slot out of range");
         if (rc == FEMGPU_OK && one_off) {
             M->fz_state = 0;
         } else if (rc == FEMGPU_OK) {
-            row_incidences(nel, neq, ien, eq, rptr, rinc);
-            rc = build_fused_plan(M, ien, scheme, eq, rptr, rinc);
+            rc = build_fused_plan(M, ien, scheme, eq, rows, rinc);
         }
         M->has_scheme = rc == FEMGPU_OK;
         if (rc == FEMGPU_OK && M->fz_state != 1) {   // slot lists, where the fused assembly does not apply
@@ -904,10 +949,6 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
         }
     }
     if (rc == FEMGPU_OK) {
-        // the right-hand side's lists, next to the fused assembly too: it serves calls without CSR values, whose
-        // gather needs neighbouring threads on neighbouring elements (641 x 502 nodes with shock capture, element
-        // matrices and load 65 us, 94 with the rows in their own order)
-        incidence_map(nel, neq, ien, eq, rptr, rinc, rdst);
         up(M->rhs_ptr, rptr.data(), rptr.size());
         up(M->rhs_src, rinc.data(), rinc.size());
         up(M->rhs_dst, rdst.data(), rdst.size());
