@@ -171,10 +171,10 @@ __global__ __launch_bounds__(256) void k_elem_ns(int nel, NsIn in, double *__res
 // per element written and read again took 112 us of device time at 257 x 257 nodes (135 us a call); this one takes 29, of which a
 // third is arithmetic and the rest waits in the chains node -> state -> element and pair -> codes -> slots.
 // Patches of 64, 128, 192 and 256 incidences: 29.1, 28.8, 28.5, 29.7 us.
-#ifndef NFT
-#define NFT 128
-#endif
-constexpr int kNfThreads = NFT, kNfSlot = 31;
+constexpr int kNfThreads = 128, kNfSlot = 31;
+// what the plan packs: a node's place in its patch in 8 bits, LDS offsets of contributions and a patch's first codes
+// (three per incidence) in 16
+static_assert(kNfThreads <= 256 && kNfSlot * kNfThreads <= 65536 && 3 * kNfThreads <= 65536, "packed fields of the plan");
 
 __global__ __launch_bounds__(kNfThreads) void k_ns_fused(int nblocks, NsIn in, const int4 *__restrict__ bptr,
                                                          const int4 *__restrict__ inc, const int4 *__restrict__ eqs,
