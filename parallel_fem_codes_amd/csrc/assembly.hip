@@ -639,7 +639,9 @@ static void incidence_map(int nel, int neq, const int *ien, const std::vector<in
         if (const int i = eq[ien[q]]; i >= 0) src[fill[rank[i]]++] = q;
 }
 
-constexpr size_t kPlanPiece = 1 << 13;   // least rows or elements worth a host thread
+// Least rows, elements (or entries of theirs) for a host thread of the planning passes: large meshes only. Below, a
+// thread that waits for a processor (4 ms beside a pool of threads that spin) would cost more than it saves.
+static size_t plan_piece(int nel) { return nel >= 1 << 18 ? 1 << 13 : SIZE_MAX; }
 
 // The fused assembly's plan from the mesh's host arrays: rows grouped into compact patches by
 // breadth-first growth over the mesh graph (up to kFzRows rows and kFzMaxSlots incidences), each
@@ -661,7 +663,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     // every row's first and last CSR slot
     std::vector<int> rfirst(neq), rlast(neq);
     std::atomic<bool> plain{true};   // no slots in prescribed rows, an element row's slots distinct
-    host_pieces(static_cast<size_t>(neq), kPlanPiece, [&](size_t i0, size_t i1) {
+    host_pieces(static_cast<size_t>(neq), plan_piece(nel), [&](size_t i0, size_t i1) {
         bool ok = true;
         for (size_t i = i0; i < i1; ++i) {
             int lo = INT32_MAX, hi = -1;
@@ -679,7 +681,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
         }
         if (!ok) plain = false;
     });
-    host_pieces(static_cast<size_t>(nel), kPlanPiece, [&](size_t e0, size_t e1) {
+    host_pieces(static_cast<size_t>(nel), plan_piece(nel), [&](size_t e0, size_t e1) {
         bool ok = true;
         for (size_t ea = 3 * e0; ea < 3 * e1; ++ea) {
             const int *sc = scheme + 3 * ea;
@@ -730,8 +732,8 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
         bptr.push_back(nord);
     }
     const int nb = static_cast<int>(bptr.size()) - 1;
-    // The blocks are independent and planned on several host threads (creating a mesh of 641 x 502 nodes:
-    // 39 ms, 64 on one thread; of 301 x 262 nodes 7.5, where slot lists take 5.5). An element belongs
+    // The blocks are independent; those of a large mesh are planned on several host threads (creating a mesh of
+    // 641 x 502 nodes: 39 ms, 64 on one thread). An element belongs
     // to the blocks of its rows, at the place of its first row there.
     std::vector<int> eptr(static_cast<size_t>(nb) + 1, 0), at(static_cast<size_t>(neq)), slots(static_cast<size_t>(nb), 0);
     std::vector<int> place(static_cast<size_t>(M->nnodes), -1);   // node -> place of its row in order (-1: prescribed)
@@ -747,8 +749,8 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     constexpr unsigned kFirst = 0x8000u;
     static_assert(kFzMaxSlots + 3 * kFzMaxInc < static_cast<int>(kFirst), "a slot and the mark in 16 bits");
     std::unique_ptr<unsigned short[]> qof(new unsigned short[static_cast<size_t>(nel) * 3]);
-    constexpr size_t kBlocks = 64;   // least blocks worth a thread
-    host_pieces(static_cast<size_t>(nb), kBlocks, [&](size_t b0, size_t b1) {
+    const size_t some = std::max<size_t>(1, plan_piece(nel) / kFzRows);   // blocks
+    host_pieces(static_cast<size_t>(nb), some, [&](size_t b0, size_t b1) {
         for (int b = static_cast<int>(b0); b < static_cast<int>(b1); ++b) {
             const int r0 = bptr[b], nr = bptr[b + 1] - r0;
             const size_t base = static_cast<size_t>(b) * ki * kFzRows;
@@ -784,7 +786,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     }
     const size_t nent = 2 * static_cast<size_t>(eptr[nb]);
     std::unique_ptr<int4[]> ent(new int4[nent]);
-    host_pieces(static_cast<size_t>(nb), kBlocks, [&](size_t b0, size_t b1) {
+    host_pieces(static_cast<size_t>(nb), some, [&](size_t b0, size_t b1) {
         for (int b = static_cast<int>(b0); b < static_cast<int>(b1); ++b) {
             int4 *o = ent.get() + 2 * static_cast<size_t>(eptr[b]);
             for (int h = bptr[b]; h < bptr[b + 1]; ++h)
@@ -924,7 +926,7 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     M->has_scheme = false;
     if (rc == FEMGPU_OK && scheme) {
         std::atomic<bool> slots_ok{true};
-        host_pieces(3 * n3, 9 * kPlanPiece, [&](size_t q0, size_t q1) {
+        host_pieces(3 * n3, plan_piece(nel), [&](size_t q0, size_t q1) {
             bool ok = true;
             for (size_t q = q0; q < q1; ++q) ok = ok && scheme[q] >= 0 && scheme[q] <= nnz;
             if (!ok) slots_ok = false;

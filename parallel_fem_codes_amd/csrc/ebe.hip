@@ -13,7 +13,6 @@
 // load of a wavefront is one contiguous run; the element rows of prescribed dofs are not stored.
 // Columns are kept as int16 offsets from the node's first unknown when the mesh numbering allows
 // (2 bytes per entry), else as int32 unknowns.
-#include <atomic>
 #include <climits>
 #include <vector>
 
@@ -469,6 +468,180 @@ static int fill_launch(femgpu_ctx *ctx, const femgpu_ebe *E, const double *Ae)
     return FEMGPU_OK;
 }
 
+// Node block rows of the FP32 product, planned on the device from the gathered columns (on the host the search for a
+// node's column nodes took 10 ms for 511 x 640 squares, a third of the creation). One lane per group: its column
+// nodes in order of appearance, each known by its first unknown; slots: the positions of every incidence's three
+// column nodes among them (8 bits each, 255: none); width: column nodes of the slice's longest group.
+constexpr int kBlockCols = 2 * kFillBlocks;   // fewer than kFillBlocks triangles: at most 2 * 23 + 1 column nodes
+
+template <typename CT, int ND>
+__global__ __launch_bounds__(64) void k_block_slots(int ngroups, int NEQ, const int *__restrict__ iptr,
+                                                    const int *__restrict__ len, const int *__restrict__ key,
+                                                    const CT *__restrict__ col, unsigned *__restrict__ slots,
+                                                    int *__restrict__ blen, int *__restrict__ width)
+{
+    constexpr int S = 3 * ND;
+    __shared__ int cols[kBlockCols * 64];
+    const int sl = blockIdx.x, l = threadIdx.x, g = sl * 64 + l;
+    const int n = g < ngroups ? len[g] : 0, kg = key && g < ngroups ? key[g] : 0, r1 = iptr[sl + 1];
+    int nc = 0;
+    for (int r = iptr[sl], j = 0; r < r1; ++r, ++j) {
+        unsigned code = ~0u;
+        for (int a = 0; a < 3 && j < n; ++a) {
+            int k = -1;
+            for (int d = 0; d < ND && k < 0; ++d) k = ebe_col<CT>(col[(static_cast<size_t>(r) * S + ND * a + d) * 64 + l], kg, NEQ);
+            if (k < 0) continue;   // a node without unknowns
+            int at = 0;
+            while (at < nc && cols[at * 64 + l] != k) ++at;
+            if (at == nc) cols[nc++ * 64 + l] = k;
+            code = (code & ~(255u << (8 * a))) | (static_cast<unsigned>(at) << (8 * a));
+        }
+        slots[static_cast<size_t>(r) * 64 + l] = code;
+    }
+    if (g < ngroups) blen[g] = nc;
+    for (int o = 32; o > 0; o >>= 1) nc = max(nc, __shfl_xor(nc, o, 64));
+    if (l == 0) width[sl] = nc;
+}
+
+// The columns of the block rows: those of the first incidence that has the node.
+template <typename CT, int ND>
+__global__ __launch_bounds__(64) void k_block_cols(int ngroups, CT sink, const int *__restrict__ iptr,
+                                                   const int *__restrict__ bptr, const int *__restrict__ len,
+                                                   const int *__restrict__ blen, const CT *__restrict__ col,
+                                                   const unsigned *__restrict__ slots, CT *__restrict__ bcol)
+{
+    constexpr int S = 3 * ND;
+    const int sl = blockIdx.x, l = threadIdx.x, g = sl * 64 + l;
+    const int n = g < ngroups ? len[g] : 0, nc = g < ngroups ? blen[g] : 0, r0 = iptr[sl], b0 = bptr[sl], b1 = bptr[sl + 1];
+    int seen = 0;
+    for (int j = 0; j < n; ++j) {
+        const unsigned code = slots[static_cast<size_t>(r0 + j) * 64 + l];
+        for (int a = 0; a < 3; ++a) {
+            if (((code >> (8 * a)) & 255u) != static_cast<unsigned>(seen)) continue;
+            for (int d = 0; d < ND; ++d)
+                bcol[(static_cast<size_t>(b0 + seen) * 64 + l) * ND + d] =
+                    col[(static_cast<size_t>(r0 + j) * S + ND * a + d) * 64 + l];
+            ++seen;
+        }
+    }
+    for (int b = b0 + nc; b < b1; ++b)
+        for (int d = 0; d < ND; ++d) bcol[(static_cast<size_t>(b) * 64 + l) * ND + d] = sink;
+}
+
+template <typename CT, int ND>
+static int block_rows_of(femgpu_ctx *ctx, femgpu_ebe *E, const CT *col, DevBuf<CT> &bcol, CT sink)
+{
+    hipStream_t st = ctx->stream;
+    DevBuf<int> width;
+    std::vector<int> bptr(static_cast<size_t>(E->nslices) + 1, 0);
+    FG_TRY(width.alloc(static_cast<size_t>(E->nslices)));
+    FG_TRY(E->slots.alloc(static_cast<size_t>(E->nrows) * 64));
+    FG_TRY(E->blen.alloc(static_cast<size_t>(E->ngroups)));
+    const int *key = E->col16 ? E->key.p : nullptr;
+    if (E->nslices > 0) {
+        k_block_slots<CT, ND><<<E->nslices, 64, 0, st>>>(E->ngroups, E->NEQ, E->iptr.p, E->len.p, key, col, E->slots.p,
+                                                        E->blen.p, width.p);
+        FG_HIP(hipGetLastError());
+        FG_HIP(hipMemcpyAsync(bptr.data() + 1, width.p, sizeof(int) * E->nslices, hipMemcpyDeviceToHost, st));
+        FG_HIP(hipStreamSynchronize(st));
+    }
+    for (int sl = 0; sl < E->nslices; ++sl) {
+        E->maxblk = std::max(E->maxblk, bptr[sl + 1]);
+        bptr[sl + 1] += bptr[sl];
+    }
+    if (E->maxblk > kFillBlocks) return FEMGPU_OK;   // too many column nodes for the fill kernel: planned as hubs
+    E->nbrows = bptr[E->nslices];
+    FG_TRY(E->bptr.upload(bptr.data(), bptr.size(), st));
+    FG_TRY(bcol.alloc(static_cast<size_t>(E->nbrows) * 64 * ND));
+    if (E->nslices > 0) {
+        k_block_cols<CT, ND><<<E->nslices, 64, 0, st>>>(E->ngroups, sink, E->iptr.p, E->bptr.p, E->len.p, E->blen.p, col,
+                                                       E->slots.p, bcol.p);
+        FG_HIP(hipGetLastError());
+    }
+    FG_HIP(hipStreamSynchronize(st));   // the host array ends here
+    return FEMGPU_OK;
+}
+
+static int block_rows(femgpu_ctx *ctx, femgpu_ebe *E)
+{
+    const short s16 = kSink16;
+    switch (E->ndof) {
+    case 1: return E->col16 ? block_rows_of<short, 1>(ctx, E, E->col16v.p, E->bcol16, s16) : block_rows_of<int, 1>(ctx, E, E->col32v.p, E->bcol32, E->NEQ);
+    case 3: return E->col16 ? block_rows_of<short, 3>(ctx, E, E->col16v.p, E->bcol16, s16) : block_rows_of<int, 3>(ctx, E, E->col32v.p, E->bcol32, E->NEQ);
+    default: return E->col16 ? block_rows_of<short, 4>(ctx, E, E->col16v.p, E->bcol16, s16) : block_rows_of<int, 4>(ctx, E, E->col32v.p, E->bcol32, E->NEQ);
+    }
+}
+
+// The same on the host, for operators with a node of too many column nodes for the fill kernel's LDS: the block
+// slots' element blocks (wptr, wsrc) in place of the incidences' positions. gptr, inc: a group's incidences 3 e + a;
+// kinc: the first unknown of every incidence's node (-1: none); gkey: a group's first unknown.
+static int hub_block_rows(femgpu_ctx *ctx, femgpu_ebe *E, const std::vector<int> &iptr, const std::vector<int> &inc,
+                          const std::vector<int> &gptr, const std::vector<int> &kinc, const std::vector<int> &gkey,
+                          const int *lm)
+{
+    const int ng = E->ngroups, nd = E->ndof, s = E->s;
+    hipStream_t st = ctx->stream;
+    std::vector<int> bptr(static_cast<size_t>(E->nslices) + 1, 0), blen(static_cast<size_t>(ng), 0);
+    std::vector<int> pos(static_cast<size_t>(E->NEQ), -1);   // a column node's position by its key
+    std::vector<int> at(3 * static_cast<size_t>(gptr[ng]), -1);
+    for (int g = 0; g < ng; ++g) {
+        for (int q = gptr[g]; q < gptr[g + 1]; ++q)
+            for (int a = 0; a < 3; ++a) {
+                const int k = kinc[inc[q] - inc[q] % 3 + a];
+                if (k < 0) continue;
+                if (pos[k] < 0) pos[k] = blen[g]++;
+                at[3 * static_cast<size_t>(q) + a] = pos[k];
+            }
+        for (int q = gptr[g]; q < gptr[g + 1]; ++q)
+            for (int a = 0; a < 3; ++a)
+                if (const int k = kinc[inc[q] - inc[q] % 3 + a]; k >= 0) pos[k] = -1;
+        bptr[(g >> 6) + 1] = std::max(bptr[(g >> 6) + 1], blen[g]);
+    }
+    E->maxblk = 0;
+    for (int sl = 0; sl < E->nslices; ++sl) {
+        E->maxblk = std::max(E->maxblk, bptr[sl + 1]);
+        bptr[sl + 1] += bptr[sl];
+    }
+    const size_t nb = static_cast<size_t>(bptr[E->nslices]) * 64;
+    std::vector<int> wptr(nb + 1, 0), wsrc, b32(E->col16 ? 0 : nb * nd, E->NEQ);
+    std::vector<short> b16(E->col16 ? nb * nd : 0, kSink16);
+    const auto slot_of = [&](int g, int p) { return (static_cast<size_t>(bptr[g >> 6]) + p) * 64 + (g & 63); };
+    for (int g = 0; g < ng; ++g)
+        for (int q = gptr[g]; q < gptr[g + 1]; ++q)
+            for (int a = 0; a < 3; ++a) {
+                const int p = at[3 * static_cast<size_t>(q) + a];
+                if (p < 0) continue;
+                const size_t o = slot_of(g, p);
+                if (wptr[o + 1]++ > 0) continue;   // the node's columns from its first incidence
+                const int *L = lm + static_cast<size_t>(inc[q] / 3) * s + nd * a;
+                for (int d = 0; d < nd; ++d) {
+                    if (L[d] >= E->NEQ) continue;
+                    if (E->col16) b16[o * nd + d] = static_cast<short>(L[d] - gkey[g]);
+                    else b32[o * nd + d] = L[d];
+                }
+            }
+    for (size_t q = 0; q < nb; ++q) wptr[q + 1] += wptr[q];
+    wsrc.resize(static_cast<size_t>(wptr[nb]));
+    for (int g = 0; g < ng; ++g)
+        for (int q = gptr[g]; q < gptr[g + 1]; ++q)
+            for (int a = 0; a < 3; ++a)
+                if (const int p = at[3 * static_cast<size_t>(q) + a]; p >= 0)
+                    wsrc[wptr[slot_of(g, p)]++] = 3 * (iptr[g >> 6] + q - gptr[g]) + a;
+    for (size_t q = nb; q > 0; --q) wptr[q] = wptr[q - 1];
+    wptr[0] = 0;
+    E->wide_slots = true;
+    E->nbrows = bptr[E->nslices];
+    E->slots.release();
+    FG_TRY(E->bptr.upload(bptr.data(), bptr.size(), st));
+    FG_TRY(E->blen.upload(blen.data(), blen.size(), st));
+    FG_TRY(E->wptr.upload(wptr.data(), wptr.size(), st));
+    FG_TRY(E->wsrc.upload(wsrc.data(), wsrc.size(), st));
+    if (E->col16) FG_TRY(E->bcol16.upload(b16.data(), b16.size(), st));
+    else FG_TRY(E->bcol32.upload(b32.data(), b32.size(), st));
+    FG_HIP(hipStreamSynchronize(st));   // the host arrays end here
+    return FEMGPU_OK;
+}
+
 }  // namespace fg
 
 using namespace fg;
@@ -486,15 +659,26 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     // incidence (e, a) -> its node's first unknown (the group key); nodes with every dof prescribed
     // contribute no rows
     std::vector<int> kinc(static_cast<size_t>(nel) * 3, -1), cnt(static_cast<size_t>(NEQ) + 1, 0);
-    for (int e = 0; e < nel; ++e)
+    // and whether the columns fit in 16 bits as offsets from it
+    bool fits16 = true;
+    for (int e = 0; e < nel; ++e) {
+        const int *L = lm + static_cast<size_t>(e) * s;
+        int *k = kinc.data() + 3 * static_cast<size_t>(e);
+        int lo = INT_MAX, hi = -1;   // the element's unknowns
+        for (int a = 0; a < 3; ++a)
+            for (int d = 0; d < nd; ++d) {
+                const int q = L[nd * a + d];
+                if (q >= NEQ) continue;
+                if (k[a] < 0) k[a] = q;
+                lo = std::min(lo, q);
+                hi = std::max(hi, q);
+            }
         for (int a = 0; a < 3; ++a) {
-            const int *L = lm + static_cast<size_t>(e) * s + nd * a;
-            int k = -1;
-            for (int d = 0; d < nd && k < 0; ++d)
-                if (L[d] < NEQ) k = L[d];
-            kinc[3 * static_cast<size_t>(e) + a] = k;
-            if (k >= 0) ++cnt[k];
+            if (k[a] < 0) continue;
+            ++cnt[k[a]];
+            fits16 = fits16 && k[a] - lo <= 32767 && hi - k[a] <= 32767;
         }
+    }
     std::vector<int> gid(static_cast<size_t>(NEQ) + 1, -1), gkey;
     for (int k = 0; k < NEQ; ++k)
         if (cnt[k] > 0) {
@@ -542,37 +726,17 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     const size_t nslots = static_cast<size_t>(nrows) * 64;
     FG_CHECK(nslots * s * nd < (size_t{1} << 40) && nslots < static_cast<size_t>(INT_MAX), FEMGPU_ERR_ARG,
              "femgpu_ebe_create: operator too large");
-    // The passes below are independent from slice to slice and run on several host threads: they are most of
-    // the time of a creation (800 x 400 squares, ndof = 4: 59 ms on one thread, 31 on eight).
-    constexpr size_t kElems = 1 << 13, kSlices = 1 << 6;   // least pieces worth a thread
-    // columns as 16-bit offsets from the node's first unknown where every one fits
-    std::atomic<bool> fits{true};
-    host_pieces(static_cast<size_t>(nel), kElems, [&](size_t e0, size_t e1) {
-        bool ok = true;
-        for (size_t e = e0; e < e1 && ok; ++e) {
-            const int *L = lm + e * s;
-            int lo = INT_MAX, hi = -1;   // the element's unknowns
-            for (int b = 0; b < s; ++b)
-                if (L[b] < NEQ) {
-                    lo = std::min(lo, L[b]);
-                    hi = std::max(hi, L[b]);
-                }
-            for (int a = 0; a < 3; ++a) {
-                const int k = kinc[3 * e + a];
-                ok = ok && (k < 0 || (static_cast<long>(lo) - k >= -32767 && static_cast<long>(hi) - k <= 32767));
-            }
-        }
-        if (!ok) fits = false;
-    });
-    const bool fits16 = fits;
+    // Per incidence its rows' place and its columns. The slices are independent: large operators take several host
+    // threads (below, a thread that waits for a processor, 4 ms beside a pool of threads that spin, would cost more
+    // than it saves).
     std::vector<int> src(nslots, -1), c32(fits16 ? 0 : nslots * s, NEQ);
     std::vector<short> c16(fits16 ? nslots * s : 0, kSink16);
-    host_pieces(static_cast<size_t>(nslices), kSlices, [&](size_t s0, size_t s1) {
+    host_pieces(static_cast<size_t>(nslices), nel >= 1 << 18 ? 1 << 8 : SIZE_MAX, [&](size_t s0, size_t s1) {
         for (int g = static_cast<int>(64 * s0); g < std::min(ng, static_cast<int>(64 * s1)); ++g) {
-            const int sl = g >> 6, l = g & 63, key = gkey[g];
+            const int l = g & 63, key = gkey[g];
             for (int j = 0; j < len[g]; ++j) {
                 const int ea = inc[gptr[g] + j], e = ea / 3, a = ea % 3;
-                const size_t r = static_cast<size_t>(iptr[sl] + j);
+                const size_t r = static_cast<size_t>(iptr[g >> 6] + j);
                 src[r * 64 + l] = e * s * s + nd * a * s;
                 const int *L = lm + static_cast<size_t>(e) * s;
                 if (fits16) {
@@ -585,113 +749,9 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
             }
         }
     });
-    // node block rows of the FP32 product: per group its column nodes (groups) in order of appearance, and
-    // the position of each incidence's three column nodes among them (three 8-bit positions per incidence,
-    // or one word each where a node has too many column nodes)
-    std::vector<int> bptr(static_cast<size_t>(nslices) + 1, 0), blen(ng, 0);
-    const bool packed = maxinc < kFillBlocks;   // n triangles around a node have n + 1 column nodes
-    std::vector<unsigned> slots(packed ? nslots : 3 * nslots, ~0u);
-    const auto set_slot = [&](size_t q, int a, int at) {
-        if (packed) slots[q] = (slots[q] & ~(255u << (8 * a))) | (static_cast<unsigned>(at) << (8 * a));
-        else slots[3 * q + a] = static_cast<unsigned>(at);
-    };
-    std::vector<int> pos(packed ? 0 : static_cast<size_t>(NEQ), -1);   // hubs: a column node's position by its key
-    const auto block_cols = [&](size_t s0, size_t s1) {
-        int cs[3 * kFillBlocks];
-        for (size_t sl = s0; sl < s1; ++sl) {
-            int w = 0;
-            for (int g = static_cast<int>(64 * sl); g < std::min(ng, static_cast<int>(64 * sl) + 64); ++g) {
-                int nc = 0;
-                for (int j = 0; j < len[g]; ++j) {
-                    const int ea = inc[gptr[g] + j], e3 = ea - ea % 3;
-                    const size_t q = static_cast<size_t>(iptr[sl] + j) * 64 + (g & 63);
-                    for (int a = 0; a < 3; ++a) {
-                        const int k = kinc[e3 + a];
-                        if (k < 0) continue;
-                        int at = 0;
-                        if (packed) {
-                            while (at < nc && cs[at] != k) ++at;
-                            if (at == nc) cs[nc++] = k;
-                        } else {
-                            if (pos[k] < 0) pos[k] = nc++;
-                            at = pos[k];
-                        }
-                        set_slot(q, a, at);
-                    }
-                }
-                if (!packed)
-                    for (int j = 0; j < len[g]; ++j)
-                        for (int ea = inc[gptr[g] + j], a = 0; a < 3; ++a)
-                            if (const int k = kinc[ea - ea % 3 + a]; k >= 0) pos[k] = -1;
-                blen[g] = nc;
-                w = std::max(w, nc);
-            }
-            bptr[sl + 1] = w;
-        }
-    };
-    if (packed) host_pieces(static_cast<size_t>(nslices), kSlices, block_cols);
-    else block_cols(0, static_cast<size_t>(nslices));
-    int maxblk = 0;
-    for (int sl = 0; sl < nslices; ++sl) {
-        maxblk = std::max(maxblk, bptr[sl + 1]);
-        bptr[sl + 1] += bptr[sl];
-    }
-    // their columns, at the first incidence that has the node
-    const size_t ncols = static_cast<size_t>(bptr[nslices]) * 64 * nd;
-    std::vector<int> b32(fits16 ? 0 : ncols, NEQ);
-    std::vector<short> b16(fits16 ? ncols : 0, kSink16);
-    host_pieces(static_cast<size_t>(nslices), kSlices, [&](size_t s0, size_t s1) {
-        for (int g = static_cast<int>(64 * s0); g < std::min(ng, static_cast<int>(64 * s1)); ++g) {
-            const int sl = g >> 6, l = g & 63;
-            int seen = 0;
-            for (int j = 0; j < len[g] && seen < blen[g]; ++j) {
-                const int ea = inc[gptr[g] + j];
-                const size_t q = static_cast<size_t>(iptr[sl] + j) * 64 + l;
-                for (int a = 0; a < 3; ++a) {
-                    const unsigned at = packed ? (slots[q] >> (8 * a)) & 255u : slots[3 * q + a];
-                    if (at != static_cast<unsigned>(seen)) continue;   // seen before, or without unknowns
-                    ++seen;
-                    const int *L = lm + static_cast<size_t>(ea / 3) * s + nd * a;
-                    const size_t o = ((static_cast<size_t>(bptr[sl]) + at) * 64 + l) * nd;
-                    for (int d = 0; d < nd; ++d) {
-                        if (L[d] >= NEQ) continue;
-                        if (fits16) b16[o + d] = static_cast<short>(L[d] - gkey[g]);
-                        else b32[o + d] = L[d];
-                    }
-                }
-            }
-        }
-    });
-    const size_t nbslots = static_cast<size_t>(bptr[nslices]) * 64;
-    // a node with too many column nodes for the fill kernel's LDS: the element blocks of every block slot instead
-    const bool wide = !packed || maxblk > kFillBlocks;
-    std::vector<int> wptr, wsrc;
-    if (wide) {
-        const auto each_block = [&](const auto &f) {   // f(block slot, 3 * incidence row + vertex), in element order
-            for (int g = 0; g < ng; ++g)
-                for (int j = 0; j < len[g]; ++j) {
-                    const size_t r = static_cast<size_t>(iptr[g >> 6] + j), q = r * 64 + (g & 63);
-                    for (int a = 0; a < 3; ++a) {
-                        const unsigned at = packed ? (slots[q] >> (8 * a)) & 255u : slots[3 * q + a];
-                        if (at != (packed ? 255u : ~0u))
-                            f((static_cast<size_t>(bptr[g >> 6]) + at) * 64 + (g & 63), static_cast<int>(3 * r) + a);
-                    }
-                }
-        };
-        wptr.assign(nbslots + 1, 0);
-        each_block([&](size_t q, int) { ++wptr[q + 1]; });
-        for (size_t q = 0; q < nbslots; ++q) wptr[q + 1] += wptr[q];
-        wsrc.resize(static_cast<size_t>(wptr[nbslots]));
-        each_block([&](size_t q, int ra) { wsrc[wptr[q]++] = ra; });
-        for (size_t q = nbslots; q > 0; --q) wptr[q] = wptr[q - 1];
-        wptr[0] = 0;
-    }
     auto *E = new femgpu_ebe();
     E->ctx = ctx;
     E->nslices = nslices;
-    E->nbrows = bptr[nslices];
-    E->wide_slots = wide;
-    E->maxblk = maxblk;
     E->nel = nel;
     E->s = s;
     E->ndof = nd;
@@ -711,14 +771,9 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     if (!rc && fits16) rc = E->col16v.upload(c16.data(), c16.size(), st);
     if (!rc && !fits16) rc = E->col32v.upload(c32.data(), c32.size(), st);
     if (!rc) rc = E->val.alloc(nslots * s * nd);
-    if (!rc) rc = E->bptr.upload(bptr.data(), bptr.size(), st);
-    if (!rc) rc = E->blen.upload(blen.data(), blen.size(), st);
-    if (!rc && fits16) rc = E->bcol16.upload(b16.data(), b16.size(), st);
-    if (!rc && !fits16) rc = E->bcol32.upload(b32.data(), b32.size(), st);
-    if (!rc && !wide) rc = E->slots.upload(slots.data(), slots.size(), st);
-    if (!rc && wide) rc = E->wptr.upload(wptr.data(), wptr.size(), st);
-    if (!rc && wide) rc = E->wsrc.upload(wsrc.data(), wsrc.size(), st);
-    if (!rc) rc = E->val32.alloc(nbslots * nd * nd);
+    if (!rc) rc = maxinc < kFillBlocks ? block_rows(ctx, E) : FEMGPU_OK;
+    if (!rc && (maxinc >= kFillBlocks || E->maxblk > kFillBlocks)) rc = hub_block_rows(ctx, E, iptr, inc, gptr, kinc, gkey, lm);
+    if (!rc) rc = E->val32.alloc(static_cast<size_t>(E->nbrows) * 64 * nd * nd);
     if (!rc && hipStreamSynchronize(st) != hipSuccess) rc = FEMGPU_ERR_HIP;   // host arrays end here
     if (rc) {
         delete E;
