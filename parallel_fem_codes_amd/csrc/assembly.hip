@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
 #include <memory>
 #include <vector>
 
@@ -663,7 +664,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     // every row's first and last CSR slot
     std::vector<int> rfirst(neq), rlast(neq);
     std::atomic<bool> plain{true};   // no slots in prescribed rows, an element row's slots distinct
-    host_pieces(static_cast<size_t>(neq), plan_piece(nel), [&](size_t i0, size_t i1) {
+    host_pieces(static_cast<size_t>(neq), plan_piece(nel), [&](size_t i0, size_t i1, size_t) {
         bool ok = true;
         for (size_t i = i0; i < i1; ++i) {
             int lo = INT32_MAX, hi = -1;
@@ -681,7 +682,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
         }
         if (!ok) plain = false;
     });
-    host_pieces(static_cast<size_t>(nel), plan_piece(nel), [&](size_t e0, size_t e1) {
+    host_pieces(static_cast<size_t>(nel), plan_piece(nel), [&](size_t e0, size_t e1, size_t) {
         bool ok = true;
         for (size_t ea = 3 * e0; ea < 3 * e1; ++ea) {
             const int *sc = scheme + 3 * ea;
@@ -733,13 +734,16 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     }
     const int nb = static_cast<int>(bptr.size()) - 1;
     // The blocks are independent; those of a large mesh are planned on several host threads (creating a mesh of
-    // 641 x 502 nodes: 39 ms, 64 on one thread). An element belongs
-    // to the blocks of its rows, at the place of its first row there.
-    std::vector<int> eptr(static_cast<size_t>(nb) + 1, 0), at(static_cast<size_t>(neq)), slots(static_cast<size_t>(nb), 0);
-    std::vector<int> place(static_cast<size_t>(M->nnodes), -1);   // node -> place of its row in order (-1: prescribed)
-    for (int h = 0; h < neq; ++h) at[order[h]] = h;
-    for (int v = 0; v < M->nnodes; ++v)
-        if (eq[v] >= 0 && eq[v] < neq) place[v] = at[eq[v]];
+    // 641 x 502 nodes: 42 ms, 64 on one thread). An element belongs
+    // to the blocks of its rows, in the order in which their rows name it first.
+    std::vector<int> eptr(static_cast<size_t>(nb) + 1, 0), slots(static_cast<size_t>(nb), 0);
+    const size_t some = std::max<size_t>(1, plan_piece(nel) / kFzRows), pieces = host_piece_count(static_cast<size_t>(nb), some);
+    // per thread, by element: 1 + the last block that has it (zero pages until touched)
+    struct Free {
+        void operator()(int *p) const { free(p); }
+    };
+    std::unique_ptr<int, Free> seen_in(static_cast<int *>(calloc(pieces * nel, sizeof(int))));
+    FG_CHECK(seen_in, FEMGPU_ERR_NOMEM, "femgpu_mesh_create: out of host memory");
     // every block's incidence codes: ki rows of kFzRows (padding 0xffffffff). The large arrays are first touched by
     // the threads that fill them.
     const size_t ninc = static_cast<size_t>(nb) * ki * kFzRows;
@@ -749,8 +753,8 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     constexpr unsigned kFirst = 0x8000u;
     static_assert(kFzMaxSlots + 3 * kFzMaxInc < static_cast<int>(kFirst), "a slot and the mark in 16 bits");
     std::unique_ptr<unsigned short[]> qof(new unsigned short[static_cast<size_t>(nel) * 3]);
-    const size_t some = std::max<size_t>(1, plan_piece(nel) / kFzRows);   // blocks
-    host_pieces(static_cast<size_t>(nb), some, [&](size_t b0, size_t b1) {
+    host_pieces(static_cast<size_t>(nb), some, [&](size_t b0, size_t b1, size_t piece) {
+        int *mark = seen_in.get() + piece * nel;
         for (int b = static_cast<int>(b0); b < static_cast<int>(b1); ++b) {
             const int r0 = bptr[b], nr = bptr[b + 1] - r0;
             const size_t base = static_cast<size_t>(b) * ki * kFzRows;
@@ -760,12 +764,9 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
                 const int i = order[r0 + t], rf = rfirst[i];
                 unsigned *ic = inc.get() + base + t;
                 for (int q = rows[i].first; q < rows[i].end; ++q, ic += kFzRows) {
-                    const int ea = rinc[q], a = ea % 3, *v = ien + (ea - a), *sc = scheme + 3 * static_cast<size_t>(ea);
-                    bool first = true;
-                    for (int c = 0; c < 3; ++c) {
-                        const int h = place[v[c]];
-                        first = first && !(h >= r0 && (h < r0 + t || (h == r0 + t && c < a)));
-                    }
+                    const int ea = rinc[q], e = ea / 3, *sc = scheme + 3 * static_cast<size_t>(ea);
+                    const bool first = mark[e] != b + 1;
+                    mark[e] = b + 1;
                     unsigned code = static_cast<unsigned>(nslot);
                     for (int c = 0; c < 3; ++c)
                         code |= (sc[c] < nnz ? static_cast<unsigned>(sc[c] - rf) : 15u) << (16 + 4 * c);
@@ -786,7 +787,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     }
     const size_t nent = 2 * static_cast<size_t>(eptr[nb]);
     std::unique_ptr<int4[]> ent(new int4[nent]);
-    host_pieces(static_cast<size_t>(nb), some, [&](size_t b0, size_t b1) {
+    host_pieces(static_cast<size_t>(nb), some, [&](size_t b0, size_t b1, size_t) {
         for (int b = static_cast<int>(b0); b < static_cast<int>(b1); ++b) {
             int4 *o = ent.get() + 2 * static_cast<size_t>(eptr[b]);
             for (int h = bptr[b]; h < bptr[b + 1]; ++h)
@@ -797,8 +798,7 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
                     unsigned sl[3];
                     for (int a = 0; a < 3; ++a) {
                         qn[a] = eq[ien[e3 + a]];
-                        const int h2 = place[ien[e3 + a]];
-                        sl[a] = h2 >= bptr[b] && h2 < bptr[b + 1] ? qof[e3 + a] & (kFirst - 1u) : 0xffffu;
+                        sl[a] = qn[a] >= 0 && blk[qn[a]] == b ? qof[e3 + a] & (kFirst - 1u) : 0xffffu;
                     }
                     *o++ = make_int4(ien[e3], ien[e3 + 1], ien[e3 + 2], qn[0]);
                     *o++ = make_int4(qn[1], qn[2], static_cast<int>(sl[0] | (sl[1] << 16)),
@@ -926,7 +926,7 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     M->has_scheme = false;
     if (rc == FEMGPU_OK && scheme) {
         std::atomic<bool> slots_ok{true};
-        host_pieces(3 * n3, plan_piece(nel), [&](size_t q0, size_t q1) {
+        host_pieces(3 * n3, plan_piece(nel), [&](size_t q0, size_t q1, size_t) {
             bool ok = true;
             for (size_t q = q0; q < q1; ++q) ok = ok && scheme[q] >= 0 && scheme[q] <= nnz;
             if (!ok) slots_ok = false;

@@ -37,24 +37,29 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
         if (r_ != FEMGPU_OK) return r_; \
     } while (0)
 
-// f(first, end) over pieces of [0, n), of `grain` items or more, on up to 8 host threads (the caller's among
-// them). f must not throw and writes to its own items only. A thread that cannot be had leaves its piece to
-// the caller.
+inline size_t host_piece_count(size_t n, size_t grain)
+{
+    return std::max<size_t>(1, std::min<size_t>({n / grain, 8, std::max(1u, std::thread::hardware_concurrency())}));
+}
+
+// f(first, end, piece) over host_piece_count pieces of [0, n), of `grain` items or more, on as many host threads (the
+// caller's among them). f must not throw and writes to its own items only. A thread that cannot be had leaves
+// its piece to the caller.
 template <typename F>
 inline void host_pieces(size_t n, size_t grain, const F &f)
 {
-    const size_t k = std::max<size_t>(1, std::min<size_t>({n / grain, 8, std::max(1u, std::thread::hardware_concurrency())}));
+    const size_t k = host_piece_count(n, grain);
     std::thread th[8];
     size_t mine = k;   // pieces from here on are the caller's
     for (size_t i = 1; i < k && mine == k; ++i) {
         try {
-            th[i] = std::thread([&f, n, k, i] { f(n * i / k, n * (i + 1) / k); });
+            th[i] = std::thread([&f, n, k, i] { f(n * i / k, n * (i + 1) / k, i); });
         } catch (...) {
             mine = i;
         }
     }
-    f(size_t{0}, n / k);
-    if (mine < k) f(n * mine / k, n);
+    f(size_t{0}, n / k, size_t{0});
+    for (size_t i = mine; i < k; ++i) f(n * i / k, n * (i + 1) / k, i);
     for (auto &t : th)
         if (t.joinable()) t.join();
 }

@@ -731,7 +731,7 @@ extern "C" int femgpu_ebe_create(femgpu_ctx *ctx, int nel, int s, int NEQ, const
     // than it saves).
     std::vector<int> src(nslots, -1), c32(fits16 ? 0 : nslots * s, NEQ);
     std::vector<short> c16(fits16 ? nslots * s : 0, kSink16);
-    host_pieces(static_cast<size_t>(nslices), nel >= 1 << 18 ? 1 << 8 : SIZE_MAX, [&](size_t s0, size_t s1) {
+    host_pieces(static_cast<size_t>(nslices), nel >= 1 << 18 ? 1 << 8 : SIZE_MAX, [&](size_t s0, size_t s1, size_t) {
         for (int g = static_cast<int>(64 * s0); g < std::min(ng, static_cast<int>(64 * s1)); ++g) {
             const int l = g & 63, key = gkey[g];
             for (int j = 0; j < len[g]; ++j) {
