@@ -364,10 +364,12 @@ int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *sys, int ns
 /* The same batched mixed-precision solve as one persistent launch with a workgroup per system:
  * each system runs its own FP64 refinement and FP32 GMRES(inner_kmax) (its own Krylov space and
  * Hessenberg matrix, fused MGS, Givens and least squares in LDS) on the sliced-ELL copy of A with
- * the parallel ILU(0) factors applied by Jacobi iterations, so a system's answer is bit-identical
- * alone and in any batch, and the whole solve costs one launch. Needs sys->csr == sys->ilu created
+ * the parallel ILU(0) factors applied by Jacobi iterations, so at one workgroup size (which sets the
+ * order of its sums) a system's answer is bit-identical alone and in any batch, and the whole solve
+ * costs one launch. An entry between two systems is refused (FEMGPU_ERR_ARG). Needs sys->csr == sys->ilu created
  * with FEMGPU_PLANS_MIXED (rows of at most 16 entries), factor_sweeps 1..16, sweep_mode 1..16,
- * inner_kmax <= 64. threads: 256, 512 or 1024 per workgroup, 0 = chosen from the mean system size.
+ * inner_kmax <= 64. threads: 256, 512 or 1024 per workgroup, 0 = chosen from the mean system size, and
+ * so from the batch.
  * For many small systems (launch latency, not bandwidth, bounds their multi-launch solve). No
  * reference counterpart. */
 int femgpu_gmres_mixed_wg(femgpu_ctx *ctx, const femgpu_system *sys, int nsys, const int *row_off,

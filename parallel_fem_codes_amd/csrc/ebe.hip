@@ -113,10 +113,13 @@ struct NodeVec {
     float v[ND];
 };
 
-// TAIL: the product inside an Arnoldi step (ArnoldiTail), which is launched for systems of some ten thousand
-// unknowns and waits in its chains of loads: a wavefront per block, so that the nodes spread over more CUs, and a
-// whole node of six triangles in one batch. 20 000 nodes of four dofs: 7.9 us with the end of the step before
-// and the nodal blocks (9.6 us with 256 threads and batches of four); as three kernels 8.9 + 4.7 + 3.3.
+// TAIL: the product inside an Arnoldi step (ArnoldiTail), which waits in its chains of loads where systems have some
+// ten thousand unknowns: a wavefront per block, so that the nodes spread over more CUs, and a whole node of six
+// triangles in one batch. 20 000 nodes of four dofs: 7.9 us with the end of the step before and the nodal blocks
+// (9.6 us with 256 threads and batches of four); as three kernels 8.9 + 4.7 + 3.3. At any size: a whole inner step
+// (CGS) of 20 000 / 80 000 / 181 000 / 321 000 nodes of four dofs takes 25.7 / 41.1 / 60.6 / 88.9 us so, 27.2 / 42.3 /
+// 60.3 / 90.6 with 256 threads and batches of four, 32.9 / 49.3 / 65.1 / 97.9 with the nodal blocks in a kernel of
+// their own; 812 000 nodes of one dof 56.5 / 56.8 / 59.7.
 constexpr int kTailThreads = 64, kTailRows = 7;
 
 template <typename CT, int ND, int U, bool TAIL>

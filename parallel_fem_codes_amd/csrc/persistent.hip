@@ -2,8 +2,8 @@
 // system in one launch -- the FP64 residual and refinement, the FP32 inner GMRES(m) on the sliced-ELL
 // copy of A with the Jacobi-applied parallel ILU(0) factors, fused MGS passes, and the Givens and
 // least-squares steps in LDS. Every system has its own Krylov space and Hessenberg matrix, so a
-// system's iterates do not depend on the other systems of the launch: its answer is bit-identical
-// alone and in any batch. For the small systems of the serving loop, where one launch per kernel
+// system's iterates do not depend on the other systems of the launch: at one workgroup size (the order
+// of its sums) its answer is bit-identical alone and in any batch. For the small systems of the serving loop, where one launch per kernel
 // step would cost more than the step's memory traffic.
 //
 // Two forms. A system whose vectors fit in the workgroup's LDS runs there, its matrix and factors in
@@ -714,11 +714,14 @@ static int wg_enqueue(femgpu_ctx *ctx, femgpu_csr *A, int nsys, const int *row_o
 }
 
 // Whether the multi-launch mixed solvers hand a solve to the workgroup solver: the same operator and
-// preconditioner, systems small enough for its LDS path, one workgroup each. Their own launches cost about
+// preconditioner, systems small enough for its LDS path (four rows for each of 1 024 threads), one workgroup each. Their own launches cost about
 // 3 us each whatever the rows, 6 + i of them in Arnoldi step i (4 with classical Gram-Schmidt). Transient
 // systems of 361 / 1 472 / 3 481 rows: 84 / 181 / 337 us against 479 / 669 / 601 us; a steady one of 3 800
 // rows 2.42 ms against 3.97 ms; batches of 16 steady systems of 1 000 / 2 000 / 3 000 rows 0.48 / 1.38 /
-// 2.06 ms against 2.06 / 2.29 / 2.51 ms for the block-diagonal launches.
+// 2.06 ms against 2.06 / 2.29 / 2.51 ms for the block-diagonal launches. On either side of the lines: a
+// transient system of 4 096 rows 389 us (launches 752), of 4 489, its vectors in global memory, 884 (716), of 8 281
+// 1 604 (784); 16 steady systems of 2 500 / 3 300 / 4 200 rows 2.04 / 2.49 / 7.15 ms against 4.86 / 5.15 / 7.44 ms of
+// launches with MGS, 2.15 / 2.41 / 3.57 ms with CGS.
 bool wg_preferred(const femgpu_ctx *ctx, const femgpu_system *S, const femgpu_mixed_opts *opt, int nsys, int widest)
 {
     const femgpu_csr *A = S->csr;

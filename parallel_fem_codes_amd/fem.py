@@ -606,7 +606,8 @@ def gmres_mixed_batched(dev: Device, A: CsrMatrix, row_off, F, X, tol=1e-8, inne
 def gmres_mixed_wg(dev: Device, A: CsrMatrix, row_off, F, X, tol=1e-8, inner_kmax=30, inner_tol=1e-4,
                    max_refinements=50, sweep_mode=2, factor_sweeps=2, threads=0):
     """The batched mixed-precision solve as one persistent launch, a workgroup per system (its own
-    Krylov space: the answer does not depend on the batch); returns one BatchInfo per system."""
+    Krylov space: at one workgroup size the answer does not depend on the batch; threads 0 takes the size
+    from the systems' mean); returns one BatchInfo per system."""
     ro = _i32(row_off)
     K = len(ro) - 1
     infos = (N.BatchInfo * K)()
