@@ -647,12 +647,13 @@ static size_t plan_piece(int nel) { return nel >= 1 << 18 ? 1 << 13 : SIZE_MAX; 
 // The fused assembly's plan from the mesh's host arrays: rows grouped into compact patches by
 // breadth-first growth over the mesh graph (up to kFzRows rows and kFzMaxSlots incidences), each
 // patch's elements in order of first touch, its incidences numbered row by row as LDS slots. eq:
-// equation of every node (-1: prescribed); rows, rinc: a row's incidences 3 e + a in element order. fz_state 1 when every
+// equation of every node (-1: prescribed); rows, rinc: a row's incidences 3 e + a in element order; entries: slots
+// that scheme names. fz_state 1 when every
 // slot of the CSR values is an entry of exactly one row (its slots contiguous, the three of an element
 // row distinct), rows have at most 15 entries and 16 incidences, and no prescribed row has slots; else
 // -1, and the assembly takes the slot lists.
 static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, const std::vector<int> &eq,
-                            const std::vector<RowList> &rows, const std::vector<int> &rinc)
+                            const std::vector<RowList> &rows, const std::vector<int> &rinc, long long entries)
 {
     M->fz_state = -1;
     const int nel = M->nel, neq = M->neq, nnz = M->nnz;
@@ -663,9 +664,11 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
     if (ki > kFzMaxInc) return FEMGPU_OK;
     // every row's first and last CSR slot
     std::vector<int> rfirst(neq), rlast(neq);
-    std::atomic<bool> plain{true};   // no slots in prescribed rows, an element row's slots distinct
+    std::atomic<bool> distinct{true};   // the slots of an element row
+    std::atomic<long long> named{0};    // slots named by the rows: all of them, if no prescribed row names one
     host_pieces(static_cast<size_t>(neq), plan_piece(nel), [&](size_t i0, size_t i1, size_t) {
         bool ok = true;
+        long long count = 0;
         for (size_t i = i0; i < i1; ++i) {
             int lo = INT32_MAX, hi = -1;
             for (int q = rows[i].first; q < rows[i].end; ++q) {
@@ -675,35 +678,34 @@ static int build_fused_plan(femgpu_mesh *M, const int *ien, const int *scheme, c
                     ok = ok && sc[b] != sc[(b + 1) % 3];
                     lo = std::min(lo, sc[b]);
                     hi = std::max(hi, sc[b]);
+                    ++count;
                 }
             }
             rfirst[i] = lo;
             rlast[i] = hi;
         }
-        if (!ok) plain = false;
+        if (!ok) distinct = false;
+        named += count;
     });
-    host_pieces(static_cast<size_t>(nel), plan_piece(nel), [&](size_t e0, size_t e1, size_t) {
-        bool ok = true;
-        for (size_t ea = 3 * e0; ea < 3 * e1; ++ea) {
-            const int *sc = scheme + 3 * ea;
-            ok = ok && (eq[ien[ea]] >= 0 || (sc[0] >= nnz && sc[1] >= nnz && sc[2] >= nnz));
-        }
-        if (!ok) plain = false;
-    });
-    if (!plain) return FEMGPU_OK;
+    if (!distinct || named != entries) return FEMGPU_OK;
     int maxlen = 0;
     long long covered = 0;
-    std::vector<char> seen(static_cast<size_t>(nnz), 0);
+    bool in_order = true;   // the rows' slots one row after the other: every slot in exactly one
     for (int i = 0; i < neq; ++i) {
         if (rlast[i] < 0 || rlast[i] - rfirst[i] >= 15) return FEMGPU_OK;
         maxlen = std::max(maxlen, rlast[i] - rfirst[i] + 1);
+        in_order = in_order && rfirst[i] == covered;
         covered += rlast[i] - rfirst[i] + 1;
-        for (int k = rfirst[i]; k <= rlast[i]; ++k) {
-            if (seen[k]) return FEMGPU_OK;
-            seen[k] = 1;
-        }
     }
     if (covered != nnz) return FEMGPU_OK;
+    if (!in_order) {
+        std::vector<char> seen(static_cast<size_t>(nnz), 0);
+        for (int i = 0; i < neq; ++i)
+            for (int k = rfirst[i]; k <= rlast[i]; ++k) {
+                if (seen[k]) return FEMGPU_OK;
+                seen[k] = 1;
+            }
+    }
     // blocks: breadth-first patches over the row graph
     std::vector<int> blk(neq, -1), order(neq), bptr{0};
     int nord = 0;
@@ -847,7 +849,7 @@ static int fused_plan_from_lists(femgpu_mesh *M)
         for (int q = aptr[k]; q < aptr[k + 1]; ++q) scheme[asrc[q]] = adst[k];
     std::vector<RowList> rows;
     incidence_map(nel, neq, ien.data(), eq, rptr, rinc, rdst, rows);
-    return build_fused_plan(M, ien.data(), scheme.data(), eq, rows, rinc);
+    return build_fused_plan(M, ien.data(), scheme.data(), eq, rows, rinc, static_cast<long long>(asrc.size()));
 }
 
 template <bool STEADY>
@@ -926,17 +928,23 @@ static int mesh_setup(femgpu_mesh *M, int nnodes, int nel, int neq, const double
     M->has_scheme = false;
     if (rc == FEMGPU_OK && scheme) {
         std::atomic<bool> slots_ok{true};
+        std::atomic<long long> entries{0};
         host_pieces(3 * n3, plan_piece(nel), [&](size_t q0, size_t q1, size_t) {
             bool ok = true;
-            for (size_t q = q0; q < q1; ++q) ok = ok && scheme[q] >= 0 && scheme[q] <= nnz;
+            long long count = 0;
+            for (size_t q = q0; q < q1; ++q) {
+                ok = ok && scheme[q] >= 0 && scheme[q] <= nnz;
+                count += scheme[q] < nnz;
+            }
             if (!ok) slots_ok = false;
+            entries += count;
         });
         if (!slots_ok) rc = FEMGPU_ERR_ARG;
         if (rc == FEMGPU_ERR_ARG) set_error("femgpu_mesh_create: scheme slot out of range");
         if (rc == FEMGPU_OK && one_off) {
             M->fz_state = 0;
         } else if (rc == FEMGPU_OK) {
-            rc = build_fused_plan(M, ien, scheme, eq, rows, rinc);
+            rc = build_fused_plan(M, ien, scheme, eq, rows, rinc, entries);
         }
         M->has_scheme = rc == FEMGPU_OK;
         if (rc == FEMGPU_OK && M->fz_state != 1) {   // slot lists, where the fused assembly does not apply
