@@ -356,7 +356,8 @@ typedef struct {
  * sequence serves the whole batch. Batches of systems of at most 3072 rows (no more systems than the
  * GPU has compute units, factor_sweeps >= 1, sweep_mode >= 1) take femgpu_gmres_mixed_wg's kernel
  * unless multi_launch is 1: a workgroup and a Krylov space per system, whose Gram-Schmidt is the
- * modified one whatever orthogonalization says. info: nsys entries. No reference counterpart. */
+ * modified one whatever orthogonalization says. Where an entry couples two systems they share the
+ * Krylov space at any size. info: nsys entries. No reference counterpart. */
 int femgpu_gmres_mixed_batched(femgpu_ctx *ctx, const femgpu_system *sys, int nsys, const int *row_off,
                                const femgpu_mixed_opts *opt, double tol, const double *d_F, double *d_X,
                                femgpu_batch_info *info);

@@ -73,7 +73,9 @@ def test_factor_rows_bit_exact(oracle, case):
 def test_factor_rows_plan_on_demand(oracle):
     """A matrix with the streamed factorisation holds no plan of the level-synchronous one (400 bytes a row) until
     it is asked for; a rebuilt matrix keeps the kernel asked for."""
+    import gc
     import torch
+    gc.collect()   # no other test's matrices are freed between the two readings
     dev = fem.Device(0)
     IA, JA = block_pattern(500, 1)
     n = len(IA) - 1
